@@ -14,6 +14,7 @@
 #include "cubql_amd/traversal.hip.h"
 #include "profile.h"
 #include "query_order.h"
+#include "wave_closest.h"
 
 namespace cubql {
 namespace pq {
@@ -27,6 +28,11 @@ constexpr int32_t kIncomplete = -2;
 __device__ __forceinline__ float3 load_pt(const float *p, uint32_t i) {
   return make_float3(p[3 * (size_t)i + 0], p[3 * (size_t)i + 1], p[3 * (size_t)i + 2]);
 }
+
+// Waves that a small closest-point batch is spread over: 1000 queries of 1M
+// points take 25.6 us as 1000 waves of one query, whose subtrees the other
+// lanes take, and took 87.7 us as 16 waves of one query per lane.
+constexpr uint32_t kWavesWanted = 4096;
 
 struct Overflow {
   uint32_t count;
@@ -54,58 +60,43 @@ __device__ __forceinline__ bool fcp_one(const BVH &bvh, const float *points, flo
   return cubql_dev::for_each_prim_except<STACK>(bvh, q.x, q.y, q.z, bestD, prim, seed, 0u, st);
 }
 
-// The same over a binary tree on a caller-provided traversal stack.
-template <typename StackT>
-__device__ __forceinline__ bool fcp_one_on(StackT &stack, const cubql_bvh3f &bvh, const float *points, float3 q,
-                                           float sqrMax, int32_t &best, float &bestD) {
-  best = -1;
-  bestD = sqrMax;
-  auto prim = [&](uint32_t pid) -> float {
-    float3 p = load_pt(points, pid);
-    float d = cubql_dev::sqr_dist_pt(p.x, p.y, p.z, q.x, q.y, q.z);
-    if (d < bestD || (d == bestD && best >= 0 && (int32_t)pid < best)) {
-      bestD = d;
-      best = (int32_t)pid;
+// Least key of a leaf's prims, four in flight.  kSorted: the prims come from
+// a copy of the points in primID-slot order (x, y, z and the primID's bits),
+// a contiguous run instead of a primID load and a gather each.
+template <bool kSorted>
+struct LeafPoints {
+  const uint32_t *primIDs;
+  const float *points;
+  const float4 *spts;
+  __device__ __forceinline__ unsigned long long operator()(uint32_t off, uint32_t cnt, float x, float y,
+                                                           float z) const {
+    unsigned long long best = ~0ull;
+    for (uint32_t j = 0; j < cnt; j += 4) {
+      float4 p[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const uint32_t slot = off + min(j + u, cnt - 1);
+        if constexpr (kSorted) {
+          p[u] = spts[slot];
+        } else {
+          const uint32_t id = primIDs[slot];
+          const float3 v = load_pt(points, id);
+          p[u] = make_float4(v.x, v.y, v.z, __uint_as_float(id));
+        }
+      }
+      // (the last prim again changes nothing)
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const unsigned long long k =
+            closest_key(cubql_dev::sqr_dist_pt(p[u].x, p[u].y, p[u].z, x, y, z), __float_as_uint(p[u].w));
+        best = k < best ? k : best;
+      }
     }
-    return bestD;
-  };
-  cubql_dev::NoStats st;
-  const uint32_t seed = cubql_dev::visit_nearest_leaf(bvh, q.x, q.y, q.z, prim, 0u, st);
-  return cubql_dev::for_each_prim_except_on(stack, bvh, q.x, q.y, q.z, bestD, prim, seed, 0u, st);
-}
+    return best;
+  }
+};
 
-// The same with the leaf prims read from a copy of the points in primID-slot
-// order (x, y, z and the primID's bits): a leaf's prims are one contiguous
-// run instead of a primID load and a gather each.  Tests the same prims in
-// the same order, so the result is the same.
-template <typename StackT>
-__device__ __forceinline__ bool fcp_sorted_on(StackT &stack, const cubql_bvh3f &bvh, const float4 *spts, float3 q,
-                                              float sqrMax, int32_t &best, float &bestD) {
-  best = -1;
-  bestD = sqrMax;
-  auto test = [&](uint32_t slot) {
-    const float4 p = spts[slot];
-    const float d = cubql_dev::sqr_dist_pt(p.x, p.y, p.z, q.x, q.y, q.z);
-    const int32_t pid = (int32_t)__float_as_uint(p.w);
-    if (d < bestD || (d == bestD && best >= 0 && pid < best)) {
-      bestD = d;
-      best = pid;
-    }
-  };
-  cubql_dev::NoStats st;
-  const uint64_t seedLeaf = cubql_dev::nearest_leaf(bvh, q.x, q.y, q.z, 0u, st);
-  const uint32_t seed = cubql_dev::oc_off(seedLeaf);
-  for (uint32_t j = 0; j < cubql_dev::oc_cnt(seedLeaf); j++) test(seed + j);
-  auto leaf = [&](const uint32_t *ids, uint32_t cnt) -> float {
-    const uint32_t off = (uint32_t)(ids - bvh.primIDs);
-    if (off == seed) return INFINITY;
-    for (uint32_t j = 0; j < cnt; j++) test(off + j);
-    return bestD;
-  };
-  return cubql_dev::for_each_leaf_on(stack, bvh, q.x, q.y, q.z, bestD, leaf, 0u, st);
-}
-
-// points in primID-slot order for fcp_sorted_on
+// points in primID-slot order
 __global__ __launch_bounds__(256) void k_slot_points(const uint32_t *primIDs, uint32_t numPrims, const float *points,
                                                      float4 *spts) {
   for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < numPrims; t += gridDim.x * 256) {
@@ -115,40 +106,52 @@ __global__ __launch_bounds__(256) void k_slot_points(const uint32_t *primIDs, ui
   }
 }
 
-// Entries of the fast kernel's LDS stack per lane: the seeded radius keeps
-// a closest-point query's stack shallow, and 8 entries x 8 bytes x 256 lanes
-// (16 KB a workgroup) leave the kernel at full occupancy; deeper queries
-// rerun in the deep kernel.
-constexpr int kLdsStack = 8;
-
-// fast path: an 8-entry LDS stack over a binary tree, a 64-entry private
-// stack over a wide one; queries that overflow go to the deep kernel.
-// BVH: cubql_bvh3f (binary) or cubql_dev::WideBVH<W>.
-// kSorted (binary trees): leaf prims from spts, the points in primID-slot order.
-template <typename BVH, bool kSorted = false>
-__global__ __launch_bounds__(kBlock) void k_fcp(BVH bvh, const float *points, const float4 *spts,
-                                                const float *queries, uint32_t nq, float sqrMax,
-                                                int32_t *outIds, float *outD, Overflow *ovf,
-                                                uint32_t *ovfList, const uint32_t *order) {
+// Closest points over a binary tree: a wave per qpw queries (wave_closest.h).
+// 10M queries of 10M points: 3.70 ms and 0.13 ms of reruns with one query per
+// lane on an 8-entry LDS stack, 1.62 ms here, bound by VALU issue.
+// Queries that lose a task to a full queue go to the deep kernel.
+template <bool kSorted>
+__global__ __launch_bounds__(kBlock) void k_fcp(cubql_bvh3f bvh, const float *points, const float4 *spts,
+                                                const float *queries, uint32_t nq, uint32_t qpw, float sqrMax,
+                                                int32_t *outIds, float *outD, Overflow *ovf, uint32_t *ovfList,
+                                                const uint32_t *order) {
+  __shared__ WaveTasks tasks[kBlock / kWave];
+  const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
   // Morton-ordered queries: one contiguous run of them per XCD
+  const uint32_t b = order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint64_t i = (uint64_t)(b * (kBlock / kWave) + wave) * qpw + lane;
+  const bool live = lane < qpw && i < nq;
+  const uint32_t qi = live ? (order ? order[i] : (uint32_t)i) : 0u;
+  float3 q = make_float3(0.f, 0.f, 0.f);
+  if (live) q = load_pt(queries, qi);
+  const unsigned long long none = closest_none(sqrMax);
+  bool failed;
+  const unsigned long long best =
+      wave_closest(tasks[wave], bvh.nodes, live, bvh.nodes[0].offsetAndCountBits, q.x, q.y, q.z, none,
+                   LeafPoints<kSorted>{bvh.primIDs, points, spts}, &failed);
+  if (!live) return;
+  if (failed) {
+    ovfList[atomicAdd(&ovf->count, 1u)] = qi;
+    return;
+  }
+  const bool found = best != none;
+  outIds[qi] = found ? (int32_t)(uint32_t)best : -1;
+  if (outD) outD[qi] = found ? __uint_as_float((uint32_t)(best >> 32)) : INFINITY;
+}
+
+// Closest points over a wide tree: one query per lane, a 64-entry private
+// stack; queries that overflow it go to the deep kernel.
+template <typename BVH>
+__global__ __launch_bounds__(kBlock) void k_fcp_wide(BVH bvh, const float *points, const float *queries, uint32_t nq,
+                                                     float sqrMax, int32_t *outIds, float *outD, Overflow *ovf,
+                                                     uint32_t *ovfList, const uint32_t *order) {
   const uint32_t i = (order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x) * kBlock + threadIdx.x;
   if (i >= nq) return;
   const uint32_t qi = order ? order[i] : i;
-  float3 q = load_pt(queries, qi);
   int32_t best;
   float bestD;
-  bool done;
-  if constexpr (std::is_same<BVH, cubql_bvh3f>::value) {
-    __shared__ uint2 sStack[kLdsStack * kBlock];
-    cubql_dev::LdsStack<kLdsStack, kBlock> stack(sStack + threadIdx.x);
-    if constexpr (kSorted) done = fcp_sorted_on(stack, bvh, spts, q, sqrMax, best, bestD);
-    else done = fcp_one_on(stack, bvh, points, q, sqrMax, best, bestD);
-  } else {
-    done = fcp_one<kFastStack>(bvh, points, q, sqrMax, best, bestD);
-  }
-  if (!done) {
-    uint32_t slot = atomicAdd(&ovf->count, 1u);
-    ovfList[slot] = qi;
+  if (!fcp_one<kFastStack>(bvh, points, load_pt(queries, qi), sqrMax, best, bestD)) {
+    ovfList[atomicAdd(&ovf->count, 1u)] = qi;
     return;
   }
   outIds[qi] = best;
@@ -593,6 +596,14 @@ const cubql_box3f *root_box_ws(const cubql_dev::WideBVH<W> &bvh, hipStream_t s, 
   return b;
 }
 
+// Queries of one wave: 64 once they fill the chip, fewer for small batches,
+// whose time is one wave's chain of dependent loads.
+inline uint32_t queries_per_wave(uint32_t nq) {
+  uint32_t w = 1;
+  while (w < (uint32_t)kWave && (uint64_t)w * kWavesWanted < nq) w *= 2;
+  return w;
+}
+
 // Closest-point queries on a caller-provided workspace of fcp_ws_bytes(nq)
 // bytes; allocates nothing.  With spts (binary trees: numPrims float4 slots)
 // the points are first copied into primID-slot order and the leaves read
@@ -617,21 +628,22 @@ int fcp_run_ws(const BVH &bvh, const float *d_points, const float *d_queries, ui
     CUBQL_CHECK(query_order_box_ws(rootBox, d_queries, numQueries, s,
                                    ws + kWsList + align256((size_t)numQueries * 4), &order));
   int ps = prof_begin(s);
-  bool sorted = false;
   if constexpr (std::is_same<BVH, cubql_bvh3f>::value) {
+    const uint32_t qpw = queries_per_wave(numQueries);
+    const uint32_t grid = div_up(div_up(numQueries, qpw), kBlock / kWave);
     if (spts) {
       k_slot_points<<<std::max(1u, std::min(div_up(bvh.numPrims, 256u), 2048u)), 256, 0, s>>>(
           bvh.primIDs, bvh.numPrims, d_points, spts);
-      k_fcp<BVH, true><<<div_up(numQueries, kBlock), kBlock, 0, s>>>(bvh, d_points, spts, d_queries, numQueries,
-                                                                     sqrMaxSearchDist, d_outIDs, d_outSqrDist, ovf,
-                                                                     ovfList, order);
-      sorted = true;
+      k_fcp<true><<<grid, kBlock, 0, s>>>(bvh, d_points, spts, d_queries, numQueries, qpw, sqrMaxSearchDist, d_outIDs,
+                                          d_outSqrDist, ovf, ovfList, order);
+    } else {
+      k_fcp<false><<<grid, kBlock, 0, s>>>(bvh, d_points, nullptr, d_queries, numQueries, qpw, sqrMaxSearchDist,
+                                           d_outIDs, d_outSqrDist, ovf, ovfList, order);
     }
-  }
-  if (!sorted) {
-    k_fcp<BVH><<<div_up(numQueries, kBlock), kBlock, 0, s>>>(bvh, d_points, nullptr, d_queries, numQueries,
-                                                             sqrMaxSearchDist, d_outIDs, d_outSqrDist, ovf, ovfList,
-                                                             order);
+  } else {
+    k_fcp_wide<BVH><<<div_up(numQueries, kBlock), kBlock, 0, s>>>(bvh, d_points, d_queries, numQueries,
+                                                                  sqrMaxSearchDist, d_outIDs, d_outSqrDist, ovf,
+                                                                  ovfList, order);
   }
   prof_end(ps, s, profName);
   // compulsory bytes only: query in, id + distance out

@@ -1,0 +1,222 @@
+// wave_closest.h -- closest-prim queries whose traversal is shared by a wave.
+//
+// One query per lane leaves a wave64 mostly idle: after the two descents to
+// the nearest leaf a query visits one or two more subtrees on average, but a
+// wave waits for its slowest query (10M uniform points and queries: 123 of
+// its 167 node-pair iterations were such side visits, with 4% of the lanes
+// on, and the node loads of those few lanes kept the address unit busy 92%
+// of the time).  Here a wave's queries keep their coordinates and best
+// (distance, id) in LDS, and every subtree still to visit is a task in the
+// wave's LDS queue that any free lane takes.
+//
+// The result does not depend on who visits what: it is the minimum of
+// (squared distance bits << 32 | id) over the prims within the radius, and a
+// task is dropped only if its box is farther than the query's best.
+//
+// Two descents come first.  (1) Every query descends along its nearer
+// children (ties to the second) to one leaf and tests its prims.  (2) It
+// walks the same path again with that radius and queues the far children
+// still within it.  While all queries of the wave are at the same node --
+// queries come in Morton order -- its pair of children is read once per wave
+// through the scalar cache.
+#pragma once
+#include "common.h"
+#include "cubql_amd/traversal.hip.h"
+
+namespace cubql {
+
+typedef float vec4f __attribute__((ext_vector_type(4)));
+
+// The child pair at nodes[i0], i0 the same in every lane: scalar loads.
+__device__ __forceinline__ void load_pair_uniform(const cubql_node3f *nodes, uint32_t i0, cubql_dev::QNode &n0,
+                                                  cubql_dev::QNode &n1) {
+  typedef const __attribute__((address_space(4))) vec4f *cptr;
+  cptr p = (cptr)(uintptr_t)(nodes + i0);
+  const vec4f a = p[0], b = p[1], c = p[2], d = p[3];
+  n0.a = make_float4(a.x, a.y, a.z, a.w);
+  n0.b = make_float4(b.x, b.y, b.z, b.w);
+  n1.a = make_float4(c.x, c.y, c.z, c.w);
+  n1.b = make_float4(d.x, d.y, d.z, d.w);
+}
+
+// Queue slots of a wave.  A task is {offset, distance with the query's lane
+// in its low 6 bits (rounded down: the test only gets weaker)} and the
+// prim count (0: an inner node).
+constexpr int kTaskCap = 512;
+// lanes at a leaf before the wave stops expanding nodes to test their prims
+constexpr int kLeafLanes = 24;
+// steps of one descent after which a query goes to the deep kernel (the
+// depth that kernel's stack holds)
+constexpr uint32_t kMaxSteps = 1024;
+
+struct WaveTasks {
+  uint2 task[kTaskCap];
+  unsigned long long best[kWave];
+  float q[3][kWave];
+  uint32_t failed[2];  // queries that lost a task to a full queue
+  uint16_t cnt[kTaskCap];
+};
+
+// Key of "nothing found within sqrMax": prims must be strictly nearer.
+__device__ __forceinline__ unsigned long long closest_none(float sqrMax) {
+  return (unsigned long long)(sqrMax > 0.f ? __float_as_uint(sqrMax) : 0u) << 32;
+}
+__device__ __forceinline__ unsigned long long closest_key(float d, uint32_t id) {
+  return ((unsigned long long)__float_as_uint(d) << 32) | id;
+}
+
+// All 64 lanes of the wave call this; lanes with `live` hold a query and the
+// offset/count word of its root.  leaf(off, cnt, x, y, z) returns the least
+// key of a leaf's prims (~0 if none).  Returns the lane's best key; *failed
+// is set if the query has to be rerun with a deeper stack.
+template <typename LeafFn>
+__device__ __forceinline__ unsigned long long wave_closest(WaveTasks &sh, const cubql_node3f *nodes, bool live,
+                                                           uint64_t rootWord, float x, float y, float z,
+                                                           unsigned long long none, LeafFn &&leaf, bool *failed) {
+  using namespace cubql_dev;
+  const uint32_t lane = lane_id();
+  unsigned long long best = none;
+  // (1) nearest leaf
+  if (live) {
+    uint32_t off = oc_off(rootWord), cnt = oc_cnt(rootWord);
+    while (cnt == 0) {
+      const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)off);
+      if (__ballot(off == u) != __ballot(true)) break;
+      QNode n0, n1;
+      load_pair_uniform(nodes, u, n0, n1);
+      const bool near0 = sqr_dist_box(x, y, z, n0) < sqr_dist_box(x, y, z, n1);
+      const uint64_t oc = near0 ? node_oc(n0) : node_oc(n1);
+      off = oc_off(oc);
+      cnt = oc_cnt(oc);
+    }
+    while (cnt == 0) {
+      const QNode n0 = load_node(nodes, off), n1 = load_node(nodes, off + 1);
+      const bool near0 = sqr_dist_box(x, y, z, n0) < sqr_dist_box(x, y, z, n1);
+      const uint64_t oc = near0 ? node_oc(n0) : node_oc(n1);
+      off = oc_off(oc);
+      cnt = oc_cnt(oc);
+    }
+    const unsigned long long k = leaf(off, cnt, x, y, z);
+    best = k < best ? k : best;
+  }
+  sh.best[lane] = best;
+  sh.q[0][lane] = x;
+  sh.q[1][lane] = y;
+  sh.q[2][lane] = z;
+  if (lane < 2) sh.failed[lane] = 0u;
+  sync_wave_lds();
+  // (2) the same path again, then the queued subtrees.  Every lane stays in
+  // these loops; what a lane does follows from its state.
+  enum : uint32_t { kFree, kInner, kLeaf };
+  float cull = __uint_as_float((uint32_t)(best >> 32));
+  uint32_t off = oc_off(rootWord), cnt = 0, q = lane, steps = 0;
+  uint32_t state = live && oc_cnt(rootWord) == 0 ? kInner : kFree;
+  bool main = true;  // on the path of (1), whose leaf is tested
+  uint32_t qn = 0;
+  auto expand = [&](const QNode &n0, const QNode &n1, bool on, bool &push, uint2 &t, uint32_t &c) {
+    const float d0 = sqr_dist_box(x, y, z, n0), d1 = sqr_dist_box(x, y, z, n1);
+    const bool near0 = d0 < d1;
+    const uint64_t ocN = near0 ? node_oc(n0) : node_oc(n1), ocF = near0 ? node_oc(n1) : node_oc(n0);
+    const float dn = fminf(d0, d1), df = fmaxf(d0, d1);
+    push = on && df <= cull;
+    t = make_uint2(oc_off(ocF), (__float_as_uint(df) & ~63u) | q);
+    c = oc_cnt(ocF);
+    if (on) {
+      off = oc_off(ocN);
+      cnt = oc_cnt(ocN);
+      state = dn > cull ? kFree : cnt == 0 ? kInner : main ? kFree : kLeaf;
+    }
+  };
+  auto enqueue = [&](bool push, uint2 t, uint32_t c) {
+    const uint64_t m = __ballot(push);
+    if (!m) return;
+    const uint32_t slot = qn + mbcnt(m);
+    if (push) {
+      if (slot < (uint32_t)kTaskCap) {
+        sh.task[slot] = t;
+        sh.cnt[slot] = (uint16_t)c;
+      } else {
+        atomicOr(&sh.failed[q >> 5], 1u << (q & 31));
+      }
+    }
+    qn = min(qn + (uint32_t)__popcll(m), (uint32_t)kTaskCap);
+    sync_wave_lds();
+  };
+  while (true) {
+    const uint64_t m = __ballot(state == kInner);
+    if (!m) break;
+    const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)off, __builtin_ctzll(m));
+    if (__ballot(state == kInner && off == u) != m) break;
+    QNode n0, n1;
+    load_pair_uniform(nodes, u, n0, n1);
+    bool push;
+    uint2 t;
+    uint32_t c;
+    expand(n0, n1, state == kInner, push, t, c);
+    if (++steps > kMaxSteps && state == kInner) {
+      atomicOr(&sh.failed[q >> 5], 1u << (q & 31));
+      state = kFree;
+    }
+    enqueue(push, t, c);
+  }
+  while (true) {
+    const uint64_t freeM = __ballot(state == kFree);
+    if (qn && freeM) {
+      // newest tasks first
+      const uint32_t r = mbcnt(freeM);
+      if (state == kFree && r < qn) {
+        const uint2 t = sh.task[qn - 1 - r];
+        const uint32_t c = sh.cnt[qn - 1 - r];
+        q = t.y & 63u;
+        cull = __uint_as_float((uint32_t)(sh.best[q] >> 32));
+        if (__uint_as_float(t.y & ~63u) <= cull) {
+          x = sh.q[0][q];
+          y = sh.q[1][q];
+          z = sh.q[2][q];
+          off = t.x;
+          cnt = c;
+          steps = 0;
+          main = false;
+          state = c ? kLeaf : kInner;
+        }
+      }
+      qn -= min(qn, (uint32_t)__popcll(freeM));
+      sync_wave_lds();
+    }
+    const uint64_t inner = __ballot(state == kInner), leafM = __ballot(state == kLeaf);
+    if (!(inner | leafM)) {
+      if (!qn) break;
+      continue;
+    }
+    if (inner && __popcll(leafM) < kLeafLanes) {
+      bool on = state == kInner;
+      // a nearly full queue: only as many lanes expand as it has room for
+      const uint32_t room = (uint32_t)kTaskCap - qn;
+      if (room && room < (uint32_t)__popcll(inner)) on = on && mbcnt(inner) < room;
+      bool push = false;
+      uint2 t = make_uint2(0u, 0u);
+      uint32_t c = 0;
+      if (on) {
+        const QNode n0 = load_node(nodes, off), n1 = load_node(nodes, off + 1);
+        expand(n0, n1, true, push, t, c);
+        if (++steps > kMaxSteps && state == kInner) {
+          atomicOr(&sh.failed[q >> 5], 1u << (q & 31));
+          state = kFree;
+        }
+      }
+      enqueue(push, t, c);
+    } else {
+      if (state == kLeaf) {
+        const unsigned long long k = leaf(off, cnt, x, y, z);
+        atomicMin(&sh.best[q], k);
+        state = kFree;
+      }
+      sync_wave_lds();
+    }
+  }
+  sync_wave_lds();
+  *failed = (sh.failed[lane >> 5] >> (lane & 31)) & 1u;
+  return sh.best[lane];
+}
+
+}  // namespace cubql
