@@ -15,8 +15,9 @@
 //     cloud's root, and its subtree is exactly the tree radix30Builder builds
 //     for the cloud alone;
 //   * exact bottom-up refit.
-// Queries run one per lane over all clouds, in Morton order of the query
-// side, each from its cloud's root in the other side's forest; the adjoint of
+// Queries run over all clouds in Morton order of the query side, each from
+// its cloud's root in the other side's forest, a wave sharing its queries'
+// subtrees; the adjoint of
 // loss[c] = mean_i d(s_i, T_c) + mean_j d(t_j, S_c) is scatter-added.  The
 // whole sequence is a fixed number of launches on one stream with no host
 // synchronisation and no allocation (caller workspace), so it can be
@@ -27,6 +28,7 @@
 #include "cubql_amd/traversal.hip.h"
 #include "profile.h"
 #include "radix_sort.h"
+#include "wave_closest.h"
 
 #include <algorithm>
 #include <vector>
@@ -243,13 +245,12 @@ __global__ void k_brefit_level(Side sd, Temp tp, int level) {
   }
 }
 
-// The closest point of one query in the tree at `root`, on a caller's
-// traversal stack (a private array, or LDS for the shallow stacks): its
+// The closest point of one query in the tree at `root` on the deep stack: its
 // global index (lowest among equal distances), its sorted slot and distance.
 // Leaf prims are read from the sorted points, a contiguous run per leaf.
-template <typename StackT>
-__device__ __forceinline__ bool fcp_forest_on(StackT &stack, const Side &tgt, uint32_t root, float3 q,
-                                              int32_t &best, uint32_t &bestSlot, float &bestD) {
+template <int STACK>
+__device__ __forceinline__ bool fcp_forest(const Side &tgt, uint32_t root, float3 q, int32_t &best,
+                                           uint32_t &bestSlot, float &bestD) {
   best = -1;
   bestSlot = kNoSlot;
   bestD = INFINITY;
@@ -259,71 +260,85 @@ __device__ __forceinline__ bool fcp_forest_on(StackT &stack, const Side &tgt, ui
   bvh.primIDs = tgt.ids;  // only for leaf slot offsets: ids are not read
   bvh.numPrims = tgt.n;
   const float4 *spts = tgt.spts;
-  auto test = [&](uint32_t slot) {
-    const float4 p = spts[slot];
-    const float d = cubql_dev::sqr_dist_pt(p.x, p.y, p.z, q.x, q.y, q.z);
-    const int32_t pid = (int32_t)__float_as_uint(p.w);
-    if (d < bestD || (d == bestD && best >= 0 && pid < best)) {
-      bestD = d;
-      best = pid;
-      bestSlot = slot;
-    }
-  };
-  // seed the radius with the nearest-child leaf, which the traversal then
-  // leaves out
-  cubql_dev::NoStats st;
-  const uint64_t seedLeaf = cubql_dev::nearest_leaf(bvh, q.x, q.y, q.z, root, st);
-  const uint32_t seed = cubql_dev::oc_off(seedLeaf);
-  for (uint32_t j = 0; j < cubql_dev::oc_cnt(seedLeaf); j++) test(seed + j);
   auto leaf = [&](const uint32_t *ids, uint32_t cnt) -> float {
     const uint32_t off = (uint32_t)(ids - tgt.ids);
-    if (off == seed) return INFINITY;
-    for (uint32_t j = 0; j < cnt; j++) test(off + j);
+    for (uint32_t j = 0; j < cnt; j++) {
+      const float4 p = spts[off + j];
+      const float d = cubql_dev::sqr_dist_pt(p.x, p.y, p.z, q.x, q.y, q.z);
+      const int32_t pid = (int32_t)__float_as_uint(p.w);
+      if (d < bestD || (d == bestD && best >= 0 && pid < best)) {
+        bestD = d;
+        best = pid;
+        bestSlot = off + j;
+      }
+    }
     return bestD;
   };
-  return cubql_dev::for_each_leaf_on(stack, bvh, q.x, q.y, q.z, bestD, leaf, root, st);
-}
-template <int STACK>
-__device__ __forceinline__ bool fcp_forest(const Side &tgt, uint32_t root, float3 q, int32_t &best,
-                                           uint32_t &bestSlot, float &bestD) {
-  cubql_dev::PrivateStack<STACK> stack;
-  return fcp_forest_on(stack, tgt, root, q, best, bestSlot, bestD);
+  return cubql_dev::for_each_leaf<STACK>(bvh, q.x, q.y, q.z, bestD, leaf, root);
 }
 
-// queries of side `qs` against the forest of side `ts`, in Morton order of qs
-template <int BLOCK, int STACK>
-__global__ __launch_bounds__(BLOCK) void k_bquery(Side qs, Side ts, int32_t *nn, float *d2, uint32_t *ovf) {
-  // queries sorted by (cloud, Morton key): one contiguous run per XCD
-  const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
-  if (t >= qs.n) return;
-  const float4 qv = qs.spts[t];
-  const uint32_t qi = __float_as_uint(qv.w);
-  const uint32_t cloud = (uint32_t)(qs.keys[t] >> kCloudShift);
-  const uint32_t root = ts.rootOf[cloud];
-  int32_t best = -1;
-  uint32_t bestSlot = kNoSlot;
-  float bestD = INFINITY;
-  if (root != kNoRoot) {
-    const float3 q = make_float3(qv.x, qv.y, qv.z);
-    bool done;
-    if constexpr (STACK <= 16) {
-      // shallow stacks live in LDS (at most 32 KB a workgroup), deeper
-      // ones in the lane's private memory
-      __shared__ uint2 sStack[STACK * BLOCK];
-      cubql_dev::LdsStack<STACK, BLOCK> stack(sStack + threadIdx.x);
-      done = fcp_forest_on(stack, ts, root, q, best, bestSlot, bestD);
-    } else {
-      done = fcp_forest<STACK>(ts, root, q, best, bestSlot, bestD);
+// Least key of a leaf's points and the sorted slot it is at, four in flight.
+struct LeafSlots {
+  const float4 *spts;
+  __device__ __forceinline__ unsigned long long operator()(uint32_t off, uint32_t cnt, float x, float y, float z,
+                                                           uint32_t &at) const {
+    unsigned long long best = ~0ull;
+    for (uint32_t j = 0; j < cnt; j += 4) {
+      float4 p[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) p[u] = spts[off + min(j + u, cnt - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const unsigned long long k =
+            closest_key(cubql_dev::sqr_dist_pt(p[u].x, p[u].y, p[u].z, x, y, z), __float_as_uint(p[u].w));
+        if (k < best) {
+          best = k;
+          at = off + min(j + u, cnt - 1);
+        }
+      }
     }
-    if (!done) {
-      ovf[2 + atomicAdd(&ovf[0], 1u)] = t;
-      return;
-    }
+    return best;
   }
-  nn[qi] = best;
-  d2[qi] = bestD;
-  qs.nnS[t] = bestSlot;
-  qs.d2S[t] = bestD;
+};
+
+// (24 and 40 lanes: within 1%)
+constexpr int kBatchLeafLanes = 32;
+
+// queries of side `qs` against the forest of side `ts`, in Morton order of
+// qs: a wave per qpw queries (wave_closest.h).  2 x 38M queries over 4096
+// clouds: 16.5 ms with one query per lane on a private stack, 8.2 ms here;
+// bound by the address unit (16-point leaves) and VALU issue.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_bquery(Side qs, Side ts, uint32_t qpw, int32_t *nn, float *d2,
+                                                  uint32_t *ovf) {
+  __shared__ WaveTasksAux tasks[BLOCK / kWave];
+  const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
+  // queries sorted by (cloud, Morton key): one contiguous run per XCD
+  const uint64_t i = (uint64_t)(xcd_chunk(blockIdx.x, gridDim.x) * (BLOCK / kWave) + wave) * qpw + lane;
+  const bool act = lane < qpw && i < qs.n;
+  const uint32_t t = act ? (uint32_t)i : 0u;
+  const float4 qv = qs.spts[t];
+  const uint32_t root = ts.rootOf[(uint32_t)(qs.keys[t] >> kCloudShift)];
+  const bool live = act && root != kNoRoot;
+  const uint64_t word = live ? ts.nodes[root].oc : 0ull;
+  const unsigned long long none = closest_none(INFINITY);
+  bool failed;
+  uint32_t slot;
+  const unsigned long long best =
+      wave_closest<kBatchLeafLanes>(tasks[wave], (const cubql_node3f *)ts.nodes, live, word, qv.x, qv.y, qv.z, none,
+                                    LeafSlots{ts.spts}, &failed, &slot);
+  if (!act) return;
+  if (live && failed) {
+    ovf[2 + atomicAdd(&ovf[0], 1u)] = t;
+    return;
+  }
+  const uint32_t qi = __float_as_uint(qv.w);
+  const bool found = best != none;
+  const float d = found ? __uint_as_float((uint32_t)(best >> 32)) : INFINITY;
+  nn[qi] = found ? (int32_t)(uint32_t)best : -1;
+  d2[qi] = d;
+  qs.nnS[t] = found ? slot : kNoSlot;
+  qs.d2S[t] = d;
 }
 
 __global__ __launch_bounds__(64) void k_bquery_deep(Side qs, Side ts, int32_t *nn, float *d2, uint32_t *ovf) {
@@ -533,28 +548,21 @@ int build_side(Side &sd, Temp &tp, const Args &a, const Plan &pl, hipStream_t s,
   return CUBQL_OK;
 }
 
-template <int BLOCK, int STACK>
+template <int BLOCK>
 void launch_query(const Side &q, const Side &t, int32_t *nn, float *d2, uint32_t *ovf, hipStream_t s) {
-  k_bquery<BLOCK, STACK><<<div_up(std::max(q.n, 1u), BLOCK), BLOCK, 0, s>>>(q, t, nn, d2, ovf);
-}
-
-template <int STACK>
-void launch_query_b(int block, const Side &q, const Side &t, int32_t *nn, float *d2, uint32_t *ovf,
-                    hipStream_t s) {
-  if (block == 64) launch_query<64, STACK>(q, t, nn, d2, ovf, s);
-  else if (block == 128) launch_query<128, STACK>(q, t, nn, d2, ovf, s);
-  else launch_query<256, STACK>(q, t, nn, d2, ovf, s);
+  const uint32_t qpw = queries_per_wave(q.n);
+  k_bquery<BLOCK><<<div_up(div_up(q.n, qpw), BLOCK / kWave), BLOCK, 0, s>>>(q, t, qpw, nn, d2, ovf);
 }
 
 int query_dir(const Side &q, const Side &t, int32_t *nn, float *d2, uint32_t *ovf, const cubql_batch_params &p,
               hipStream_t s) {
   if (q.n == 0) return CUBQL_OK;
   CUBQL_CHECK(fill_u32(ovf, 0u, 2, s));
-  const int b = p.blockSize, st = p.stackDepth;
-  if (st == 8) launch_query_b<8>(b, q, t, nn, d2, ovf, s);
-  else if (st == 16) launch_query_b<16>(b, q, t, nn, d2, ovf, s);
-  else if (st == 32) launch_query_b<32>(b, q, t, nn, d2, ovf, s);
-  else launch_query_b<64>(b, q, t, nn, d2, ovf, s);
+  // (stackDepth picks nothing any more: a wave's queue has taken the place
+  // of the lanes' stacks)
+  if (p.blockSize == 64) launch_query<64>(q, t, nn, d2, ovf, s);
+  else if (p.blockSize == 128) launch_query<128>(q, t, nn, d2, ovf, s);
+  else launch_query<256>(q, t, nn, d2, ovf, s);
   k_bquery_deep<<<64, 64, 0, s>>>(q, t, nn, d2, ovf);
   CUBQL_LAUNCH_CHECK();
   return CUBQL_OK;

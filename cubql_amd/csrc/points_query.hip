@@ -29,11 +29,6 @@ __device__ __forceinline__ float3 load_pt(const float *p, uint32_t i) {
   return make_float3(p[3 * (size_t)i + 0], p[3 * (size_t)i + 1], p[3 * (size_t)i + 2]);
 }
 
-// Waves that a small closest-point batch is spread over: 1000 queries of 1M
-// points take 25.6 us as 1000 waves of one query, whose subtrees the other
-// lanes take, and took 87.7 us as 16 waves of one query per lane.
-constexpr uint32_t kWavesWanted = 4096;
-
 struct Overflow {
   uint32_t count;
   uint32_t deepFailed;
@@ -68,8 +63,8 @@ struct LeafPoints {
   const uint32_t *primIDs;
   const float *points;
   const float4 *spts;
-  __device__ __forceinline__ unsigned long long operator()(uint32_t off, uint32_t cnt, float x, float y,
-                                                           float z) const {
+  __device__ __forceinline__ unsigned long long operator()(uint32_t off, uint32_t cnt, float x, float y, float z,
+                                                           uint32_t &) const {
     unsigned long long best = ~0ull;
     for (uint32_t j = 0; j < cnt; j += 4) {
       float4 p[4];
@@ -106,9 +101,12 @@ __global__ __launch_bounds__(256) void k_slot_points(const uint32_t *primIDs, ui
   }
 }
 
+// (12 lanes: 2% slower, 36 and 48 the same)
+constexpr int kFcpLeafLanes = 24;
+
 // Closest points over a binary tree: a wave per qpw queries (wave_closest.h).
 // 10M queries of 10M points: 3.70 ms and 0.13 ms of reruns with one query per
-// lane on an 8-entry LDS stack, 1.62 ms here, bound by VALU issue.
+// lane on an 8-entry LDS stack, 1.47 ms here, bound by VALU issue.
 // Queries that lose a task to a full queue go to the deep kernel.
 template <bool kSorted>
 __global__ __launch_bounds__(kBlock) void k_fcp(cubql_bvh3f bvh, const float *points, const float4 *spts,
@@ -127,7 +125,7 @@ __global__ __launch_bounds__(kBlock) void k_fcp(cubql_bvh3f bvh, const float *po
   const unsigned long long none = closest_none(sqrMax);
   bool failed;
   const unsigned long long best =
-      wave_closest(tasks[wave], bvh.nodes, live, bvh.nodes[0].offsetAndCountBits, q.x, q.y, q.z, none,
+      wave_closest<kFcpLeafLanes>(tasks[wave], bvh.nodes, live, bvh.nodes[0].offsetAndCountBits, q.x, q.y, q.z, none,
                    LeafPoints<kSorted>{bvh.primIDs, points, spts}, &failed);
   if (!live) return;
   if (failed) {
@@ -594,14 +592,6 @@ const cubql_box3f *root_box_ws(const cubql_dev::WideBVH<W> &bvh, hipStream_t s, 
   cubql_box3f *b = (cubql_box3f *)(ws + kWsRoot);
   k_wide_root_box<W><<<1, 64, 0, s>>>((const cubql_wide_child3f *)bvh.nodes, b);
   return b;
-}
-
-// Queries of one wave: 64 once they fill the chip, fewer for small batches,
-// whose time is one wave's chain of dependent loads.
-inline uint32_t queries_per_wave(uint32_t nq) {
-  uint32_t w = 1;
-  while (w < (uint32_t)kWave && (uint64_t)w * kWavesWanted < nq) w *= 2;
-  return w;
 }
 
 // Closest-point queries on a caller-provided workspace of fcp_ws_bytes(nq)

@@ -20,6 +20,8 @@
 // queries come in Morton order -- its pair of children is read once per wave
 // through the scalar cache.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "cubql_amd/traversal.hip.h"
 
@@ -39,12 +41,12 @@ __device__ __forceinline__ void load_pair_uniform(const cubql_node3f *nodes, uin
   n1.b = make_float4(d.x, d.y, d.z, d.w);
 }
 
-// Queue slots of a wave.  A task is {offset, distance with the query's lane
+// Queue slots of a wave: 512 leave fewer waves in flight (10M queries of 10M
+// points: 2.21 ms a call against 2.04 ms), 256 send more queries of clustered
+// and Gaussian clouds to the deep kernel.  A task is {offset, distance with the query's lane
 // in its low 6 bits (rounded down: the test only gets weaker)} and the
 // prim count (0: an inner node).
-constexpr int kTaskCap = 512;
-// lanes at a leaf before the wave stops expanding nodes to test their prims
-constexpr int kLeafLanes = 24;
+constexpr int kTaskCap = 320;
 // steps of one descent after which a query goes to the deep kernel (the
 // depth that kernel's stack holds)
 constexpr uint32_t kMaxSteps = 1024;
@@ -56,6 +58,22 @@ struct WaveTasks {
   uint32_t failed[2];  // queries that lost a task to a full queue
   uint16_t cnt[kTaskCap];
 };
+// the same with a word kept beside each query's best key
+struct WaveTasksAux : WaveTasks {
+  uint32_t aux[kWave];
+};
+
+// Waves that a small batch is spread over: 1000 queries of 1M points take
+// 25.6 us as 1000 waves of one query, whose subtrees the other lanes take,
+// and took 87.7 us as 16 waves of one query per lane.
+constexpr uint32_t kWavesWanted = 4096;
+// Queries of one wave: 64 once they fill the chip, fewer for small batches,
+// whose time is one wave's chain of dependent loads.
+inline uint32_t queries_per_wave(uint32_t nq) {
+  uint32_t w = 1;
+  while (w < (uint32_t)kWave && (uint64_t)w * kWavesWanted < nq) w *= 2;
+  return w;
+}
 
 // Key of "nothing found within sqrMax": prims must be strictly nearer.
 __device__ __forceinline__ unsigned long long closest_none(float sqrMax) {
@@ -66,16 +84,22 @@ __device__ __forceinline__ unsigned long long closest_key(float d, uint32_t id) 
 }
 
 // All 64 lanes of the wave call this; lanes with `live` hold a query and the
-// offset/count word of its root.  leaf(off, cnt, x, y, z) returns the least
-// key of a leaf's prims (~0 if none).  Returns the lane's best key; *failed
-// is set if the query has to be rerun with a deeper stack.
-template <typename LeafFn>
-__device__ __forceinline__ unsigned long long wave_closest(WaveTasks &sh, const cubql_node3f *nodes, bool live,
+// offset/count word of its root.  leaf(off, cnt, x, y, z, aux) returns the
+// least key of a leaf's prims (~0 if none) and sets aux, a word that is kept
+// with the best key if Tasks is WaveTasksAux (*auxOut).  LEAF_LANES lanes at a
+// leaf make the wave stop expanding nodes and test their prims.  Returns the
+// lane's best key; *failed is set if the query has to be rerun with a deeper
+// stack.
+template <int LEAF_LANES, typename Tasks, typename LeafFn>
+__device__ __forceinline__ unsigned long long wave_closest(Tasks &sh, const cubql_node3f *nodes, bool live,
                                                            uint64_t rootWord, float x, float y, float z,
-                                                           unsigned long long none, LeafFn &&leaf, bool *failed) {
+                                                           unsigned long long none, LeafFn &&leaf, bool *failed,
+                                                           uint32_t *auxOut = nullptr) {
   using namespace cubql_dev;
+  constexpr bool kAux = std::is_same<Tasks, WaveTasksAux>::value;
   const uint32_t lane = lane_id();
   unsigned long long best = none;
+  uint32_t aux = 0;
   // (1) nearest leaf
   if (live) {
     uint32_t off = oc_off(rootWord), cnt = oc_cnt(rootWord);
@@ -96,10 +120,11 @@ __device__ __forceinline__ unsigned long long wave_closest(WaveTasks &sh, const 
       off = oc_off(oc);
       cnt = oc_cnt(oc);
     }
-    const unsigned long long k = leaf(off, cnt, x, y, z);
+    const unsigned long long k = leaf(off, cnt, x, y, z, aux);
     best = k < best ? k : best;
   }
   sh.best[lane] = best;
+  if constexpr (kAux) sh.aux[lane] = aux;
   sh.q[0][lane] = x;
   sh.q[1][lane] = y;
   sh.q[2][lane] = z;
@@ -144,7 +169,7 @@ __device__ __forceinline__ unsigned long long wave_closest(WaveTasks &sh, const 
   };
   while (true) {
     const uint64_t m = __ballot(state == kInner);
-    if (!m) break;
+    if (!m || qn + kWave > (uint32_t)kTaskCap) break;
     const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)off, __builtin_ctzll(m));
     if (__ballot(state == kInner && off == u) != m) break;
     QNode n0, n1;
@@ -188,11 +213,11 @@ __device__ __forceinline__ unsigned long long wave_closest(WaveTasks &sh, const 
       if (!qn) break;
       continue;
     }
-    if (inner && __popcll(leafM) < kLeafLanes) {
+    // a nearly full queue: only as many lanes expand as it has room for
+    const uint32_t room = (uint32_t)kTaskCap - qn;
+    if (inner && (!leafM || (room && __popcll(leafM) < LEAF_LANES))) {
       bool on = state == kInner;
-      // a nearly full queue: only as many lanes expand as it has room for
-      const uint32_t room = (uint32_t)kTaskCap - qn;
-      if (room && room < (uint32_t)__popcll(inner)) on = on && mbcnt(inner) < room;
+      if (room < (uint32_t)__popcll(inner)) on = on && mbcnt(inner) < max(room, 1u);
       bool push = false;
       uint2 t = make_uint2(0u, 0u);
       uint32_t c = 0;
@@ -207,15 +232,21 @@ __device__ __forceinline__ unsigned long long wave_closest(WaveTasks &sh, const 
       enqueue(push, t, c);
     } else {
       if (state == kLeaf) {
-        const unsigned long long k = leaf(off, cnt, x, y, z);
+        const unsigned long long k = leaf(off, cnt, x, y, z, aux);
         atomicMin(&sh.best[q], k);
         state = kFree;
+        if constexpr (kAux) {
+          // (keys of one query differ: only the lane that holds the best writes)
+          sync_wave_lds();
+          if (sh.best[q] == k) sh.aux[q] = aux;
+        }
       }
       sync_wave_lds();
     }
   }
   sync_wave_lds();
   *failed = (sh.failed[lane >> 5] >> (lane & 31)) & 1u;
+  if constexpr (kAux) *auxOut = sh.aux[lane];
   return sh.best[lane];
 }
 

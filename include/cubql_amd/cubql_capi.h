@@ -345,8 +345,9 @@ int cubql_points_distance_backward_f3(const float *d_points, uint32_t numPoints,
 /* Tunables of the batched path (chosen by cubql_amd.autotune):
    leafSize      leaf threshold T of every per-cloud tree (>= 1);
    blockSize     query workgroup size: 64, 128 or 256;
-   stackDepth    traversal stack entries before the deep fallback: 8, 16, 32
-                 or 64 (queries that need more rerun with a deeper stack);
+   stackDepth    8, 16, 32 or 64: checked, and has no effect (a query wave
+                 shares one task queue; it took the place of the lanes'
+                 traversal stacks);
    maxCloudSize  optional upper bound on any cloud's size (0 = unknown); it
                  only bounds the number of hierarchy launches. */
 typedef struct {
