@@ -4,14 +4,14 @@
 // builders (builder/cuda/radix.h:666-687, rebinMortonBuilder.h:1242-1263):
 // keys (uint32 or uint64) with uint32 values, ascending, stable.
 //
-// Design: 8-bit digits.  One histogram pass computes the digit counts of
-// every sort pass at once (per-workgroup histograms, summed in chunks with
-// one atomic per digit and chunk).  Each sort pass is then a single read + single write of the
-// data: a workgroup claims a 4096-key tile (ticket order, so it only waits
-// on tiles that running workgroups hold), ranks keys per digit with wave64
-// ballots, resolves each digit's global offset by a decoupled look-back over
-// earlier tiles, stages the tile in LDS in digit order and writes it out so
-// that consecutive lanes write consecutive addresses.
+// Design: 8-bit digits.  One pass over the keys counts the digits of every
+// sort pass at once (LDS histograms per wave, one global atomic per digit and
+// workgroup).  Each sort pass is then a single read + single write of the
+// data: a workgroup claims a tile (ticket order, so it only waits on tiles
+// that running workgroups hold), loads all its pairs, ranks keys per digit
+// with wave64 ballots, resolves each digit's global offset by a decoupled
+// look-back over earlier tiles, and writes keys and then values in digit
+// order through LDS, so that consecutive lanes write consecutive addresses.
 #pragma once
 #include "common.h"
 

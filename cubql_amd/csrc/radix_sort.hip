@@ -9,142 +9,158 @@
 namespace cubql {
 namespace rs {
 
-constexpr int kBlock = 256;
-constexpr int kNW = kBlock / kWave;        // 4 waves
-constexpr int kPerWave = 1024;             // keys per wave per tile
-constexpr int kTile = kNW * kPerWave;      // 4096 keys per tile
-constexpr int kWaveItems = kPerWave / kWave;  // 16 keys per lane
+// A tile is 512 threads x ITEMS keys, staged in LDS once for the keys and
+// once for the values.  Large sorts take large tiles (longer runs per digit:
+// 32M random 24-bit pairs 0.75 ms with 20 keys a thread, 0.84 with 12; 32M
+// 64-bit pairs 1.95 ms with 16, 2.35 with 8), small ones take 8 keys a thread,
+// so that more CUs have a tile (100K 64-bit pairs 117 us with 8, 152 with 16;
+// 1M 192 and 210).
+constexpr int kBlock = 512;
+constexpr int kSmallItems = 8;
+constexpr uint32_t kSmallSort = 1u << 21;
+template <typename K>
+constexpr int kLargeItems = sizeof(K) == 4 ? 20 : 16;
+constexpr uint32_t kDigits = 256;
 
 // status word of (tile, digit): tag(22) | flag(2) | value(32)
 __device__ __forceinline__ uint64_t st_word(uint32_t tag, uint32_t flag, uint32_t v) {
   return ((uint64_t)tag << 34) | ((uint64_t)flag << 32) | v;
 }
 
-// Digit histograms of every pass over kHistSpan tiles of keys: one partial
-// histogram per workgroup (no global atomics), counted in one LDS
-// sub-histogram per wave; k_hist_reduce sums them.
-constexpr uint32_t kHistSpan = 2;
-
+// Digit counts of every pass: a sub-histogram per wave in LDS, then one
+// global atomic per digit, pass and workgroup.
+constexpr int kHistBlock = 256;
+constexpr int kHistWaves = kHistBlock / kWave;
 template <typename K>
-__global__ __launch_bounds__(kBlock) void k_hist(const K *keys, const uint32_t *nPtr, int passes,
-                                                 uint32_t *tileHist) {
-  __shared__ uint32_t h[kNW][8][256];
-  const uint32_t n = *nPtr;
-  for (int i = threadIdx.x; i < kNW * 8 * 256; i += kBlock) (&h[0][0][0])[i] = 0;
-  __syncthreads();
-  const uint32_t w = threadIdx.x / kWave;
-  const uint32_t base = blockIdx.x * kTile * kHistSpan;
-  const uint32_t end = (uint32_t)min((uint64_t)n, (uint64_t)base + (uint64_t)kTile * kHistSpan);
-  for (uint32_t i = base + threadIdx.x; i < end; i += kBlock) {
-    const K key = keys[i];
-    for (int p = 0; p < passes; p++) atomicAdd(&h[w][p][(uint32_t)(key >> (8 * p)) & 255u], 1u);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < passes * 256; i += kBlock) {
-    uint32_t v = 0;
-    for (int ww = 0; ww < kNW; ww++) v += (&h[ww][0][0])[i];
-    tileHist[(size_t)blockIdx.x * passes * 256 + i] = v;
-  }
-}
-
-// Sum of the partial histograms: workgroup (pass, chunk) adds the rows of
-// its chunk of blocks, one atomic per digit.
-constexpr uint32_t kHistChunks = 32;
-__global__ __launch_bounds__(256) void k_hist_reduce(const uint32_t *tileHist, uint32_t numBlocks, int passes,
+__global__ __launch_bounds__(kHistBlock) void k_hist(const K *keys, const uint32_t *nPtr, int passes,
                                                      uint32_t *digitCount) {
-  const int p = blockIdx.x;
-  const uint32_t per = div_up(numBlocks, kHistChunks);
-  const uint32_t t0 = blockIdx.y * per, t1 = min(numBlocks, t0 + per);
-  uint32_t sum = 0;
-  for (uint32_t t = t0; t < t1; t++) sum += tileHist[(size_t)t * passes * 256 + p * 256 + threadIdx.x];
-  if (sum) atomicAdd(&digitCount[p * 256 + threadIdx.x], sum);
-}
-
-// exclusive scan over the digits of each pass
-__global__ __launch_bounds__(256) void k_digit_scan(const uint32_t *digitCount, uint32_t *digitBase) {
-  __shared__ uint32_t ss[256 / kWave + 1];
-  const int p = blockIdx.x;
-  uint32_t tot;
-  digitBase[p * 256 + threadIdx.x] = block_excl_scan<256>(digitCount[p * 256 + threadIdx.x], ss, &tot);
-}
-
-template <typename K>
-__global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin,
-                                                     const uint32_t *__restrict__ vin,
-                                                     K *__restrict__ kout, uint32_t *__restrict__ vout,
-                                                     const uint32_t *nPtr, int shift, uint32_t tag,
-                                                     const uint32_t *digitBase, uint64_t *status,
-                                                     uint32_t *ticket, uint32_t *err) {
-  __shared__ uint32_t sHist[kNW][256];
-  __shared__ uint32_t sTileExcl[256];
-  __shared__ uint32_t sGlob[256];
-  __shared__ uint32_t ss[256 / kWave + 1];
-  __shared__ K sK[kTile];
-  __shared__ uint32_t sV[kTile];
-  __shared__ uint32_t sTile;
+  extern __shared__ uint32_t h[];  // [kHistWaves][passes][kDigits]
   const uint32_t n = *nPtr;
-  const uint32_t numTiles = div_up(n, kTile);
+  const int words = passes * (int)kDigits;
+  for (int i = threadIdx.x; i < kHistWaves * words; i += kHistBlock) h[i] = 0;
+  __syncthreads();
+  uint32_t *hw = h + (threadIdx.x / kWave) * words;
+  constexpr int U = 4;
+  const uint64_t stride = (uint64_t)gridDim.x * kHistBlock * U;
+  for (uint64_t i0 = (uint64_t)blockIdx.x * kHistBlock * U + threadIdx.x; i0 < n; i0 += stride) {
+    K key[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint64_t i = i0 + u * kHistBlock;
+      key[u] = i < n ? keys[i] : (K)0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (i0 + u * kHistBlock < n)
+        for (int p = 0; p < passes; p++) atomicAdd(&hw[p * kDigits + ((uint32_t)(key[u] >> (8 * p)) & 255u)], 1u);
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < words; i += kHistBlock) {
+    uint32_t v = 0;
+    for (int w = 0; w < kHistWaves; w++) v += h[w * words + i];
+    if (v) atomicAdd(&digitCount[i], v);
+  }
+}
+
+// One pass over 8 key bits, a tile per workgroup.  Tiles are claimed in
+// ticket order, so every tile a look-back waits on is held by a running
+// workgroup.  What bounds it: the latency of a tile's chain (loads, ranking,
+// look-back, two copies out) against the tiles in flight; all of a thread's
+// loads are issued before the ranking, and keys and values share one LDS
+// buffer so that more tiles fit a CU.
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin,
+                                                              const uint32_t *__restrict__ vin,
+                                                              K *__restrict__ kout, uint32_t *__restrict__ vout,
+                                                              const uint32_t *nPtr, int shift, uint32_t tag,
+                                                              const uint32_t *digitCount, uint64_t *status,
+                                                              uint32_t *ticket, uint32_t *err) {
+  constexpr int BLOCK = kBlock, NW = BLOCK / kWave;
+  constexpr uint32_t TILE = BLOCK * ITEMS;
+  static_assert(BLOCK >= (int)kDigits, "one thread per digit");
+  __shared__ uint32_t sHist[NW][kDigits];
+  __shared__ uint32_t sGlob[kDigits];  // global slot of a digit's first key less its slot in the tile
+  __shared__ uint32_t ss[2][BLOCK / kWave + 1];
+  __shared__ __align__(16) unsigned char sBuf[TILE * sizeof(K)];
+  __shared__ uint32_t sTile;
+  K *const sK = reinterpret_cast<K *>(sBuf);
+  uint32_t *const sV = reinterpret_cast<uint32_t *>(sBuf);
+  const uint32_t n = *nPtr;
   const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  while (true) {
-    if (threadIdx.x == 0) sTile = atomicAdd(ticket, 1u);
-    for (int i = threadIdx.x; i < kNW * 256; i += kBlock) (&sHist[0][0])[i] = 0;
-    __syncthreads();
-    const uint32_t t = sTile;
-    if (t >= numTiles) break;
-    const uint32_t tileBase = t * kTile;
-    const uint32_t tileN = min((uint32_t)kTile, n - tileBase);
-    K key[kWaveItems];
-    uint32_t val[kWaveItems], rank[kWaveItems];
-    uint32_t dig[kWaveItems];
+  if (threadIdx.x == 0) sTile = atomicAdd(ticket, 1u);
+  for (int i = threadIdx.x; i < NW * (int)kDigits; i += BLOCK) (&sHist[0][0])[i] = 0;
+  const uint32_t dgt = threadIdx.x;
+  const uint32_t dcount = dgt < kDigits ? digitCount[dgt] : 0u;
+  __syncthreads();
+  const uint32_t t = sTile;
+  if (t >= div_up(n, TILE)) return;
+  const uint32_t tileBase = t * TILE;
+  const uint32_t tileN = min(TILE, n - tileBase);
+  const uint32_t li0 = w * (ITEMS * kWave) + lane;
+  K key[ITEMS];
+  uint32_t val[ITEMS], rank[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kWaveItems; k++) {
-      const uint32_t li = w * kPerWave + k * kWave + lane;
-      const bool valid = li < tileN;
-      key[k] = valid ? kin[tileBase + li] : (K)0;
-      val[k] = valid ? vin[tileBase + li] : 0u;
-      const uint32_t d = (uint32_t)(key[k] >> shift) & 255u;
-      dig[k] = d;
-      uint64_t peers = __ballot(valid);
+  for (int k = 0; k < ITEMS; k++) key[k] = li0 + k * kWave < tileN ? kin[tileBase + li0 + k * kWave] : (K)0;
 #pragma unroll
-      for (int b = 0; b < 8; b++) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t m = __ballot(bit);
-        peers &= bit ? m : ~m;
-      }
-      const uint32_t cnt = (uint32_t)__popcll(peers);
-      const uint32_t pre = (uint32_t)__popcll(peers & lt);
-      const uint32_t leader = peers ? (uint32_t)__builtin_ctzll(peers) : 64u;
-      uint32_t basev = valid ? sHist[w][d] : 0u;
-      rank[k] = basev + pre;
-      __builtin_amdgcn_wave_barrier();
-      if (valid && lane == leader) sHist[w][d] = basev + cnt;
-      __builtin_amdgcn_wave_barrier();
+  for (int k = 0; k < ITEMS; k++) {
+    const uint32_t i = tileBase + li0 + k * kWave;
+    val[k] = li0 + k * kWave < tileN ? (vin ? vin[i] : i) : 0u;
+  }
+  uint32_t tot;
+  const uint32_t digitBase = block_excl_scan<BLOCK, true>(dcount, ss[0], &tot);
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++) {
+    const bool valid = li0 + k * kWave < tileN;
+    const uint32_t d = (uint32_t)(key[k] >> shift) & 255u;
+    // lanes with the same digit
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; b++) {
+      const bool bit = (d >> b) & 1u;
+      const uint64_t m = __ballot(bit);
+      peers &= bit ? m : ~m;
     }
-    __syncthreads();
-    // per digit: exclusive offsets across waves, tile total
-    const uint32_t dgt = threadIdx.x;  // kBlock == 256 digits
-    uint32_t tot = 0;
+    const uint32_t pre = mbcnt(peers);
+    const uint32_t base = valid ? sHist[w][d] : 0u;
+    rank[k] = base + pre;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && pre == 0) sHist[w][d] = base + (uint32_t)__popcll(peers);
+    __builtin_amdgcn_wave_barrier();
+  }
+  sync_block_lds();
+  // per digit: exclusive offsets across waves, tile total
+  uint32_t dtot = 0;
+  uint64_t *const my = status + (size_t)t * kDigits + dgt;
+  if (dgt < kDigits) {
 #pragma unroll
-    for (int ww = 0; ww < kNW; ww++) {
-      uint32_t c = sHist[ww][dgt];
-      sHist[ww][dgt] = tot;
-      tot += c;
+    for (int ww = 0; ww < NW; ww++) {
+      const uint32_t c = sHist[ww][dgt];
+      sHist[ww][dgt] = dtot;
+      dtot += c;
     }
-    uint32_t tileTot;
-    const uint32_t tileEx = block_excl_scan<256>(tot, ss, &tileTot);
-    sTileExcl[dgt] = tileEx;
-    // decoupled look-back for this digit across earlier tiles
+    __hip_atomic_store(my, st_word(tag, t == 0 ? 2 : 1, dtot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const uint32_t tileEx = block_excl_scan<BLOCK, true>(dtot, ss[1], &tot);
+  // slot of each key in the tile's digit order
+  if (dgt < kDigits)
+#pragma unroll
+    for (int ww = 0; ww < NW; ww++) sHist[ww][dgt] += tileEx;
+  sync_block_lds();
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++) {
+    const uint32_t d = (uint32_t)(key[k] >> shift) & 255u;
+    rank[k] += sHist[w][d];
+    if (li0 + k * kWave < tileN) sK[rank[k]] = key[k];
+  }
+  // decoupled look-back for this digit across earlier tiles
+  if (dgt < kDigits) {
     uint32_t prefix = 0;
-    uint64_t *my = status + (size_t)t * 256 + dgt;
-    if (t == 0) {
-      __hip_atomic_store(my, st_word(tag, 2, tot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      __hip_atomic_store(my, st_word(tag, 1, tot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t) {
       uint32_t j = t - 1;
       uint32_t spins = 0;
       while (true) {
-        const uint64_t wv = __hip_atomic_load(status + (size_t)j * 256 + dgt, __ATOMIC_RELAXED,
+        const uint64_t wv = __hip_atomic_load(status + (size_t)j * kDigits + dgt, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT);
         const uint32_t wt = (uint32_t)(wv >> 34), wf = (uint32_t)(wv >> 32) & 3u;
         if (wt != tag || wf == 0) {
@@ -161,74 +177,62 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin,
         if (wf == 2) break;
         j--;
       }
-      __hip_atomic_store(my, st_word(tag, 2, prefix + tot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(my, st_word(tag, 2, prefix + dtot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    sGlob[dgt] = digitBase[dgt] + prefix;
-    __syncthreads();
-    // stage the tile in digit order
+    sGlob[dgt] = digitBase + prefix - tileEx;
+  }
+  sync_block_lds();
+  // keys, then values, in digit order: runs of consecutive addresses
+  uint32_t dst[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kWaveItems; k++) {
-      const uint32_t li = w * kPerWave + k * kWave + lane;
-      if (li < tileN) {
-        const uint32_t d = dig[k];
-        const uint32_t p = sTileExcl[d] + sHist[w][d] + rank[k];
-        sK[p] = key[k];
-        sV[p] = val[k];
-      }
-    }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < tileN; i += kBlock) {
+  for (int k = 0; k < ITEMS; k++) {
+    const uint32_t i = k * BLOCK + threadIdx.x;
+    if (i < tileN) {
       const K kk = sK[i];
-      const uint32_t d = (uint32_t)(kk >> shift) & 255u;
-      const uint32_t dst = sGlob[d] + (i - sTileExcl[d]);
-      kout[dst] = kk;
-      vout[dst] = sV[i];
+      dst[k] = sGlob[(uint32_t)(kk >> shift) & 255u] + i;
+      kout[dst[k]] = kk;
     }
-    __syncthreads();
+  }
+  sync_block_lds();
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++)
+    if (li0 + k * kWave < tileN) sV[rank[k]] = val[k];
+  sync_block_lds();
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++) {
+    const uint32_t i = k * BLOCK + threadIdx.x;
+    if (i < tileN) vout[dst[k]] = sV[i];
   }
 }
 
-// Scratch layout (bytes): status | tileHist | digitBase | digitCount |
-// tickets.
+// Scratch layout (bytes): status | digitCount | tickets, cleared by one fill.
 size_t sort_ws_bytes(uint32_t nMax, int keyBits) {
   const int passes = (keyBits + 7) / 8;
-  const size_t maxTiles = std::max<uint32_t>(1u, div_up(nMax, kTile));
-  const size_t histBlocks = div_up((uint32_t)maxTiles, kHistSpan);
-  return maxTiles * 256 * 8 + histBlocks * passes * 256 * 4 + 2 * passes * 256 * 4 + 64 + 256;
+  const size_t maxTiles = std::max<uint32_t>(1u, div_up(nMax, kBlock * kSmallItems));
+  return maxTiles * kDigits * 8 + (size_t)passes * kDigits * 4 + 64 + 256;
 }
 
 template <typename K>
 int sort_pairs_ws(K *kA, uint32_t *vA, K *kB, uint32_t *vB, const uint32_t *nDev, uint32_t nMax,
-                  int keyBits, hipStream_t s, void *ws, K **kRes, uint32_t **vRes, uint32_t *err = nullptr) {
+                  int keyBits, hipStream_t s, void *ws, K **kRes, uint32_t **vRes, uint32_t *err = nullptr,
+                  bool iota = false) {
   const int passes = (keyBits + 7) / 8;
-  const uint32_t maxTiles = std::max<uint32_t>(1u, div_up(nMax, kTile));
-  const uint32_t histBlocks = div_up(maxTiles, kHistSpan);
-  char *p = (char *)ws;
-  uint64_t *status = (uint64_t *)p;
-  p += (size_t)maxTiles * 256 * 8;
-  uint32_t *tileHist = (uint32_t *)p;
-  p += (size_t)histBlocks * passes * 256 * 4;
-  uint32_t *digitBase = (uint32_t *)p;
-  p += (size_t)passes * 256 * 4;
-  uint32_t *digitCount = (uint32_t *)p;
-  p += (size_t)passes * 256 * 4;
-  uint32_t *tickets = (uint32_t *)p;
-  CUBQL_CHECK(fill_u32((uint32_t *)status, 0u, (size_t)maxTiles * 512, s));
-  CUBQL_CHECK(fill_u32(digitCount, 0u, (size_t)passes * 256 + 16, s));  // digit counts and the tickets after them
-  k_hist<K><<<histBlocks, kBlock, 0, s>>>(kA, nDev, passes, tileHist);
-  k_hist_reduce<<<dim3(passes, kHistChunks), 256, 0, s>>>(tileHist, histBlocks, passes, digitCount);
-  k_digit_scan<<<passes, 256, 0, s>>>(digitCount, digitBase);
-  int dev = 0, numCU = 256;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&numCU, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    numCU = 256;
-  const uint32_t grid = std::min<uint32_t>(maxTiles, (uint32_t)numCU * 4);
+  const bool small = nMax < kSmallSort;
+  const uint32_t maxTiles = std::max<uint32_t>(1u, div_up(nMax, kBlock * (small ? kSmallItems : kLargeItems<K>)));
+  uint64_t *status = (uint64_t *)ws;
+  uint32_t *digitCount = (uint32_t *)(status + (size_t)maxTiles * kDigits);
+  uint32_t *tickets = digitCount + (size_t)passes * kDigits;
+  CUBQL_CHECK(fill_u32((uint32_t *)status, 0u, (size_t)maxTiles * kDigits * 2 + (size_t)passes * kDigits + 16, s));
+  // (two workgroups a CU: the global atomics of more would queue up)
+  const uint32_t histBlocks = std::max(1u, std::min(div_up(nMax, 4096), 512u));
+  k_hist<K><<<histBlocks, kHistBlock, (size_t)kHistWaves * passes * kDigits * 4, s>>>(kA, nDev, passes, digitCount);
   K *ki = kA, *ko = kB;
   uint32_t *vi = vA, *vo = vB;
   for (int p = 0; p < passes; p++) {
     int ps = prof_begin(s);
-    k_onesweep<K><<<grid, kBlock, 0, s>>>(ki, vi, ko, vo, nDev, 8 * p, (uint32_t)(p + 1),
-                                          digitBase + p * 256, status, tickets + p, err);
+    const auto pass = small ? k_onesweep<K, kSmallItems> : k_onesweep<K, kLargeItems<K>>;
+    pass<<<maxTiles, kBlock, 0, s>>>(ki, iota && p == 0 ? nullptr : vi, ko, vo, nDev, 8 * p, (uint32_t)(p + 1),
+                                     digitCount + p * kDigits, status, tickets + p, err);
     prof_end(ps, s, "radix_onesweep");
     prof_set(ps, (double)nMax * 2.0 * (sizeof(K) + 4), nMax);
     std::swap(ki, ko);
