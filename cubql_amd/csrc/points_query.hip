@@ -578,12 +578,17 @@ int root_box(const cubql_dev::WideBVH<W> &bvh, hipStream_t s, Scratch &scr, cons
   return CUBQL_OK;
 }
 
+// The tree as a binary one, if it is.
+inline const cubql_bvh3f *binary_tree(const cubql_bvh3f &bvh) { return &bvh; }
+template <int W>
+const cubql_bvh3f *binary_tree(const cubql_dev::WideBVH<W> &) { return nullptr; }
+
 // Workspace of one closest-point call over nq queries (256-byte aligned
 // slots): overflow counters | root box | overflow list | query order.
 constexpr size_t kWsOvf = 0, kWsRoot = 128, kWsList = 256;
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 inline size_t fcp_ws_bytes(uint32_t nq) {
-  return kWsList + align256((size_t)nq * 4) + (nq >= kQueryOrderMin ? query_order_ws_bytes(nq) : 0);
+  return kWsList + align256((size_t)nq * 4) + query_order_ws_bytes(nq);
 }
 
 inline const cubql_box3f *root_box_ws(const cubql_bvh3f &bvh, hipStream_t, char *) { return &bvh.nodes[0].bounds; }
@@ -614,9 +619,8 @@ int fcp_run_ws(const BVH &bvh, const float *d_points, const float *d_queries, ui
   const cubql_box3f *rootBox = root_box_ws(bvh, s, ws);
   CUBQL_LAUNCH_CHECK();
   const uint32_t *order = nullptr;
-  if (numQueries >= kQueryOrderMin)
-    CUBQL_CHECK(query_order_box_ws(rootBox, d_queries, numQueries, s,
-                                   ws + kWsList + align256((size_t)numQueries * 4), &order));
+  CUBQL_CHECK(query_order_ws(rootBox, binary_tree(bvh), {d_queries, numQueries, false}, s,
+                             ws + kWsList + align256((size_t)numQueries * 4), &order));
   int ps = prof_begin(s);
   if constexpr (std::is_same<BVH, cubql_bvh3f>::value) {
     const uint32_t qpw = queries_per_wave(numQueries);
@@ -681,7 +685,7 @@ int knn_run(const BVH &bvh, const float *d_points, const float *d_queries, uint3
   if (numQueries >= kQueryOrderMin) {
     char *w = nullptr;
     CUBQL_CHECK(scr.alloc(&w, query_order_ws_bytes(numQueries)));
-    CUBQL_CHECK(query_order_box_ws(rootBox, d_queries, numQueries, s, w, &order));
+    CUBQL_CHECK(query_order_ws(rootBox, binary_tree(bvh), {d_queries, numQueries, false}, s, w, &order));
   }
   // the slot-ordered copy pays when the queries test at least about as many
   // prims as the copy moves

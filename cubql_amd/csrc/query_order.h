@@ -1,10 +1,14 @@
-// query_order.h -- Morton ordering of a batch of queries.
+// query_order.h -- spatial ordering of a batch of queries.
 //
-// Queries are processed one per lane; lanes of a wave that start from nearby
-// points walk nearly the same nodes, so sorting a large batch by the Morton
-// code of its queries (cells of the tree's root box) makes node loads
-// coherent and cuts divergence.  Results are written back to each query's
-// own slot, so the output is independent of the order.
+// Lanes of a wave whose queries are close to each other walk nearly the same
+// nodes, so a large batch is sorted by place before it is traversed, which
+// makes node loads coherent and cuts divergence.  Results are written back to
+// each query's own slot, so the output is independent of the order.
+//
+// The place is the Morton code of the query in cells of the tree's root box,
+// or, where a few far-off prims leave most queries in a few cells, the primID
+// slot of the leaf the query descends to (binary trees).  A sample of the
+// queries decides on the device.
 #pragma once
 #include "common.h"
 
@@ -13,19 +17,21 @@ namespace cubql {
 // Batches below this size run in input order.
 constexpr uint32_t kQueryOrderMin = 32768;
 
-// On success *order is a device permutation (sorted position -> query
-// index) valid until `scr` is destroyed, or nullptr for small batches.
-int query_order(const cubql_bvh3f &bvh, const float *queries, uint32_t nq, hipStream_t s, Scratch &scr,
-                const uint32_t **order);
+// The places of a batch: points (stride 3 floats) or the centres of boxes
+// (stride 6: lower xyz, upper xyz).
+struct QueryPlaces {
+  const float *p;
+  uint32_t n;
+  bool boxes;
+};
 
-// The same on a caller-provided workspace of query_order_ws_bytes(nq)
-// bytes (256-byte aligned); *order points into it.  Allocates nothing.
+// Orders `q` on a caller's workspace of query_order_ws_bytes(q.n) bytes
+// (256-byte aligned): *order points into it, a device permutation (sorted
+// position -> query index), or is nullptr for small batches.  rootBox: the
+// box the cells are taken over (device).  bvh: the tree for the slot keys, or
+// nullptr.  Allocates nothing.
 size_t query_order_ws_bytes(uint32_t nq);
-int query_order_ws(const cubql_bvh3f &bvh, const float *queries, uint32_t nq, hipStream_t s, void *ws,
+int query_order_ws(const cubql_box3f *rootBox, const cubql_bvh3f *bvh, const QueryPlaces &q, hipStream_t s, void *ws,
                    const uint32_t **order);
-// The same with the cells taken over a device box (rootBox == nullptr:
-// no ordering).
-int query_order_box_ws(const cubql_box3f *rootBox, const float *queries, uint32_t nq, hipStream_t s, void *ws,
-                       const uint32_t **order);
 
 }  // namespace cubql

@@ -262,6 +262,10 @@ int radix_sort_pairs_ws_u32(uint32_t *kA, uint32_t *vA, uint32_t *kB, uint32_t *
                             uint32_t **vRes) {
   return rs::sort_pairs_ws<uint32_t>(kA, vA, kB, vB, nDev, nMax, keyBits, s, ws, kRes, vRes);
 }
+int radix_sort_iota_ws_u32(uint32_t *kA, uint32_t *vA, uint32_t *kB, uint32_t *vB, const uint32_t *nDev,
+                           uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint32_t **kRes, uint32_t **vRes) {
+  return rs::sort_pairs_ws<uint32_t>(kA, vA, kB, vB, nDev, nMax, keyBits, s, ws, kRes, vRes, nullptr, true);
+}
 int radix_sort_pairs_ws_u64(uint64_t *kA, uint32_t *vA, uint64_t *kB, uint32_t *vB, const uint32_t *nDev,
                             uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint64_t **kRes,
                             uint32_t **vRes) {

@@ -392,7 +392,11 @@ extern "C" int cubql_fcp_triangles_f3(const cubql_bvh3f *bvh, const int32_t *d_t
   CUBQL_CHECK(scr.alloc(&ovfList, numQueries));
   CUBQL_CHECK(fill_u32((uint32_t *)ovf, 0u, 2, s));
   const uint32_t *order = nullptr;
-  CUBQL_CHECK(query_order(*bvh, d_queries, numQueries, s, scr, &order));
+  if (numQueries >= kQueryOrderMin) {
+    char *w = nullptr;
+    CUBQL_CHECK(scr.alloc(&w, query_order_ws_bytes(numQueries)));
+    CUBQL_CHECK(query_order_ws(&bvh->nodes[0].bounds, bvh, {d_queries, numQueries, false}, s, w, &order));
+  }
   // the slot-ordered copy of the mesh pays when the queries test at least
   // about as many triangles as the copy moves
   float4 *stris = nullptr;
