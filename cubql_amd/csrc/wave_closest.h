@@ -24,22 +24,9 @@
 
 #include "common.h"
 #include "cubql_amd/traversal.hip.h"
+#include "uniform_load.h"
 
 namespace cubql {
-
-typedef float vec4f __attribute__((ext_vector_type(4)));
-
-// The child pair at nodes[i0], i0 the same in every lane: scalar loads.
-__device__ __forceinline__ void load_pair_uniform(const cubql_node3f *nodes, uint32_t i0, cubql_dev::QNode &n0,
-                                                  cubql_dev::QNode &n1) {
-  typedef const __attribute__((address_space(4))) vec4f *cptr;
-  cptr p = (cptr)(uintptr_t)(nodes + i0);
-  const vec4f a = p[0], b = p[1], c = p[2], d = p[3];
-  n0.a = make_float4(a.x, a.y, a.z, a.w);
-  n0.b = make_float4(b.x, b.y, b.z, b.w);
-  n1.a = make_float4(c.x, c.y, c.z, c.w);
-  n1.b = make_float4(d.x, d.y, d.z, d.w);
-}
 
 // Queue slots of a wave: 512 leave fewer waves in flight (10M queries of 10M
 // points: 2.21 ms a call against 2.04 ms), 256 send more queries of clustered
