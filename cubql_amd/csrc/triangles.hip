@@ -212,81 +212,120 @@ __global__ void k_tri_boxes(const int32_t *tris, const float *verts, uint32_t n,
   }
 }
 
+// Each query's terms for the three vertices go through LDS so that three
+// neighbouring lanes add x, y and z of one vertex: the memory side takes one
+// request per vertex instead of three.  Bound by those requests (4M queries,
+// 1.3M triangles: 348 us with one, 1841 us with three).
 __global__ __launch_bounds__(kBlock) void k_tri_backward(const int32_t *tris, const float *verts,
                                                          const float *queries, uint32_t nq,
                                                          const int32_t *ids, const float *gradDist,
                                                          float *gradQ, float *gradV) {
+  __shared__ uint32_t sVert[kBlock * 3];
+  __shared__ float sTerm[kBlock * 9];
   const uint32_t qi = blockIdx.x * kBlock + threadIdx.x;
-  if (qi >= nq) return;
-  const int32_t t = ids[qi];
-  const F3 q = ld3(queries, qi);
+  const bool act = qi < nq;
+  const int32_t t = act ? ids[qi] : -1;
   F3 gq = {0.f, 0.f, 0.f};
+  float w[3] = {0.f, 0.f, 0.f};
+  uint32_t v[3] = {0u, 0u, 0u};
   if (t >= 0) {
+    const F3 q = ld3(queries, qi);
     F3 a, b, c, P;
-    tri_verts(tris, verts, (uint32_t)t, a, b, c);
-    float w[3];
+    for (int j = 0; j < 3; j++) v[j] = tris ? (uint32_t)tris[3 * (size_t)t + j] : 3u * (uint32_t)t + j;
+    a = ld3(verts, v[0]);
+    b = ld3(verts, v[1]);
+    c = ld3(verts, v[2]);
     const float s = tri_closest<true>(a, b, c, q, P, w);
     const float d = sqrtf(s);
     if (d > 0.f) {
-      const float g = gradDist[qi] / d;
-      const F3 dir = sub(q, P);
-      gq = mul(g, dir);
-      if (gradV) {
-        for (int j = 0; j < 3; j++) {
-          const size_t v = tris ? (size_t)tris[3 * (size_t)t + j] : 3 * (size_t)t + j;
-          atomicAdd(&gradV[3 * v + 0], -w[j] * gq.x);
-          atomicAdd(&gradV[3 * v + 1], -w[j] * gq.y);
-          atomicAdd(&gradV[3 * v + 2], -w[j] * gq.z);
-        }
-      }
+      gq = mul(gradDist[qi] / d, sub(q, P));
+    } else {
+      w[0] = w[1] = w[2] = 0.f;
     }
   }
-  if (gradQ) {
+  if (gradQ && act) {
     gradQ[3 * (size_t)qi] = gq.x;
     gradQ[3 * (size_t)qi + 1] = gq.y;
     gradQ[3 * (size_t)qi + 2] = gq.z;
+  }
+  if (!gradV) return;
+  // a wave's own part of the arrays: no barrier is needed
+  const uint32_t lane = lane_id(), w0 = threadIdx.x - lane;
+  uint32_t *const wv = sVert + 3 * w0;
+  float *const wt = sTerm + 9 * w0;
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    wv[3 * lane + j] = v[j];
+    wt[9 * lane + 3 * j + 0] = -w[j] * gq.x;
+    wt[9 * lane + 3 * j + 1] = -w[j] * gq.y;
+    wt[9 * lane + 3 * j + 2] = -w[j] * gq.z;
+  }
+  sync_wave_lds();
+#pragma unroll
+  for (uint32_t i = 0; i < 9; i++) {
+    const uint32_t c = i * kWave + lane;
+    const float term = wt[c];
+    if (term != 0.f) atomicAdd(&gradV[3 * (size_t)wv[c / 3] + c % 3], term);
   }
 }
 
-// points: d = |q-p| for each (query, neighbour) entry e = qi*k + j.  The
-// query gradient is summed per lane.  The point gradient is not scattered
-// here: when gv is given, each entry's point term -g (0 for skipped
-// entries) goes to gv[e] and its sort key to key[e] (the point id, or
-// numPoints for entries that contribute nothing), val[e] = e.
+// The term of entry (query, neighbour) of a point distance: gradDist / d *
+// (q - p), or false where it contributes nothing.
+__device__ __forceinline__ bool point_term(F3 q, F3 p, const float *gradDist, size_t e, F3 &g) {
+  const F3 diff = sub(q, p);
+  const float d = sqrtf(dot(diff, diff));
+  g = {0.f, 0.f, 0.f};
+  if (!(d > 0.f)) return false;
+  g = mul(gradDist[e] / d, diff);
+  return true;
+}
+
+// points: d = |q-p| for each (query, neighbour) entry e = qi*k + j, a thread
+// per entry so that ids, weights and keys are read and written in order
+// (2M x 16 entries: 655 us, bound by the gather of the points; 2150 us with a
+// thread per query, which strides).
+// The query gradient is the sum of its terms in entry order, taken from LDS.
+// The point gradient is not scattered here: when key is given, gv[e] is the
+// entry's point term and key[e] its sort key (the point id, or numPoints for
+// entries that contribute nothing).
+constexpr uint32_t kBackEntries = 1024;  // terms of a workgroup, in LDS
 __global__ __launch_bounds__(kBlock) void k_point_backward(const float *points, const float *queries,
-                                                           uint32_t nq, int k, const int32_t *ids,
-                                                           const float *gradDist, float *gradQ, float *gv,
-                                                           uint32_t *key, uint32_t *val, uint32_t numPoints) {
-  const uint32_t qi = blockIdx.x * kBlock + threadIdx.x;
-  if (qi >= nq) return;
-  const F3 q = ld3(queries, qi);
-  F3 gq = {0.f, 0.f, 0.f};
-  for (int j = 0; j < k; j++) {
-    const size_t e = (size_t)qi * k + j;
-    const int32_t p = ids[e];
-    F3 g = {0.f, 0.f, 0.f};
-    bool live = false;
-    if (p >= 0) {
-      const F3 diff = sub(q, ld3(points, (size_t)p));
-      const float d = sqrtf(dot(diff, diff));
-      if (d > 0.f) {
-        g = mul(gradDist[e] / d, diff);
-        gq = add(gq, g);
-        live = true;
+                                                           uint32_t nq, uint32_t k, uint32_t perBlock,
+                                                           const int32_t *ids, const float *gradDist, float *gradQ,
+                                                           float *gv, uint32_t *key, uint32_t numPoints) {
+  __shared__ float sT[3 * kBackEntries];
+  const uint32_t q0 = blockIdx.x * perBlock;
+  const uint32_t nHere = min(perBlock, nq - q0);
+  const uint32_t kc = min(k, kBackEntries);
+  float carry = 0.f;  // (k > kBackEntries: a query's sum so far, one query here)
+  for (uint32_t j0 = 0; j0 < k; j0 += kc) {
+    const uint32_t kn = min(kc, k - j0);  // (several queries: all k)
+    for (uint32_t i = threadIdx.x; i < nHere * kn; i += kBlock) {
+      const uint32_t qi = q0 + i / kn;
+      const size_t e = (size_t)qi * k + j0 + i % kn;
+      const int32_t p = ids[e];
+      F3 g = {0.f, 0.f, 0.f};
+      const bool live = p >= 0 && point_term(ld3(queries, qi), ld3(points, (size_t)p), gradDist, e, g);
+      sT[3 * i] = g.x;
+      sT[3 * i + 1] = g.y;
+      sT[3 * i + 2] = g.z;
+      if (key) {
+        gv[3 * e] = -g.x;
+        gv[3 * e + 1] = -g.y;
+        gv[3 * e + 2] = -g.z;
+        key[e] = live && (uint32_t)p < numPoints ? (uint32_t)p : numPoints;
       }
     }
-    if (gv) {
-      gv[3 * e + 0] = -g.x;
-      gv[3 * e + 1] = -g.y;
-      gv[3 * e + 2] = -g.z;
-      key[e] = live && (uint32_t)p < numPoints ? (uint32_t)p : numPoints;
-      val[e] = (uint32_t)e;
+    if (!gradQ) continue;
+    sync_block_lds();
+    for (uint32_t c = threadIdx.x; c < 3 * nHere; c += kBlock) {
+      const float *t = sT + 3 * (size_t)(c / 3) * kn + c % 3;
+      float sum = carry;
+      for (uint32_t j = 0; j < kn; j++) sum += t[3 * j];
+      if (j0 + kn < k) carry = sum;
+      else gradQ[3 * (size_t)q0 + c] = sum;
     }
-  }
-  if (gradQ) {
-    gradQ[3 * (size_t)qi] = gq.x;
-    gradQ[3 * (size_t)qi + 1] = gq.y;
-    gradQ[3 * (size_t)qi + 2] = gq.z;
+    sync_block_lds();
   }
 }
 
@@ -296,7 +335,9 @@ __global__ __launch_bounds__(kBlock) void k_point_backward(const float *points, 
 // with a plain read-modify-write, and only runs that touch the wave's first
 // or last lane (which may continue in the next or previous wave) use
 // atomics.  No float atomic per entry, and the sum order inside a run is
-// fixed.
+// fixed.  Bound by the gather of the terms, a line each (2M x 16 entries:
+// 1150 us; as much with 16-byte terms in one load, 1385 us computing the terms
+// again from the query and the weight).
 __global__ __launch_bounds__(kBlock) void k_point_scatter(const uint32_t *key, const uint32_t *val,
                                                           const float *gv, uint32_t n, uint32_t numPoints,
                                                           float *gradP) {
@@ -306,10 +347,10 @@ __global__ __launch_bounds__(kBlock) void k_point_scatter(const uint32_t *key, c
   const uint32_t p = act ? key[i] : numPoints;
   float sx = 0.f, sy = 0.f, sz = 0.f;
   if (act && p < numPoints) {
-    const uint32_t e = val[i];
-    sx = gv[3 * (size_t)e + 0];
-    sy = gv[3 * (size_t)e + 1];
-    sz = gv[3 * (size_t)e + 2];
+    const F3 g = ld3(gv, val[i]);
+    sx = g.x;
+    sy = g.y;
+    sz = g.z;
   }
   const uint32_t pPrev = (uint32_t)__shfl_up((int)p, 1, kWave);
   const bool head = lane == 0 || pPrev != p;
@@ -464,6 +505,10 @@ extern "C" int cubql_points_distance_backward_f3(const float *d_points, uint32_t
   ScratchArena scr(mem, s);
   float *gv = nullptr;
   uint32_t *kA = nullptr, *vA = nullptr, *kB = nullptr, *vB = nullptr, *cnt = nullptr;
+  char *sortWs = nullptr;
+  // key bits: enough for the sentinel numPoints
+  int bits = 1;
+  while (bits < 32 && (numPoints >> bits) != 0) bits++;
   if (scatter) {
     CUBQL_CHECK(scr.reserve(&gv, 3 * ne));
     CUBQL_CHECK(scr.reserve(&kA, ne));
@@ -471,21 +516,24 @@ extern "C" int cubql_points_distance_backward_f3(const float *d_points, uint32_t
     CUBQL_CHECK(scr.reserve(&kB, ne));
     CUBQL_CHECK(scr.reserve(&vB, ne));
     CUBQL_CHECK(scr.reserve(&cnt, 1));
+    CUBQL_CHECK(scr.reserve(&sortWs, radix_sort_ws_bytes((uint32_t)ne, bits)));
     CUBQL_CHECK(scr.commit());
     CUBQL_CHECK(fill_u32(cnt, (uint32_t)ne, 1, s));
   }
   int ps = prof_begin(s);
-  tri::k_point_backward<<<div_up(numQueries, tri::kBlock), tri::kBlock, 0, s>>>(
-      d_points, d_queries, numQueries, k, d_ids, d_gradDist, d_gradQueries, gv, kA, vA, numPoints);
-  CUBQL_LAUNCH_CHECK();
+  if (scatter || d_gradQueries) {
+    // a query's k terms stay in one workgroup's LDS
+    const uint32_t perBlock = std::max(1u, tri::kBackEntries / (uint32_t)k);
+    tri::k_point_backward<<<div_up(numQueries, perBlock), tri::kBlock, 0, s>>>(
+        d_points, d_queries, numQueries, (uint32_t)k, perBlock, d_ids, d_gradDist, d_gradQueries, gv, kA,
+        numPoints);
+    CUBQL_LAUNCH_CHECK();
+  }
   if (scatter) {
-    // key bits: enough for the sentinel numPoints
-    int bits = 1;
-    while (bits < 32 && (numPoints >> bits) != 0) bits++;
     uint32_t *kRes = nullptr, *vRes = nullptr;
-    CUBQL_CHECK(radix_sort_pairs_dev_u32(kA, vA, kB, vB, cnt, (uint32_t)ne, bits, s, mem, &kRes, &vRes));
-    tri::k_point_scatter<<<div_up((uint32_t)ne, tri::kBlock), tri::kBlock, 0, s>>>(kRes, vRes, gv, (uint32_t)ne,
-                                                                                  numPoints, d_gradPoints);
+    CUBQL_CHECK(radix_sort_iota_ws_u32(kA, vA, kB, vB, cnt, (uint32_t)ne, bits, s, sortWs, &kRes, &vRes));
+    tri::k_point_scatter<<<div_up((uint32_t)ne, tri::kBlock), tri::kBlock, 0, s>>>(
+        kRes, vRes, gv, (uint32_t)ne, numPoints, d_gradPoints);
     CUBQL_LAUNCH_CHECK();
   }
   prof_end(ps, s, "points_backward");
