@@ -38,14 +38,24 @@ __host__ __device__ inline uint32_t oc_count(uint64_t oc) { return (uint32_t)(oc
 
 // The dispatcher hands workgroup b of a launch to XCD b % 8, and each of
 // the 8 XCDs has its own L2.  For nb workgroups over work stored in a
-// locality order (Morton-sorted queries), xcd_chunk(b, nb) is the index of
-// the piece of work workgroup b takes such that each XCD gets one contiguous
-// run of pieces (a bijection on [0, nb)), so an XCD's L2 serves one region
-// of the tree instead of all of it.
+// locality order (spatially sorted queries), xcd_chunk(b, nb) is the index of
+// the piece of work workgroup b takes such that each XCD gets runs of
+// kXcdRun contiguous pieces (a bijection on [0, nb)), so an XCD's L2 serves a
+// few regions of the tree at a time.  One run of nb / 8 pieces an XCD would
+// serve one, but leaves the XCD with the costliest region running alone (10M
+// closest-point queries 1932 us so and 1915 in runs of 32, the same in runs of
+// 8 and 128; a training step on 2M clustered points 11.56 and 11.31 ms).
 constexpr uint32_t kXcds = 8;
+constexpr uint32_t kXcdRun = 32;
 __device__ __forceinline__ uint32_t xcd_chunk(uint32_t b, uint32_t nb) {
+  constexpr uint32_t G = kXcds * kXcdRun;
+  const uint32_t full = nb / G * G;
+  if (b < full) return b / G * G + (b % kXcds) * kXcdRun + b % G / kXcds;
+  // the rest: one run an XCD
+  b -= full;
+  nb -= full;
   const uint32_t q = nb / kXcds, r = nb % kXcds, x = b % kXcds, j = b / kXcds;
-  return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + j;
+  return full + (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + j;
 }
 
 // ---------------------------------------------------------------- errors
