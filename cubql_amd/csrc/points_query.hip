@@ -15,6 +15,7 @@
 #include "profile.h"
 #include "query_order.h"
 #include "wave_closest.h"
+#include "wave_knn.h"
 
 namespace cubql {
 namespace pq {
@@ -419,25 +420,110 @@ __device__ __forceinline__ bool knn_seeded_on(StackT &stack, const cubql_bvh3f &
   }
 }
 
-// kNN lists of up to kKnnSeededMax entries over a binary tree take the
-// seeded traversal on an LDS stack of kKnnLdsStack entries per lane (32 KB a
-// workgroup; deeper queries rerun in the deep kernel).  Longer lists keep
-// the unseeded traversal on a private stack: on the clustered Gaussian-
-// mixture workload (2M points, k = 16) the LDS versions were slower (16
-// entries: 264 Mq/s, 24 entries: 224 Mq/s, against 293 Mq/s), the queries
-// that overflow the LDS stack being the slowest ones, which the deep rerun
-// then no longer overlaps with the others.
+// Lists of up to kKnnWaveMax entries over a binary tree: a wave per qpw
+// queries (wave_knn.h).  A longer list does not fit the registers.  1M queries
+// of 10M points, 8 neighbours: 1.62 ms with one query per lane and a seeded
+// traversal on a 16-entry LDS stack, 0.79 ms here; 2M clustered queries, 16
+// neighbours: 5.17 ms on a 64-entry private stack, 2.80 ms here; bound by VALU
+// issue and, with 16, the latency three waves a SIMD leave open.
+constexpr int kKnnWaveMax = 16;
+// (the deep and statistics kernels' seeded traversal, one query per lane)
 constexpr int kKnnSeededMax = 8;
-constexpr int kKnnLdsStack = 16;
 
-// kSorted (binary trees): leaf prims from spts, the points in primID-slot order.
+template <bool kSorted>
+struct SlotPoint {
+  const uint32_t *primIDs;
+  const float *points;
+  const float4 *spts;
+  __device__ __forceinline__ float4 operator()(uint32_t slot) const {
+    if constexpr (kSorted) return spts[slot];
+    const uint32_t id = primIDs[slot];
+    const float3 v = load_pt(points, id);
+    return make_float4(v.x, v.y, v.z, __uint_as_float(id));
+  }
+};
+
+// aligned: the output rows are 16-byte aligned and k is a multiple of four
+template <int K, bool kSorted>
+__global__ __launch_bounds__(kBlock) void k_knn_wave(cubql_bvh3f bvh, const float *points, const float4 *spts,
+                                                     const float *queries, uint32_t nq, uint32_t qpw, int k,
+                                                     float sqrMax, bool aligned, int32_t *outIds, float *outD,
+                                                     int32_t *outFound, Overflow *ovf, uint32_t *ovfList,
+                                                     const uint32_t *order) {
+  __shared__ WaveKnn<K> share[kBlock / kWave];
+  const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
+  // spatially ordered queries: one contiguous run of them per XCD
+  const uint32_t b = order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint64_t i = (uint64_t)(b * (kBlock / kWave) + wave) * qpw + lane;
+  const bool live = lane < qpw && i < nq;
+  const uint32_t qi = live ? (order ? order[i] : (uint32_t)i) : 0u;
+  float3 q = make_float3(0.f, 0.f, 0.f);
+  if (live) q = load_pt(queries, qi);
+  const unsigned long long none = closest_none(sqrMax);
+  int32_t *oi = outIds + (size_t)qi * k;
+  float *od = outD + (size_t)qi * k;
+  // Queries that lost a task run again, eight at a time and then alone (the
+  // queue holds more of each), and last in the deep kernel.
+  uint64_t todo = __ballot(live);
+  for (uint32_t together = kWave; todo; together /= 8) {
+    uint64_t again = 0;
+    while (todo) {
+      const bool on = ((todo >> lane) & 1u) && mbcnt(todo) < together;
+      unsigned long long list[K];
+      bool failed;
+      wave_knn<K>(share[wave], bvh.nodes, on, q.x, q.y, q.z, k, none, SlotPoint<kSorted>{bvh.primIDs, points, spts},
+                  list, &failed);
+      todo &= ~__ballot(on);
+      failed = failed && on;
+      if (on && !failed) {
+        int found = 0;
+        int32_t id[K];
+        float d[K];
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+          const bool has = list[j] != ~0ull;
+          if (has && j < k) found++;
+          id[j] = has ? (int32_t)(uint32_t)list[j] : -1;
+          d[j] = has ? __uint_as_float((uint32_t)(list[j] >> 32)) : INFINITY;
+        }
+        if (aligned) {
+#pragma unroll
+          for (int j = 0; j < K; j += 4) {
+            if (j < k) {
+              *reinterpret_cast<int4 *>(oi + j) = make_int4(id[j], id[j + 1], id[j + 2], id[j + 3]);
+              *reinterpret_cast<float4 *>(od + j) = make_float4(d[j], d[j + 1], d[j + 2], d[j + 3]);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < K; j++) {
+            if (j < k) {
+              oi[j] = id[j];
+              od[j] = d[j];
+            }
+          }
+        }
+        if (outFound) outFound[qi] = found;
+      } else if (failed && together == 1) {
+        ovfList[atomicAdd(&ovf->count, 1u)] = qi;
+      }
+      if (together > 1) again |= __ballot(failed);
+      sync_wave_lds();
+    }
+    todo = again;
+  }
+}
+
+// One query per lane on a 64-entry private stack: wide trees and lists longer
+// than kKnnWaveMax.  kSorted (binary trees): leaf prims from spts, the points
+// in primID-slot order.
 template <int K, typename BVH, bool kSorted = false>
 __global__ __launch_bounds__(kBlock) void k_knn(BVH bvh, const float *points, const float4 *spts,
                                                 const float *queries, uint32_t nq, int k,
                                                 float sqrMax, int32_t *outIds, float *outD,
                                                 int32_t *outFound, Overflow *ovf,
                                                 uint32_t *ovfList, const uint32_t *order) {
-  // Morton-ordered queries: one contiguous run of them per XCD
+  // spatially ordered queries: one contiguous run of them per XCD
   const uint32_t i = (order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x) * kBlock + threadIdx.x;
   if (i >= nq) return;
   const uint32_t qi = order ? order[i] : i;
@@ -445,15 +531,7 @@ __global__ __launch_bounds__(kBlock) void k_knn(BVH bvh, const float *points, co
   int32_t ids[K];
   float ds[K];
   int found;
-  bool done;
-  if constexpr (std::is_same<BVH, cubql_bvh3f>::value && K <= kKnnSeededMax) {
-    __shared__ uint2 sStack[kKnnLdsStack * kBlock];
-    cubql_dev::LdsStack<kKnnLdsStack, kBlock> stack(sStack + threadIdx.x);
-    done = knn_seeded_on<K, kSorted>(stack, bvh, points, spts, q, k, sqrMax, ids, ds, found);
-  } else {
-    done = knn_one<K, kFastStack, kSorted>(bvh, points, spts, q, k, sqrMax, ids, ds, found);
-  }
-  if (!done) {
+  if (!knn_one<K, kFastStack, kSorted>(bvh, points, spts, q, k, sqrMax, ids, ds, found)) {
     uint32_t slot = atomicAdd(&ovf->count, 1u);
     ovfList[slot] = qi;
     return;
@@ -518,17 +596,23 @@ int launch_knn(const BVH &bvh, const float *points, const float *queries, uint32
                int k, float sqrMax, int32_t *ids, float *d, int32_t *found, Overflow *ovf,
                uint32_t *ovfList, const uint32_t *order, float4 *spts, hipStream_t s) {
   int ps = prof_begin(s);
-  bool sorted = false;
-  if constexpr (std::is_same<BVH, cubql_bvh3f>::value) {
-    if (spts) {
+  constexpr bool kBinary = std::is_same<BVH, cubql_bvh3f>::value;
+  if constexpr (kBinary) {
+    if (spts)
       k_slot_points<<<std::max(1u, std::min(div_up(bvh.numPrims, 256u), 2048u)), 256, 0, s>>>(
           bvh.primIDs, bvh.numPrims, points, spts);
-      k_knn<K, BVH, true><<<div_up(nq, kBlock), kBlock, 0, s>>>(bvh, points, spts, queries, nq, k, sqrMax, ids, d,
-                                                                found, ovf, ovfList, order);
-      sorted = true;
-    }
   }
-  if (!sorted) {
+  if constexpr (kBinary && K <= kKnnWaveMax) {
+    const uint32_t qpw = queries_per_wave(nq);
+    const bool aligned = k % 4 == 0 && ((uintptr_t)ids | (uintptr_t)d) % 16 == 0;
+    const auto kern = spts ? k_knn_wave<K, true> : k_knn_wave<K, false>;
+    kern<<<div_up(div_up(nq, qpw), kBlock / kWave), kBlock, 0, s>>>(bvh, points, spts, queries, nq, qpw, k, sqrMax,
+                                                                    aligned, ids, d, found, ovf, ovfList, order);
+  } else if constexpr (kBinary) {
+    const auto kern = spts ? k_knn<K, BVH, true> : k_knn<K, BVH, false>;
+    kern<<<div_up(nq, kBlock), kBlock, 0, s>>>(bvh, points, spts, queries, nq, k, sqrMax, ids, d, found, ovf, ovfList,
+                                               order);
+  } else {
     k_knn<K, BVH><<<div_up(nq, kBlock), kBlock, 0, s>>>(bvh, points, nullptr, queries, nq, k, sqrMax, ids, d, found,
                                                         ovf, ovfList, order);
   }
