@@ -60,11 +60,20 @@ constexpr uint32_t kAccB = 24;
 // Pass B gathers the grandchild bounds of a split child only when the child
 // has more than kLazyBounds prims: a smaller child's grandchildren are
 // nearly always small (their own phase computes their boxes), and the emit
-// reduces the bounds of an open one from its prims.
-constexpr uint32_t kLazyBounds = 4 * kMedium;
+// reduces the bounds of an open one from its prims.  Gathering for fewer
+// children saves 1% where the grandchildren fall below kMedium anyway (3M
+// uniform points: 648 us with 4096, 656 with 1280), but the emit then reduces
+// thousands of ranges where they do not: 1.5M points 982 us with 4096, 511 with
+// 1280, 6M 1997 and 1062, 1M clustered 1318 and 838.
+constexpr uint32_t kLazyBounds = kMedium + kMedium / 4;
 __host__ __device__ __forceinline__ bool gather_bounds(uint32_t split, uint32_t childSize) {
   return split != 0 && childSize > kLazyBounds;
 }
+
+// Ranges of up to kFixWave prims whose bounds pass B did not gather are
+// reduced by one wave of the emit each (one after the other by the workgroup:
+// 1M clustered points 975 us a build, by waves 838).
+constexpr uint32_t kFixWave = 8192;
 
 struct Counters {
   uint32_t numValid;
@@ -1060,7 +1069,7 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit2(Ctx c, int pass) {
       c.nodes[g.node].oc = pack_oc(child, 0);
     }
     c.topNodes[topBase + s] = g.node;
-    int nf = 0;
+#pragma unroll
     for (int side = 0; side < 2; side++) {
       const uint32_t cb = side ? mid : begin, ce = side ? end : mid;
       const uint32_t rv = child_rev(mode, side);
@@ -1082,6 +1091,7 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit2(Ctx c, int pass) {
       c.topNodes[topBase + n + xi] = cid;
       xi++;
       if (rv && (nCL[side] == 0 || nCL[side] == ce - cb)) sRev[atomicAdd(&sNumRev, 1u)] = make_uint2(cb, ce - cb);
+#pragma unroll
       for (uint32_t gs = 0; gs < 2; gs++) {
         const GrandKid gk = grand_kid(cb, ce, nCL[side], rv, gs, T);
         if (!gk.large) {
@@ -1106,10 +1116,9 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit2(Ctx c, int pass) {
         }
         const uint32_t tiles = div_up(gk.e - gk.b, kTile);
         c.tileStart[np][li] = ti;
-        fillStart[nf] = ti;
-        fillCount[nf] = tiles;
-        fillSeg[nf] = li;
-        nf++;
+        fillStart[2 * side + gs] = ti;
+        fillCount[2 * side + gs] = tiles;
+        fillSeg[2 * side + gs] = li;
         ti += tiles;
         li++;
       }
@@ -1119,6 +1128,7 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit2(Ctx c, int pass) {
   // the top passes' few big segments, which the whole wave writes
   constexpr uint32_t kOwnFill = 256;
   const uint32_t lane = lane_id();
+#pragma unroll
   for (int f = 0; f < 4; f++) {
     if (fillCount[f] <= kOwnFill)
       for (uint32_t t = 0; t < fillCount[f]; t++) c.tileSeg[np][fillStart[f] + t] = fillSeg[f];
@@ -1151,8 +1161,43 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit2(Ctx c, int pass) {
   // ranges before these read them)
   __syncthreads();
   const uint32_t nFix = sNumFix;
+  auto plane = [&](uint32_t li, const float (&lo)[3], const float (&hi)[3]) __attribute__((always_inline)) {
+    int dim;
+    float pos;
+    choose_split(lo, hi, dim, pos);
+    c.segDim[np][li] = dim;
+    c.segPos[np][li] = pos;
+  };
+  // a wave per range, four items a lane in flight
+  for (uint32_t f = w; f < nFix; f += NW) {
+    const uint32_t li = sFix[f].x, pb = sFix[f].y, sz = sFix[f].z;
+    if (sz > kFixWave) continue;
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (uint32_t i0 = lane; i0 < sz; i0 += 4 * kWave) {
+      float4 it[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) it[u] = items[pb + min(i0 + u * kWave, sz - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        lo[0] = fminf(lo[0], it[u].x); lo[1] = fminf(lo[1], it[u].y); lo[2] = fminf(lo[2], it[u].z);
+        hi[0] = fmaxf(hi[0], it[u].x); hi[1] = fmaxf(hi[1], it[u].y); hi[2] = fmaxf(hi[2], it[u].z);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) { lo[d] = wave_min_dpp(lo[d]); hi[d] = wave_max_dpp(hi[d]); }
+    if (lane == 0) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        c.segs[np][li].cb[d] = enc_f(lo[d]);
+        c.segs[np][li].cb[d + 3] = enc_f(hi[d]);
+      }
+      plane(li, lo, hi);
+    }
+  }
+  // longer ranges by the workgroup
   for (uint32_t f = 0; f < nFix; f++) {
     const uint32_t li = sFix[f].x, pb = sFix[f].y, sz = sFix[f].z;
+    if (sz <= kFixWave) continue;
     float v[12];
     for (int j = 0; j < 12; j++) v[j] = (j % 6) < 3 ? INFINITY : -INFINITY;
     for (uint32_t i = threadIdx.x; i < sz; i += kEmitBlock) {
@@ -1164,11 +1209,7 @@ __global__ __launch_bounds__(kEmitBlock) void k_emit2(Ctx c, int pass) {
     if (threadIdx.x < 6) c.segs[np][li].cb[threadIdx.x] = enc_f(v[threadIdx.x]);
     if (threadIdx.x == 0) {
       const float lo[3] = {v[0], v[1], v[2]}, hi[3] = {v[3], v[4], v[5]};
-      int dim;
-      float pos;
-      choose_split(lo, hi, dim, pos);
-      c.segDim[np][li] = dim;
-      c.segPos[np][li] = pos;
+      plane(li, lo, hi);
     }
   }
 }
@@ -1909,7 +1950,10 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
   // so deeper trees take a check and another batch instead of slack here.
   int levels = 0;
   for (uint64_t m = (uint64_t)kMedium; m < n; m *= 2) levels++;
-  int batch = std::max(kPassesPerSync, (levels + 1) / 2);
+  // Up to 64K prims one pass more than that, for uneven splits (2000 points 260
+  // -> 241 us a build, 800, which take no pass, 223 -> 173, against four passes
+  // always).
+  int batch = levels ? std::max(std::min(kPassesPerSync, (levels + 1) / 2 + 1), (levels + 1) / 2) : 0;
   bool firstBatch = true;
   int specPass = -1, smallSlot = -1;
   uint32_t specGrid = 0;
