@@ -112,13 +112,15 @@ __global__ __launch_bounds__(256) void k_bkeys(Side sd, uint32_t numClouds) {
 }
 
 // points in sorted order, with their global index in w: a leaf's prims are
-// then one contiguous run for the refit and the queries
+// then one contiguous run for the refit and the queries.  Bound by the gathered
+// lines: a thread per point, an XCD at neighbouring workgroups of points (a
+// grid-stride loop over 1024 workgroups: 980 us for 2 x 38M points, 810 so)
 __global__ __launch_bounds__(256) void k_bgather(Side sd) {
-  for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < sd.n; t += gridDim.x * 256) {
-    const uint32_t i = sd.ids[t];
-    sd.spts[t] = make_float4(sd.pts[3 * (size_t)i], sd.pts[3 * (size_t)i + 1], sd.pts[3 * (size_t)i + 2],
-                             __uint_as_float(i));
-  }
+  const uint32_t t = xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+  if (t >= sd.n) return;
+  const uint32_t i = sd.ids[t];
+  sd.spts[t] = make_float4(sd.pts[3 * (size_t)i], sd.pts[3 * (size_t)i + 1], sd.pts[3 * (size_t)i + 2],
+                           __uint_as_float(i));
 }
 
 __global__ void k_binit(Side sd, Temp tp, uint32_t numClouds) {
@@ -367,85 +369,150 @@ __global__ __launch_bounds__(64) void k_bquery_deep(Side qs, Side ts, int32_t *n
   }
 }
 
-// adjoint of loss[c] = mean over the query cloud of d(q, nearest).
-// The query's own term goes to gradQ[qi] without an atomic: in the first
-// direction (ownFirst) every point of the side is a query exactly once, so
-// a store initialises gradQ; in the second only this lane touches
-// gradQ[qi] (the other lanes scatter into the other side's array), so a
-// plain read-modify-write adds to what the first direction scattered.  The
-// neighbour's term is scattered into gradT: queries run in Morton order, so
-// lanes next to each other often share their nearest point; a segmented
-// wave sum over runs of equal neighbour ids leaves one atomic per run.
-// The query, its result and the neighbour are read by sorted position.
-__global__ __launch_bounds__(256) void k_bback(Side qs, Side ts, float *loss, float *gradQ, float *gradT,
-                                               bool ownFirst) {
-  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-  const bool act = t < qs.n;
-  const uint32_t lane = lane_id();
-  uint32_t qi = 0, cloud = 0;
-  int32_t p = -1;
-  float contrib = 0.f, gx = 0.f, gy = 0.f, gz = 0.f;
-  if (act) {
-    const float4 qv = qs.spts[t];
-    qi = __float_as_uint(qv.w);
-    cloud = (uint32_t)(qs.keys[t] >> kCloudShift);
-    const uint32_t ps = qs.nnS[t];
-    if (ps != kNoSlot) {
-      const float4 pv = ts.spts[ps];
-      p = (int32_t)__float_as_uint(pv.w);
-      const float d = sqrtf(qs.d2S[t]);
-      const float g = 1.f / (float)(qs.off[cloud + 1] - qs.off[cloud]);
-      contrib = g * d;
-      if (d > 0.f) {
-        const float s = g / d;
-        gx = s * (qv.x - pv.x);
-        gy = s * (qv.y - pv.y);
-        gz = s * (qv.z - pv.z);
-      }
-    }
-    if (gradQ) {
-      float *o = gradQ + 3 * (size_t)qi;
-      if (ownFirst) {
-        o[0] = gx; o[1] = gy; o[2] = gz;
-      } else {
-        o[0] += gx; o[1] += gy; o[2] += gz;
-      }
-    }
+// adjoint of loss[c] = mean over the query cloud of d(q, nearest).  A
+// workgroup takes kBackChunk queries, and the neighbours' terms are summed by
+// sorted slot: both sides run in Morton order, so nearly all neighbours of a
+// chunk lie within a window of kBackWindow slots around its middle query's,
+// which is held in LDS and added to accT (by sorted slot too) once per chunk,
+// with whole lines of adds that follow each other; the rest is added straight
+// away, three lanes to a point.  ownQ, if given, receives a query's own term at its slot; gradQ, given
+// once all terms of a side are there, own term + accQ at its input index,
+// three lanes to a point.  Scattered memory requests and atomics, which are
+// done in memory and not in an XCD's L2, bound the kernel.  2 x 38M points:
+// 7.7 ms with both kinds of terms added at the input indices and the loss by
+// one atomic per wave, 4.6 ms with three lanes to a point and an XCD at neighbouring chunks, 2.9 ms as here.
+// (512 threads, 2048 queries and 2560 slots, four workgroups to a CU, against
+// 256/1024/2048 to 1024/8192/10240: within 2% of each other.)
+constexpr int kBackBlock = 512;
+constexpr uint32_t kBackChunk = 2048, kBackWindow = 2560;
+__global__ __launch_bounds__(kBackBlock) void k_bback(Side qs, Side ts, float *loss, float *ownQ, float *gradQ,
+                                                      const float *accQ, float *accT) {
+  __shared__ uint32_t sAt[kBackBlock];
+  __shared__ float sTerm[3 * kBackBlock];
+  __shared__ float sAcc[3 * kBackWindow];
+  __shared__ float sLoss[kBackBlock / kWave];
+  const uint32_t first = xcd_chunk(blockIdx.x, gridDim.x) * kBackChunk;
+  const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
+  const uint32_t last = min(first + kBackChunk, qs.n);
+  // (first < qs.n: the grid has a block per started chunk)
+  const uint32_t cloud0 = (uint32_t)(qs.keys[first] >> kCloudShift);
+  const uint32_t mid = qs.nnS[first + (last - first) / 2];
+  const uint32_t base = mid == kNoSlot || mid < kBackWindow / 2 ? 0 : mid - kBackWindow / 2;
+  if (accT) {
+    for (uint32_t i = threadIdx.x; i < 3 * kBackWindow; i += kBackBlock) sAcc[i] = 0.f;
+    __syncthreads();
   }
-  if (gradT) {
-    // segmented inclusive sums over runs of equal p (a run starts at lane 0
-    // or where p differs from the lane before)
-    const int32_t pPrev = __shfl_up(p, 1, kWave);
-    bool seen = lane == 0 || pPrev != p;
-    float sx = gx, sy = gy, sz = gz;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const float ux = __shfl_up(sx, o, kWave), uy = __shfl_up(sy, o, kWave), uz = __shfl_up(sz, o, kWave);
-      const bool us = __shfl_up((int)seen, o, kWave) != 0;
-      if (lane >= (uint32_t)o && !seen) {
-        sx += ux; sy += uy; sz += uz;
-        seen = us;
+  uint32_t *const wAt = sAt + wave * kWave;
+  float *const wTerm = sTerm + 3 * wave * kWave;
+  float sum = 0.f;
+  for (uint32_t tw = first + wave * kWave; tw < last; tw += kBackBlock) {
+    const uint32_t t = tw + lane;
+    const bool act = t < last;
+    uint32_t qi = 0, cloud = cloud0, p = kNoSlot;
+    float contrib = 0.f, gx = 0.f, gy = 0.f, gz = 0.f;
+    if (act) {
+      const float4 qv = qs.spts[t];
+      qi = __float_as_uint(qv.w);
+      cloud = (uint32_t)(qs.keys[t] >> kCloudShift);
+      p = qs.nnS[t];
+      if (p != kNoSlot) {
+        const float4 pv = ts.spts[p];
+        const float d = sqrtf(qs.d2S[t]);
+        const float g = 1.f / (float)(qs.off[cloud + 1] - qs.off[cloud]);
+        contrib = g * d;
+        if (d > 0.f) {
+          const float s = g / d;
+          gx = s * (qv.x - pv.x);
+          gy = s * (qv.y - pv.y);
+          gz = s * (qv.z - pv.z);
+        }
       }
     }
-    const int32_t pNext = __shfl_down(p, 1, kWave);
-    const bool runEnd = lane == kWave - 1 || pNext != p;
-    if (runEnd && p >= 0 && (sx != 0.f || sy != 0.f || sz != 0.f)) {
-      atomicAdd(&gradT[3 * (size_t)p + 0], -sx);
-      atomicAdd(&gradT[3 * (size_t)p + 1], -sy);
-      atomicAdd(&gradT[3 * (size_t)p + 2], -sz);
+    if (ownQ || gradQ) {
+      // (a wave's own part of the arrays: no barrier is needed)
+      wAt[lane] = qi;
+      wTerm[3 * lane] = gx;
+      wTerm[3 * lane + 1] = gy;
+      wTerm[3 * lane + 2] = gz;
+      sync_wave_lds();
+      const uint32_t n = 3 * min(last - tw, (uint32_t)kWave);
+#pragma unroll
+      for (uint32_t i = 0; i < 3; i++) {
+        const uint32_t c = i * kWave + lane;
+        if (c < n) {
+          const size_t at = 3 * (size_t)tw + c;
+          if (ownQ) ownQ[at] = wTerm[c];
+          if (gradQ) gradQ[3 * (size_t)wAt[c / 3] + c % 3] = wTerm[c] + accQ[at];
+        }
+      }
+      sync_wave_lds();
+    }
+    if (accT) {
+      const bool add = gx != 0.f || gy != 0.f || gz != 0.f;
+      const uint32_t w = p - base;  // (wraps below the window)
+      if (add && w < kBackWindow) {
+        atomicAdd(&sAcc[3 * w], -gx);
+        atomicAdd(&sAcc[3 * w + 1], -gy);
+        atomicAdd(&sAcc[3 * w + 2], -gz);
+      }
+      const bool out = add && w >= kBackWindow;
+      const uint64_t m = __ballot(out);
+      if (out) {
+        const uint32_t j = mbcnt(m);
+        wAt[j] = p;
+        wTerm[3 * j] = -gx;
+        wTerm[3 * j + 1] = -gy;
+        wTerm[3 * j + 2] = -gz;
+      }
+      sync_wave_lds();
+      const uint32_t n = 3 * (uint32_t)__popcll(m);
+      for (uint32_t c = lane; c < n; c += kWave) atomicAdd(&accT[3 * (size_t)wAt[c / 3] + c % 3], wTerm[c]);
+      sync_wave_lds();
+    }
+    if (loss) {
+      // the chunk's first cloud is summed up to its end, any other one by
+      // waves that lie in it or by single queries
+      const bool other = act && cloud != cloud0;
+      if (!other) sum += contrib;
+      const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane(cloud);
+      if (__all(!act || (other && cloud == c0))) {
+        float v = contrib;
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+        if (lane == 0) atomicAdd(&loss[c0], v);
+      } else if (other && contrib != 0.f) {
+        atomicAdd(&loss[cloud], contrib);
+      }
     }
   }
   if (loss) {
-    // one atomic per wave when all active lanes share the cloud
-    const uint32_t c0 = __shfl(cloud, 0, kWave);
-    const bool uniform = __all(!act || cloud == c0);
-    if (uniform) {
-      float sum = contrib;
-      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
-      if (lane == 0 && __any(act)) atomicAdd(&loss[c0], sum);
-    } else if (act && contrib != 0.f) {
-      atomicAdd(&loss[cloud], contrib);
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+    if (lane == 0) sLoss[wave] = sum;
+  }
+  __syncthreads();
+  if (loss && threadIdx.x == 0) {
+    float v = 0.f;
+    for (int w = 0; w < kBackBlock / kWave; w++) v += sLoss[w];
+    atomicAdd(&loss[cloud0], v);
+  }
+  if (accT)
+    for (uint32_t i = threadIdx.x; i < 3 * kBackWindow; i += kBackBlock) {
+      const float v = sAcc[i];
+      if (v != 0.f) atomicAdd(&accT[3 * (size_t)base + i], v);
     }
+}
+
+// the sums by sorted slot to their input indices, three lanes to a point
+__global__ __launch_bounds__(256) void k_bscatter(Side qs, const float *accQ, float *gradQ) {
+  const uint32_t t0 = (xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x) / kWave * kWave;
+  if (t0 >= qs.n) return;
+  const uint32_t lane = lane_id();
+  const uint32_t qi = t0 + lane < qs.n ? qs.ids[t0 + lane] : 0;
+  const uint32_t n = 3 * min(qs.n - t0, (uint32_t)kWave);
+#pragma unroll
+  for (uint32_t i = 0; i < 3; i++) {
+    const uint32_t c = i * kWave + lane;
+    const uint32_t at = (uint32_t)__shfl((int)qi, c / 3, kWave);
+    if (c < n) gradQ[3 * (size_t)at + c % 3] = accQ[3 * (size_t)t0 + c];
   }
 }
 
@@ -487,6 +554,8 @@ Plan make_plan(uint32_t numClouds, uint32_t nSrc, uint32_t nTgt) {
     p.roots[s] = L.take(4 * (size_t)std::max(numClouds, 1u));
     p.ctr[s] = L.take(4 * C_WORDS);
   }
+  // (the backward keeps 12 bytes a point of one side in keysB and valsB and
+  // of the other in ranges)
   p.keysB = L.take(8 * (size_t)nMax);
   p.valsB = L.take(4 * (size_t)nMax);
   p.ranges = L.take(8 * (2 * (size_t)nMax + 2));
@@ -533,7 +602,7 @@ int build_side(Side &sd, Temp &tp, const Args &a, const Plan &pl, hipStream_t s,
     CUBQL_HIP(hipMemcpyAsync(sd.ids, vr, 4 * (size_t)sd.n, hipMemcpyDeviceToDevice, s));
   }
   const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(div_up(sd.n, 256), (uint32_t)numCU * 4));
-  if (sd.n) k_bgather<<<grid, 256, 0, s>>>(sd);
+  if (sd.n) k_bgather<<<div_up(sd.n, 256), 256, 0, s>>>(sd);
   k_binit<<<std::max(1u, std::min<uint32_t>(div_up(a.numClouds, 256), 64)), 256, 0, s>>>(sd, tp, a.numClouds);
   k_bsingle_root<<<1, 64, 0, s>>>(sd);
   // depth bound: cloud bits + 30 Morton bits + mid splits of equal keys
@@ -606,22 +675,22 @@ int run(const Args &a, hipStream_t s) {
   prof_set(ps, (12.0 + 12.0 + 8.0 * 2 * 6 + 8.0 + 24.0 + 32.0) * (a.nSrc + a.nTgt), a.nSrc + a.nTgt);
   const uint32_t fg = 1024;
   if (a.loss) k_fill_f32<<<std::max(1u, std::min(div_up(a.numClouds, 256), fg)), 256, 0, s>>>(a.loss, 0.f, a.numClouds);
-  // gradSrc is initialised by the first backward direction's stores; an
-  // empty source side leaves it nothing to initialise
-  if (a.gradSrc && !a.nSrc) k_fill_f32<<<fg, 256, 0, s>>>(a.gradSrc, 0.f, 3 * (size_t)a.nSrc);
-  if (a.gradTgt) k_fill_f32<<<fg, 256, 0, s>>>(a.gradTgt, 0.f, 3 * (size_t)a.nTgt);
   ps = prof_begin(s);
   CUBQL_CHECK(query_dir(side[0], side[1], a.srcNN, a.srcD2, tp.ovf, a.prm, s));
   CUBQL_CHECK(query_dir(side[1], side[0], a.tgtNN, a.tgtD2, tp.ovf, a.prm, s));
   prof_end(ps, s, "batch_query");
   prof_set(ps, 20.0 * (a.nSrc + a.nTgt), a.nSrc + a.nTgt);
   ps = prof_begin(s);
-  if (a.loss || a.gradSrc || a.gradTgt) {
-    if (a.nSrc)
-      k_bback<<<div_up(a.nSrc, 256), 256, 0, s>>>(side[0], side[1], a.loss, a.gradSrc, a.gradTgt, true);
-    if (a.nTgt)
-      k_bback<<<div_up(a.nTgt, 256), 256, 0, s>>>(side[1], side[0], a.loss, a.gradTgt, a.gradSrc, false);
-  }
+  // the sides' sums by sorted slot, in build temporaries that are free now
+  float *accSrc = a.gradSrc ? (float *)tp.ranges : nullptr, *accTgt = a.gradTgt ? (float *)tp.keysB : nullptr;
+  if (accTgt) k_fill_f32<<<fg, 256, 0, s>>>(accTgt, 0.f, 3 * (size_t)a.nTgt);
+  if (a.nSrc && (a.loss || accSrc || accTgt))
+    k_bback<<<div_up(a.nSrc, kBackChunk), kBackBlock, 0, s>>>(side[0], side[1], a.loss, accSrc, nullptr, nullptr,
+                                                              accTgt);
+  if (a.nTgt && (a.loss || accSrc || accTgt))
+    k_bback<<<div_up(a.nTgt, kBackChunk), kBackBlock, 0, s>>>(side[1], side[0], a.loss, nullptr, a.gradTgt, accTgt,
+                                                              accSrc);
+  if (a.nSrc && accSrc) k_bscatter<<<div_up(a.nSrc, 256), 256, 0, s>>>(side[0], accSrc, a.gradSrc);
   prof_end(ps, s, "batch_backward");
   prof_set(ps, 68.0 * (a.nSrc + a.nTgt), a.nSrc + a.nTgt);
   CUBQL_LAUNCH_CHECK();
