@@ -7,14 +7,12 @@
 //     30-bit Morton keys with that cloud's own quantizer (radix.h:41-70); the
 //     sort key is (cloud << 30) | morton, the value the global point index;
 //   * one stable onesweep radix sort over all keys (segmented Morton sort);
-//   * one level-synchronous top-down hierarchy over the sorted keys where a
-//     range that spans several clouds is always split (its highest differing
-//     key bit is a cloud bit, so the split lands on a cloud boundary) and a
-//     single-cloud range follows radix.h:446-570 (leaf if <= T, equal keys
-//     split in the middle).  The node of each single-cloud range is that
-//     cloud's root, and its subtree is exactly the tree radix30Builder builds
-//     for the cloud alone;
-//   * exact bottom-up refit.
+//   * one hierarchy per cloud over its sorted keys, which follows
+//     radix.h:446-570 (leaf if <= T, equal keys split in the middle) and is
+//     exactly the tree radix30Builder builds for the cloud alone, with its
+//     exact bounds: runs of small clouds and the ranges of up to 16384 points
+//     that large clouds are split into are built by one workgroup each, from
+//     the roots down and back up, with the keys in LDS.
 // Queries run over all clouds in Morton order of the query side, each from
 // its cloud's root in the other side's forest, a wave sharing its queries'
 // subtrees; the adjoint of
@@ -58,16 +56,22 @@ struct Side {
 struct Temp {
   uint64_t *keysB;
   uint32_t *valsB;
-  uint2 *ranges;
-  uint32_t *levels;     // node ids level by level (capacity 2n+2)
+  float *acc;           // 3 floats per point of a side
+  uint4 *units;         // see k_bunits
+  uint4 *open;          // ranges of large clouds, level by level: node, begin, end
   void *sortWs;
   uint32_t *ovf;        // [0] count, [1] deep failures, then the list
 };
 
-// [C_LEVEL0 + l] node count of level l; [C_LSTART0 + l] its start in the
-// all-levels node list
-enum { C_NODES = 0, C_N = 1, C_LEVEL0 = 8, C_LSTART0 = 256, C_WORDS = 512 };
-constexpr int kMaxLevels = C_LSTART0 - C_LEVEL0 - 4;
+// [C_LSTART0 + l] start of level l in the list of open ranges
+enum { C_N = 1, C_UNITS = 2, C_TICKET = 3, C_OPEN = 4, C_LEVELS = 5, C_LSTART0 = 256, C_WORDS = 512 };
+
+// A unit has up to kUnit points (its keys, 64 KB of LDS, two workgroups to a
+// CU).  Clouds of up to kBin points share one.
+constexpr uint32_t kUnit = 16384, kBin = kUnit / 2;
+// levels of a tree: 30 key bits, then halvings of equal keys (18 of them reach
+// kUnit from 2^32, 14 reach one point from there)
+constexpr int kTopLevels = 64, kUnitLevels = 64;
 
 __device__ __forceinline__ uint32_t spread10(uint32_t v) {
   uint32_t x = v & 0x3ffu;
@@ -123,127 +127,222 @@ __global__ __launch_bounds__(256) void k_bgather(Side sd) {
                            __uint_as_float(i));
 }
 
-__global__ void k_binit(Side sd, Temp tp, uint32_t numClouds) {
-  for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < numClouds; c += gridDim.x * blockDim.x)
-    sd.rootOf[c] = kNoRoot;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    sd.ctr[C_NODES] = 2;
-    Node z;
-    for (int d = 0; d < 3; d++) { z.lo[d] = 0.f; z.hi[d] = 0.f; }
-    z.oc = 0;
-    sd.nodes[1] = z;
-    sd.ctr[C_LSTART0] = 0;
-    if (sd.n > 0) {
-      tp.ranges[0] = make_uint2(0u, sd.n);
-      tp.levels[0] = 0;
-      sd.ctr[C_LEVEL0] = 1;
-    }
-  }
-}
-
-// the root of a forest that holds a single cloud is node 0
-__global__ void k_bsingle_root(Side sd) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && sd.n > 0) {
-    const uint64_t c0 = sd.keys[0] >> kCloudShift, c1 = sd.keys[sd.n - 1] >> kCloudShift;
-    if (c0 == c1) sd.rootOf[c0] = 0;
-  }
-}
-
-__device__ __forceinline__ uint32_t find_split64(const uint64_t *keys, uint32_t b, uint32_t e) {
-  const uint64_t fk = keys[b], lk = keys[e - 1];
-  if (fk == lk) return (uint32_t)(((uint64_t)b + e) / 2);
-  const int nm = __clzll((unsigned long long)(fk ^ lk));
-  const uint64_t search = lk & (~0ull << (63 - nm));
+// where a range of one cloud's sorted keys is split (all high words equal)
+template <class Key>
+__device__ __forceinline__ uint32_t find_split(const Key *keys, uint32_t b, uint32_t e) {
+  const Key fk = keys[b], lk = keys[e - 1];
+  if (fk == lk) return b + (e - b) / 2;
+  const Key search = lk & ~(Key)(0x7fffffffu >> __clz((uint32_t)(fk ^ lk)));
   uint32_t lo = b, hi = e;
   while (hi > lo) {
-    const uint32_t mid = (lo + hi) / 2;
+    const uint32_t mid = lo + (hi - lo) / 2;
     if (keys[mid] < search) lo = mid + 1;
     else hi = mid;
   }
   return lo;
 }
 
-__global__ __launch_bounds__(256) void k_blevel(Side sd, Temp tp, uint32_t T, int level) {
-  __shared__ uint32_t ss[256 / kWave + 1];
-  __shared__ uint32_t sNode, sOpen;
-  const uint32_t nOpen = sd.ctr[C_LEVEL0 + level];
-  const uint32_t start = sd.ctr[C_LSTART0 + level];
-  const uint32_t *open = tp.levels + start;
-  uint32_t *next = tp.levels + start + nOpen;
-  if (blockIdx.x == 0 && threadIdx.x == 0) sd.ctr[C_LSTART0 + level + 1] = start + nOpen;
-  for (uint32_t b0 = blockIdx.x * 256; b0 < nOpen; b0 += gridDim.x * 256) {
-    const uint32_t i = b0 + threadIdx.x;
-    uint32_t node = 0, split = 0;
-    uint2 r = make_uint2(0, 0);
-    bool doSplit = false, multi = false;
-    if (i < nOpen) {
-      node = open[i];
-      r = tp.ranges[node];
-      const uint32_t size = r.y - r.x;
-      const uint32_t c0 = (uint32_t)(sd.keys[r.x] >> kCloudShift), c1 = (uint32_t)(sd.keys[r.y - 1] >> kCloudShift);
-      multi = c0 != c1;
-      if (multi) {
-        // the highest differing key bit is a cloud bit: the first key at or
-        // above the search key find_split64 would look for is the first point
-        // of cloud cs, which the offsets give without a search
-        const uint32_t cs = c1 & (~0u << (31 - __clz(c0 ^ c1)));
-        split = sd.off[cs];
-        doSplit = true;
-      } else if (size > T) {
-        split = find_split64(sd.keys, r.x, r.y);
-        doSplit = true;
+__device__ __forceinline__ uint32_t first_cloud_from(const uint32_t *off, uint32_t numClouds, uint64_t at) {
+  uint32_t lo = 0, hi = numClouds;
+  while (hi > lo) {
+    const uint32_t mid = lo + (hi - lo) / 2;
+    if (off[mid] < at) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// The units the trees are built in: for each kBin points, the clouds that
+// start there and have up to kBin points, as one unit (begin, end, first
+// cloud, end cloud), and at most one larger cloud after them, a unit of its
+// own or, above `most` points, an open range.  Nodes need no counter: a tree
+// over points [b, e) has at most 2 (e - b) - 1 nodes, and a unit keeps its own
+// in [2b, 2e).
+__global__ __launch_bounds__(256) void k_bunits(Side sd, Temp tp, uint32_t numClouds, uint32_t most) {
+  const uint32_t step = gridDim.x * 256, first = blockIdx.x * 256 + threadIdx.x;
+  for (uint32_t c = first; c < numClouds; c += step)
+    if (sd.off[c] == sd.off[c + 1]) sd.rootOf[c] = kNoRoot;
+  for (uint32_t k = first; (uint64_t)k * kBin < sd.n; k += step) {
+    const uint32_t c0 = first_cloud_from(sd.off, numClouds, (uint64_t)k * kBin);
+    uint32_t c1 = first_cloud_from(sd.off, numClouds, ((uint64_t)k + 1) * kBin);
+    if (c1 == c0) continue;
+    const uint32_t b = sd.off[c1 - 1], e = sd.off[c1];
+    if (e - b > kBin) {
+      c1--;
+      if (e - b <= most) {
+        tp.units[atomicAdd(&sd.ctr[C_UNITS], 1u)] = make_uint4(b, e, c1, c1 + 1);
       } else {
-        sd.nodes[node].oc = pack_oc(r.x, size);
+        sd.rootOf[c1] = 2 * b + 1;
+        tp.open[atomicAdd(&sd.ctr[C_OPEN], 1u)] = make_uint4(2 * b + 1, b, e, 0u);
       }
     }
-    uint32_t tot;
-    const uint32_t ex = block_excl_scan<256>(doSplit ? 1u : 0u, ss, &tot);
-    if (threadIdx.x == 0 && tot) {
-      sNode = atomicAdd(&sd.ctr[C_NODES], 2 * tot);
-      sOpen = atomicAdd(&sd.ctr[C_LEVEL0 + level + 1], 2 * tot);
+    if (sd.off[c1] > sd.off[c0])
+      tp.units[atomicAdd(&sd.ctr[C_UNITS], 1u)] = make_uint4(sd.off[c0], sd.off[c1], c0, c1);
+  }
+}
+
+// One workgroup splits the open ranges, level by level, until none has more
+// than `most` points; the parts become units of one node (begin, end, node,
+// kNoRoot).  The children of a range that is split at s are nodes 2s and
+// 2s + 1, which no unit uses: s begins one, and its own start at 2s + 2.
+__global__ __launch_bounds__(1024) void k_btop(Side sd, Temp tp, uint32_t most) {
+  __shared__ uint32_t sEnd;
+  uint32_t start = 0, end = sd.ctr[C_OPEN];
+  int level = 0;
+  if (threadIdx.x == 0) sEnd = end;
+  while (start < end) {
+    __syncthreads();
+    if (threadIdx.x == 0) sd.ctr[C_LSTART0 + level] = start;
+    for (uint32_t i = start + threadIdx.x; i < end; i += 1024) {
+      const uint4 r = tp.open[i];
+      const uint32_t s = find_split(sd.keys, r.y, r.z);
+      sd.nodes[r.x].oc = pack_oc(2 * (uint64_t)s, 0);
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const uint32_t b = h ? s : r.y, e = h ? r.z : s;
+        if (e - b > most) tp.open[atomicAdd(&sEnd, 1u)] = make_uint4(2 * s + h, b, e, 0u);
+        else tp.units[atomicAdd(&sd.ctr[C_UNITS], 1u)] = make_uint4(b, e, 2 * s + h, kNoRoot);
+      }
     }
     __syncthreads();
-    if (doSplit) {
-      const uint32_t child = sNode + 2 * ex;
-      sd.nodes[node].oc = pack_oc(child, 0);
-      tp.ranges[child] = make_uint2(r.x, split);
-      tp.ranges[child + 1] = make_uint2(split, r.y);
-      next[sOpen + 2 * ex] = child;
-      next[sOpen + 2 * ex + 1] = child + 1;
-      if (multi) {
-        const uint64_t cl = sd.keys[r.x] >> kCloudShift, cm = sd.keys[split - 1] >> kCloudShift;
-        if (cl == cm) sd.rootOf[cl] = child;
-        const uint64_t cr = sd.keys[split] >> kCloudShift, ce = sd.keys[r.y - 1] >> kCloudShift;
-        if (cr == ce) sd.rootOf[cr] = child + 1;
+    start = end;
+    end = sEnd;
+    level++;
+  }
+  if (threadIdx.x == 0) {
+    sd.ctr[C_LEVELS] = (uint32_t)level;
+    sd.ctr[C_LSTART0 + level] = end;
+  }
+}
+
+__device__ __forceinline__ void fit_leaf(const Side &sd, Node *nd) {
+  const uint64_t oc = nd->oc;
+  const uint32_t cnt = oc_count(oc), o = (uint32_t)oc_offset(oc);
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  for (uint32_t j = 0; j < cnt; j += 4) {
+    float4 p[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) p[u] = sd.spts[o + min(j + u, cnt - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const float x[3] = {p[u].x, p[u].y, p[u].z};
+      for (int d = 0; d < 3; d++) {
+        lo[d] = fminf(lo[d], x[d]);
+        hi[d] = fmaxf(hi[d], x[d]);
       }
     }
+  }
+  for (int d = 0; d < 3; d++) { nd->lo[d] = lo[d]; nd->hi[d] = hi[d]; }
+}
+
+// an inner node from its children
+__device__ __forceinline__ void fit_node(const Side &sd, Node *nd) {
+  const uint32_t o = (uint32_t)oc_offset(nd->oc);
+  const Node l = sd.nodes[o], r = sd.nodes[o + 1];
+  for (int d = 0; d < 3; d++) {
+    nd->lo[d] = fminf(l.lo[d], r.lo[d]);
+    nd->hi[d] = fmaxf(l.hi[d], r.hi[d]);
+  }
+}
+
+// bounds of the open ranges' nodes, the deepest level first
+__global__ __launch_bounds__(1024) void k_btop_fit(Side sd, Temp tp) {
+  for (int l = (int)sd.ctr[C_LEVELS] - 1; l >= 0; l--) {
+    const uint32_t end = sd.ctr[C_LSTART0 + l + 1];
+    for (uint32_t i = sd.ctr[C_LSTART0 + l] + threadIdx.x; i < end; i += 1024) fit_node(sd, &sd.nodes[tp.open[i].x]);
     __syncthreads();
   }
 }
 
-// bottom-up refit, one launch per level from the deepest (no atomics)
-__global__ void k_brefit_level(Side sd, Temp tp, int level) {
-  const uint32_t n = sd.ctr[C_LEVEL0 + level];
-  const uint32_t *ids = tp.levels + sd.ctr[C_LSTART0 + level];
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    Node *nd = &sd.nodes[ids[i]];
-    const uint64_t oc = nd->oc;
-    const uint32_t cnt = oc_count(oc), o = (uint32_t)oc_offset(oc);
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    if (cnt) {
-      for (uint32_t j = 0; j < cnt; j++) {
-        const float4 p = sd.spts[o + j];
-        const float x[3] = {p.x, p.y, p.z};
-        for (int d = 0; d < 3; d++) {
-          lo[d] = fminf(lo[d], x[d]);
-          hi[d] = fmaxf(hi[d], x[d]);
-        }
-      }
+// The trees of the units: a workgroup takes the next unit, splits its ranges
+// level by level with the keys in LDS, a thread per node (a node's range stands
+// in its own offset and count until it is split), and then fits the levels'
+// bounds from the last one up.  Latency of the levels bounds it.
+// @@
+#ifndef UB
+#define UB 1024
+#endif
+constexpr int kUnitBlock = UB;
+__global__ __launch_bounds__(kUnitBlock) void k_bunit(Side sd, Temp tp, uint32_t T) {
+  __shared__ uint32_t sKey[kUnit];
+  __shared__ uint32_t ss[kUnitBlock / kWave + 1], sLo[kUnitLevels], sHi[kUnitLevels];
+  __shared__ uint32_t sUnit;
+  const uint32_t numUnits = sd.ctr[C_UNITS], tid = threadIdx.x;
+  for (;;) {
+    if (tid == 0) sUnit = atomicAdd(&sd.ctr[C_TICKET], 1u);
+    __syncthreads();
+    const uint32_t u = sUnit;
+    if (u >= numUnits) return;
+    const uint4 un = tp.units[u];
+    const uint32_t b = un.x, size = un.y - un.x;
+    // (a unit of more points than kUnit is one leaf)
+    if (size <= kUnit)
+      for (uint32_t i = tid; i < size; i += kUnitBlock) sKey[i] = (uint32_t)sd.keys[b + i] & ((1u << kCloudShift) - 1);
+    uint32_t lo, hi, at;
+    if (un.w == kNoRoot) {
+      lo = un.z;
+      hi = lo + 1;
+      at = 2 * b + 2;
+      if (tid == 0) sd.nodes[lo].oc = pack_oc(b, size);
     } else {
-      const Node l = sd.nodes[o], r = sd.nodes[o + 1];
-      for (int d = 0; d < 3; d++) { lo[d] = fminf(l.lo[d], r.lo[d]); hi[d] = fmaxf(l.hi[d], r.hi[d]); }
+      lo = hi = 2 * b;
+      for (uint32_t c0 = un.z; c0 < un.w; c0 += kUnitBlock) {
+        const uint32_t c = c0 + tid;
+        const uint32_t cb = c < un.w ? sd.off[c] : 0u, ce = c < un.w ? sd.off[c + 1] : 0u;
+        uint32_t tot;
+        const uint32_t ex = block_excl_scan<kUnitBlock>(ce > cb ? 1u : 0u, ss, &tot);
+        if (ce > cb) {
+          sd.nodes[hi + ex].oc = pack_oc(cb, ce - cb);
+          sd.rootOf[c] = hi + ex;
+        }
+        hi += tot;
+      }
+      at = (hi + 1) & ~1u;
     }
-    for (int d = 0; d < 3; d++) { nd->lo[d] = lo[d]; nd->hi[d] = hi[d]; }
+    int level = 0;
+    const uint32_t level1 = at;
+    while (lo < hi) {
+      __syncthreads();
+      if (tid == 0) {
+        sLo[level] = lo;
+        sHi[level] = hi;
+      }
+      const uint32_t first = at;
+      for (uint32_t i0 = lo; i0 < hi; i0 += kUnitBlock) {
+        const uint32_t node = i0 + tid;
+        const uint64_t oc = node < hi ? sd.nodes[node].oc : 0ull;
+        const uint32_t cnt = oc_count(oc), p = (uint32_t)oc_offset(oc);
+        const bool split = cnt > T;
+        uint32_t s = 0;
+        if (split) s = b + find_split(sKey, p - b, p - b + cnt);
+        uint32_t tot;
+        const uint32_t ex = block_excl_scan<kUnitBlock>(split ? 1u : 0u, ss, &tot);
+        if (split) {
+          const uint32_t child = at + 2 * ex;
+          sd.nodes[node].oc = pack_oc(child, 0);
+          sd.nodes[child].oc = pack_oc(p, s - p);
+          sd.nodes[child + 1].oc = pack_oc(s, p + cnt - s);
+        }
+        at += 2 * tot;
+      }
+      lo = first;
+      hi = at;
+      level++;
+    }
+    __syncthreads();
+    // (all leaves together: they lie on several levels)
+    for (int l = 0; l < 2; l++) {
+      const uint32_t end = l ? at : sHi[0];
+      for (uint32_t i = (l ? level1 : sLo[0]) + tid; i < end; i += kUnitBlock)
+        if (oc_count(sd.nodes[i].oc)) fit_leaf(sd, &sd.nodes[i]);
+    }
+    __syncthreads();
+    for (int l = level - 1; l >= 0; l--) {
+      const uint32_t end = sHi[l];
+      for (uint32_t i = sLo[l] + tid; i < end; i += kUnitBlock)
+        if (!oc_count(sd.nodes[i].oc)) fit_node(sd, &sd.nodes[i]);
+      __syncthreads();
+    }
   }
 }
 
@@ -533,9 +632,8 @@ struct Layout {
 
 struct Plan {
   size_t keys[2], ids[2], spts[2], nnS[2], d2S[2], nodes[2], roots[2], ctr[2];
-  size_t keysB, valsB, ranges, levels, sortWs, ovf;
+  size_t keysB, valsB, acc, open, units, sortWs, ovf;
   size_t total;
-  uint32_t maxLevels;
 };
 
 Plan make_plan(uint32_t numClouds, uint32_t nSrc, uint32_t nTgt) {
@@ -554,12 +652,14 @@ Plan make_plan(uint32_t numClouds, uint32_t nSrc, uint32_t nTgt) {
     p.roots[s] = L.take(4 * (size_t)std::max(numClouds, 1u));
     p.ctr[s] = L.take(4 * C_WORDS);
   }
-  // (the backward keeps 12 bytes a point of one side in keysB and valsB and
-  // of the other in ranges)
+  // (the backward keeps 12 bytes a point of one side in keysB and valsB, and
+  // of the other in acc)
   p.keysB = L.take(8 * (size_t)nMax);
   p.valsB = L.take(4 * (size_t)nMax);
-  p.ranges = L.take(8 * (2 * (size_t)nMax + 2));
-  p.levels = L.take(4 * (2 * (size_t)nMax + 2));
+  p.acc = L.take(12 * (size_t)nMax);
+  const size_t maxOpen = (size_t)kTopLevels * (nMax / kUnit);
+  p.open = L.take(16 * std::max<size_t>(maxOpen, 1));
+  p.units = L.take(16 * (2 * ((size_t)nMax / kBin + 1) + 2 * maxOpen));
   int cloudBits = 0;
   while ((1u << cloudBits) < std::max(numClouds, 1u)) cloudBits++;
   p.sortWs = L.take(radix_sort_ws_bytes(nMax, kCloudShift + cloudBits));
@@ -601,18 +701,13 @@ int build_side(Side &sd, Temp &tp, const Args &a, const Plan &pl, hipStream_t s,
     CUBQL_HIP(hipMemcpyAsync(sd.keys, kr, 8 * (size_t)sd.n, hipMemcpyDeviceToDevice, s));
     CUBQL_HIP(hipMemcpyAsync(sd.ids, vr, 4 * (size_t)sd.n, hipMemcpyDeviceToDevice, s));
   }
-  const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(div_up(sd.n, 256), (uint32_t)numCU * 4));
   if (sd.n) k_bgather<<<div_up(sd.n, 256), 256, 0, s>>>(sd);
-  k_binit<<<std::max(1u, std::min<uint32_t>(div_up(a.numClouds, 256), 64)), 256, 0, s>>>(sd, tp, a.numClouds);
-  k_bsingle_root<<<1, 64, 0, s>>>(sd);
-  // depth bound: cloud bits + 30 Morton bits + mid splits of equal keys
-  int midBits = 0;
-  const uint32_t maxCloud = a.prm.maxCloudSize ? a.prm.maxCloudSize : std::max(sd.n, 1u);
-  while ((1ull << midBits) < maxCloud) midBits++;
-  const int levels = std::min(cbits + kCloudShift + midBits + 2, kMaxLevels);
-  const uint32_t T = (uint32_t)std::max(1, std::min(a.prm.leafSize, 65535));
-  for (int l = 0; l < levels; l++) k_blevel<<<grid, 256, 0, s>>>(sd, tp, T, l);
-  for (int l = levels - 1; l >= 0; l--) k_brefit_level<<<grid, 256, 0, s>>>(sd, tp, l);
+  const uint32_t T = (uint32_t)std::max(1, std::min(a.prm.leafSize, 65535)), most = std::max(kUnit, T);
+  const uint32_t bins = div_up(sd.n, kBin), work = std::max(std::max(bins, a.numClouds), 1u);
+  k_bunits<<<std::min(div_up(work, 256), (uint32_t)numCU * 4), 256, 0, s>>>(sd, tp, a.numClouds, most);
+  if (sd.n > most) k_btop<<<1, 1024, 0, s>>>(sd, tp, most);
+  if (sd.n) k_bunit<<<std::min(2 * bins, 2 * (uint32_t)numCU), kUnitBlock, 0, s>>>(sd, tp, T);
+  if (sd.n > most) k_btop_fit<<<1, 1024, 0, s>>>(sd, tp);
   CUBQL_LAUNCH_CHECK();
   return CUBQL_OK;
 }
@@ -663,8 +758,9 @@ int run(const Args &a, hipStream_t s) {
   Temp tp;
   tp.keysB = (uint64_t *)(a.ws + pl.keysB);
   tp.valsB = (uint32_t *)(a.ws + pl.valsB);
-  tp.ranges = (uint2 *)(a.ws + pl.ranges);
-  tp.levels = (uint32_t *)(a.ws + pl.levels);
+  tp.acc = (float *)(a.ws + pl.acc);
+  tp.open = (uint4 *)(a.ws + pl.open);
+  tp.units = (uint4 *)(a.ws + pl.units);
   tp.sortWs = a.ws + pl.sortWs;
   tp.ovf = (uint32_t *)(a.ws + pl.ovf);
 
@@ -681,8 +777,8 @@ int run(const Args &a, hipStream_t s) {
   prof_end(ps, s, "batch_query");
   prof_set(ps, 20.0 * (a.nSrc + a.nTgt), a.nSrc + a.nTgt);
   ps = prof_begin(s);
-  // the sides' sums by sorted slot, in build temporaries that are free now
-  float *accSrc = a.gradSrc ? (float *)tp.ranges : nullptr, *accTgt = a.gradTgt ? (float *)tp.keysB : nullptr;
+  // the sides' sums by sorted slot
+  float *accSrc = a.gradSrc ? tp.acc : nullptr, *accTgt = a.gradTgt ? (float *)tp.keysB : nullptr;
   if (accTgt) k_fill_f32<<<fg, 256, 0, s>>>(accTgt, 0.f, 3 * (size_t)a.nTgt);
   if (a.nSrc && (a.loss || accSrc || accTgt))
     k_bback<<<div_up(a.nSrc, kBackChunk), kBackBlock, 0, s>>>(side[0], side[1], a.loss, accSrc, nullptr, nullptr,
