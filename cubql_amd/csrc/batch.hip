@@ -257,12 +257,11 @@ __global__ __launch_bounds__(1024) void k_btop_fit(Side sd, Temp tp) {
 // The trees of the units: a workgroup takes the next unit, splits its ranges
 // level by level with the keys in LDS, a thread per node (a node's range stands
 // in its own offset and count until it is split), and then fits the levels'
-// bounds from the last one up.  Latency of the levels bounds it.
-// @@
-#ifndef UB
-#define UB 1024
-#endif
-constexpr int kUnitBlock = UB;
+// bounds from the last one up.  2 x 38M points in 4096 clouds: 0.70 ms a side,
+// and 0.12 ms for the open ranges; 1.76 ms with two launches per level.  Bound
+// by the latency of the levels.  (1024 threads, two workgroups to a CU; 512:
+// the same, 256: 3% of the whole call slower.)
+constexpr int kUnitBlock = 1024;
 __global__ __launch_bounds__(kUnitBlock) void k_bunit(Side sd, Temp tp, uint32_t T) {
   __shared__ uint32_t sKey[kUnit];
   __shared__ uint32_t ss[kUnitBlock / kWave + 1], sLo[kUnitLevels], sHi[kUnitLevels];
@@ -408,10 +407,11 @@ constexpr int kBatchLeafLanes = 32;
 // queries of side `qs` against the forest of side `ts`, in Morton order of
 // qs: a wave per qpw queries (wave_closest.h).  2 x 38M queries over 4096
 // clouds: 16.5 ms with one query per lane on a private stack, 8.2 ms here;
-// bound by the address unit (16-point leaves) and VALU issue.
+// bound by the address unit (16-point leaves) and VALU issue.  (Held to 64
+// registers: 8 waves to a SIMD, 3.83 ms a launch, 3.92 with 7.)
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_bquery(Side qs, Side ts, uint32_t qpw, int32_t *nn, float *d2,
-                                                  uint32_t *ovf) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
+void k_bquery(Side qs, Side ts, uint32_t qpw, int32_t *nn, float *d2, uint32_t *ovf) {
   __shared__ WaveTasksAux tasks[BLOCK / kWave];
   const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
   // queries sorted by (cloud, Morton key): one contiguous run per XCD
@@ -423,13 +423,32 @@ __global__ __launch_bounds__(BLOCK) void k_bquery(Side qs, Side ts, uint32_t qpw
   const bool live = act && root != kNoRoot;
   const uint64_t word = live ? ts.nodes[root].oc : 0ull;
   const unsigned long long none = closest_none(INFINITY);
-  bool failed;
-  uint32_t slot;
-  const unsigned long long best =
-      wave_closest<kBatchLeafLanes>(tasks[wave], (const cubql_node3f *)ts.nodes, live, word, qv.x, qv.y, qv.z, none,
-                                    LeafSlots{ts.spts}, &failed, &slot);
+  unsigned long long best = none;
+  uint32_t slot = kNoSlot;
+  // Queries that lost a task run again, eight at a time and then alone (the
+  // queue holds more of each), and last in the deep kernel.
+  uint64_t lost = 0, todo = __ballot(live);
+  for (uint32_t together = kWave; todo; together /= 8) {
+    uint64_t again = 0;
+    while (todo) {
+      const bool on = ((todo >> lane) & 1u) && mbcnt(todo) < together;
+      bool failed;
+      uint32_t at;
+      const unsigned long long k =
+          wave_closest<kBatchLeafLanes>(tasks[wave], (const cubql_node3f *)ts.nodes, on, word, qv.x, qv.y, qv.z, none,
+                                        LeafSlots{ts.spts}, &failed, &at);
+      todo &= ~__ballot(on);
+      again |= __ballot(on && failed);
+      if (on && !failed) {
+        best = k;
+        slot = at;
+      }
+    }
+    if (together == 1) lost = again;
+    else todo = again;
+  }
   if (!act) return;
-  if (live && failed) {
+  if ((lost >> lane) & 1u) {
     ovf[2 + atomicAdd(&ovf[0], 1u)] = t;
     return;
   }
@@ -474,12 +493,13 @@ __global__ __launch_bounds__(64) void k_bquery_deep(Side qs, Side ts, int32_t *n
 // chunk lie within a window of kBackWindow slots around its middle query's,
 // which is held in LDS and added to accT (by sorted slot too) once per chunk,
 // with whole lines of adds that follow each other; the rest is added straight
-// away, three lanes to a point.  ownQ, if given, receives a query's own term at its slot; gradQ, given
-// once all terms of a side are there, own term + accQ at its input index,
-// three lanes to a point.  Scattered memory requests and atomics, which are
-// done in memory and not in an XCD's L2, bound the kernel.  2 x 38M points:
-// 7.7 ms with both kinds of terms added at the input indices and the loss by
-// one atomic per wave, 4.6 ms with three lanes to a point and an XCD at neighbouring chunks, 2.9 ms as here.
+// away, three lanes to a point.  ownQ, if given, receives a query's own term
+// at its slot; gradQ, given once all terms of a side are there, own term +
+// accQ at its input index, three lanes to a point.  Scattered memory requests
+// and atomics, which are done in memory and not in an XCD's L2, bound the
+// kernel.  2 x 38M points: 7.7 ms with both kinds of terms added at the input
+// indices and the loss by one atomic per wave, 4.6 ms with three lanes to a
+// point and an XCD at neighbouring chunks, 2.9 ms as here.
 // (512 threads, 2048 queries and 2560 slots, four workgroups to a CU, against
 // 256/1024/2048 to 1024/8192/10240: within 2% of each other.)
 constexpr int kBackBlock = 512;

@@ -348,8 +348,8 @@ int cubql_points_distance_backward_f3(const float *d_points, uint32_t numPoints,
    stackDepth    8, 16, 32 or 64: checked, and has no effect (a query wave
                  shares one task queue; it took the place of the lanes'
                  traversal stacks);
-   maxCloudSize  optional upper bound on any cloud's size (0 = unknown); it
-                 only bounds the number of hierarchy launches. */
+   maxCloudSize  optional upper bound on any cloud's size (0 = unknown): has
+                 no effect (the number of launches does not depend on it). */
 typedef struct {
   int leafSize;
   int blockSize;
