@@ -183,6 +183,28 @@ __device__ __forceinline__ void bin_add(int32_t *bins, int nb, float eps, const 
   }
 }
 
+// As bin_add for many prims per bin: a bound is only sent to LDS as an atomic
+// if it is beyond the one that a plain read finds there, which few are.
+// (Atomics of lanes that meet in a bin, as neighbouring prims do, run one
+// after the other; reads of one word do not.)
+__device__ __forceinline__ void bin_add_read(int32_t *bins, int nb, float eps, const Item &it,
+                                             const float (&clo)[3], const float (&chi)[3]) {
+  const int32_t v[6] = {enc_f(it.a.x), enc_f(it.a.y), enc_f(it.a.z), enc_f(it.b.x), enc_f(it.b.y), enc_f(it.b.z)};
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    int32_t *w = bins + (d * nb + sah_bin(item_center(it, d), clo[d], chi[d], nb, eps)) * kBinWords;
+    const int4 a = *reinterpret_cast<const int4 *>(w);
+    const int2 b = *reinterpret_cast<const int2 *>(w + 4);
+    if (v[0] < a.x) atomicMin(&w[0], v[0]);
+    if (v[1] < a.y) atomicMin(&w[1], v[1]);
+    if (v[2] < a.z) atomicMin(&w[2], v[2]);
+    if (v[3] > a.w) atomicMax(&w[3], v[3]);
+    if (v[4] > b.x) atomicMax(&w[4], v[4]);
+    if (v[5] > b.y) atomicMax(&w[5], v[5]);
+    atomicAdd(&w[6], 1);
+  }
+}
+
 // Split costs for the candidates held by this lane's (dim, bin): the left
 // side is the prefix scan over bins shifted by one lane, the right side the
 // prefix scan over the reversed bins read back from lane rev.
@@ -439,8 +461,13 @@ __device__ __forceinline__ void seg_cb(const Seg &g, float (&lo)[3], float (&hi)
 }
 
 // Bin: one LDS bin set per binning tile, written out as that tile's partial.
-__global__ __launch_bounds__(kBlock) void k_bin(Ctx c, int level) {
-  __shared__ int32_t sBins[3 * kMaxBins * kBinWords];
+// Bound by LDS.  1.31M prims, the first level: 136 us with 21 atomics per prim
+// from 256 threads, 42 us with bin_add_read from 512 (all levels 1349 -> 535
+// us).  (Tiles of 4096 or 2048 prims: 3% and 6% of the build slower, through
+// the sums over them.)
+constexpr int kBinBlock = 512;
+__global__ __launch_bounds__(kBinBlock) void k_bin(Ctx c, int level) {
+  __shared__ __align__(16) int32_t sBins[3 * kMaxBins * kBinWords];
   __shared__ uint32_t sSeg;
   const int par = level & 1;
   const uint32_t nbt = c.ctr->numBinTiles;
@@ -450,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void k_bin(Ctx c, int level) {
   const int W = 3 * nb * kBinWords;
   for (uint32_t bt = blockIdx.x; bt < nbt; bt += gridDim.x) {
     if (threadIdx.x == 0) sSeg = find_seg(c.binStart, nSeg, bt);
-    for (int w = threadIdx.x; w < W; w += kBlock) sBins[w] = bin_init(w);
+    for (int w = threadIdx.x; w < W; w += kBinBlock) sBins[w] = bin_init(w);
     sync_block_lds();
     const uint32_t s = sSeg;
     const Seg g = c.segs[par][s];
@@ -458,16 +485,18 @@ __global__ __launch_bounds__(kBlock) void k_bin(Ctx c, int level) {
     seg_cb(g, clo, chi);
     const uint32_t b0 = g.begin + (bt - c.binStart[s]) * kBinTile;
     const uint32_t e0 = min(b0 + (uint32_t)kBinTile, g.end);
-    for (uint32_t i = b0 + threadIdx.x; i < e0; i += kBlock) bin_add(sBins, nb, c.binEps, src[i], clo, chi);
+    for (uint32_t i = b0 + threadIdx.x; i < e0; i += kBinBlock) bin_add_read(sBins, nb, c.binEps, src[i], clo, chi);
     sync_block_lds();
     int32_t *out = c.partial + (size_t)bt * W;
-    for (int w = threadIdx.x; w < W; w += kBlock) out[w] = sBins[w];
+    for (int w = threadIdx.x; w < W; w += kBinBlock) out[w] = sBins[w];
     sync_block_lds();
   }
 }
 
 // Select: reduce a node's partials, evaluate SAH, record the decision and
-// the node's box (the union of its bins); leaves are final here.
+// the node's box (the union of its bins); leaves are final here.  Bound by the
+// latency of the partials, eight in flight (the root of 1.31M prims, 160 of
+// them: 93 us one after the other, 32 us so).
 __global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
   __shared__ int32_t sBins[3 * kMaxBins * kBinWords];
   const int par = level & 1;
@@ -480,10 +509,16 @@ __global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
       const int k = w & (kBinWords - 1);
       int32_t acc = bin_init(w);
       const int32_t *p = c.partial + (size_t)tb * W + w;
-      for (uint32_t t = tb; t < te; t++, p += W) {
-        const int32_t v = *p;
-        acc = k < 3 ? min(acc, v) : (k < 6 ? max(acc, v) : acc + v);
+      auto add = [&](int32_t v) { acc = k < 3 ? min(acc, v) : (k < 6 ? max(acc, v) : acc + v); };
+      uint32_t t = tb;
+      for (; t + 8 <= te; t += 8, p += 8 * (size_t)W) {
+        int32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = p[u * (size_t)W];
+#pragma unroll
+        for (int u = 0; u < 8; u++) add(v[u]);
       }
+      for (; t < te; t++, p += W) add(*p);
       sBins[w] = acc;
     }
     sync_block_lds();
@@ -958,7 +993,7 @@ int sah_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T
   while (n) {
     for (int i = 0; i < kLevelsPerSync && level < (int)maxLevels; i++, level++) {
       int pb = prof_begin(s);
-      k_bin<<<binGrid, kBlock, 0, s>>>(c, level);
+      k_bin<<<binGrid, kBinBlock, 0, s>>>(c, level);
       prof_end(pb, s, "sah_bin");
       if (pb >= 0) binSlots.push_back({pb, level});
       k_select<<<selGrid, kBlock, 0, s>>>(c, level);
