@@ -33,21 +33,25 @@ __device__ inline void choose_split(const float lo[3], const float hi[3], int &d
 
 // One wave copies a finished small segment's cnt local nodes to the final
 // array: local node 0 to `root`, local node j >= 1 to base + j - 1, with an
-// inner node's child offset (a local id) rebased the same way.  A node moves
-// as two 16-byte words; the second holds hi[1], hi[2] and oc.
+// inner node's child offset (a local id) rebased the same way.  With place,
+// the local nodes' pairs are put in another order: pair p, of local nodes
+// 1 + 2p and 2 + 2p, as the place[p]-th.  A node moves as two 16-byte words;
+// the second holds hi[1], hi[2] and oc.
 __device__ __forceinline__ void copy_local_nodes(const Node *loc, uint32_t cnt, uint32_t root, uint32_t base,
-                                                 Node *out) {
+                                                 Node *out, const uint16_t *place = nullptr) {
   const uint4 *src = reinterpret_cast<const uint4 *>(loc);
   for (uint32_t j = lane_id(); j < cnt; j += kWave) {
+    const uint32_t to = j == 0 || !place ? j : 1 + 2 * (uint32_t)place[(j - 1) / 2] + ((j - 1) & 1u);
     const uint4 a = src[2 * j];
     uint4 b = src[2 * j + 1];
     const uint64_t oc = ((uint64_t)b.w << 32) | b.z;
     if (oc_count(oc) == 0) {
-      const uint64_t g = pack_oc(base + (uint32_t)oc_offset(oc) - 1, 0);
+      const uint32_t child = (uint32_t)oc_offset(oc) - 1;
+      const uint64_t g = pack_oc(base + (place ? 2 * (uint32_t)place[child / 2] : child), 0);
       b.z = (uint32_t)g;
       b.w = (uint32_t)(g >> 32);
     }
-    uint4 *d = reinterpret_cast<uint4 *>(out + (j == 0 ? root : base + j - 1));
+    uint4 *d = reinterpret_cast<uint4 *>(out + (j == 0 ? root : base + to - 1));
     d[0] = a;
     d[1] = b;
   }

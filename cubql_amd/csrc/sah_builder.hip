@@ -747,8 +747,233 @@ __global__ __launch_bounds__(1024) void k_emit(Ctx c, int level) {
 // One wave finishes a node of <= kSmall prims (or a leaf of any size) in
 // LDS with the same rules; nodes are numbered locally (local 0 = the node
 // itself) into loc[2*begin + j] and renumbered by k_small_scan/k_small_emit.
+// A split's children are the pair 1 + 2 * (its place among the splits, in
+// depth-first order, left first).
+//
+// VALU issue bounds it: a split takes the wave about a thousand instructions
+// whatever its size, and most splits are of few prims.  So the wave splits
+// nodes one by one only while they have more than kRow prims; the subtrees
+// under those, kept in order in frontier[], are then built four at a time, one
+// in each row of 16 lanes, a prim and a bin to a lane (bin counts up to 16).
+// Splits are given pairs as they come; their places in depth-first order are
+// left for k_small_emit.  1.31M prims, leaves of 4: 1330 us with one node at a
+// time, @@ us so.
+constexpr uint32_t kRow = 16;
+
+struct SmallShare {
+  uint32_t stack[kSmall + 2];      // nodes to do, packed by pack_task
+  uint32_t frontier[kSmall / 2];   // subtrees of at most kRow prims (and at least 2)
+  uint32_t before[kSmall / 2 + 1]; // splits in subtrees before
+  uint16_t at[kSmall / 2];         // splits above that come before the subtree's
+  uint16_t pair[kSmall];           // per pair: subtrees before it, or which split of which one
+};
+
+__device__ __forceinline__ uint32_t pack_task(uint32_t b, uint32_t e, uint32_t me) { return b | e << 9 | me << 18; }
+__device__ __forceinline__ void unpack_task(uint32_t t, uint32_t &b, uint32_t &e, uint32_t &me) {
+  b = t & 511u;
+  e = t >> 9 & 511u;
+  me = t >> 18;
+}
+
+// Scans and reductions within a row of 16 lanes.  OP: 0 min, 1 max, 2 add.
+template <int OP>
+__device__ __forceinline__ int32_t row_op(int32_t a, int32_t b) {
+  return OP == 0 ? min(a, b) : (OP == 1 ? max(a, b) : a + b);
+}
+template <int OP, int CTRL>
+__device__ __forceinline__ int32_t row_step(int32_t v) {
+  constexpr int32_t I = OP == 0 ? INT32_MAX : (OP == 1 ? INT32_MIN : 0);
+  return row_op<OP>(v, __builtin_amdgcn_update_dpp(I, v, CTRL, 0xF, 0xF, false));
+}
+// union of the lanes before (exclusive)
+template <int OP>
+__device__ __forceinline__ int32_t row_before(int32_t v) {
+  constexpr int32_t I = OP == 0 ? INT32_MAX : (OP == 1 ? INT32_MIN : 0);
+  v = __builtin_amdgcn_update_dpp(I, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  return row_step<OP, 0x118>(row_step<OP, 0x114>(row_step<OP, 0x112>(row_step<OP, 0x111>(v))));
+}
+// union of this lane and those after (row_shl)
+template <int OP>
+__device__ __forceinline__ int32_t row_from(int32_t v) {
+  return row_step<OP, 0x108>(row_step<OP, 0x104>(row_step<OP, 0x102>(row_step<OP, 0x101>(v))));
+}
+// of the whole row, in every lane (row_ror)
+template <int OP>
+__device__ __forceinline__ int32_t row_all(int32_t v) {
+  v = row_op<OP>(v, __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false));
+  v = row_op<OP>(v, __builtin_amdgcn_mov_dpp(v, 0x124, 0xF, 0xF, false));
+  v = row_op<OP>(v, __builtin_amdgcn_mov_dpp(v, 0x122, 0xF, 0xF, false));
+  return row_op<OP>(v, __builtin_amdgcn_mov_dpp(v, 0x121, 0xF, 0xF, false));
+}
+
+// Places of a small segment's pairs: its part of the item buffer that it was
+// not left in.
+__device__ __forceinline__ uint16_t *pair_places(const Ctx &c, const SmallSeg &sg) {
+  return reinterpret_cast<uint16_t *>(c.items[sg.buf ^ 1] + sg.begin);
+}
+
+// The subtrees of frontier[0 .. numSub), a row of lanes each, and the places
+// of the segment's pairs.  numPairs: pairs of the splits above.  Returns the
+// number of the segment's pairs.  (Every lane stays in the loop: a row without a
+// subtree computes on identities.)
+__device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sBins, SmallShare &sh, uint32_t numSub,
+                               uint32_t numPairs, uint16_t *place) {
+  const uint32_t lane = lane_id(), r = lane & 15u, row0 = lane & 48u;
+  const uint64_t rowMask = 0xffffull << row0, rowsBefore = (1ull << row0) - 1;
+  const int nb = c.nb;
+  Node *loc = c.loc + 2 * (size_t)gb;
+  int32_t *bins = sBins + row0 * kBinWords;
+  uint32_t *stack = sh.stack + row0;  // right siblings: at most kRow - 1
+  const uint32_t above = numPairs;
+  uint32_t next = 0, sub = 0, splits = 0, sp = 0;
+  uint32_t b = 0, e = 0, me = 0;
+  bool on = false, idle = true;  // a node to do; a subtree wanted
+  while (true) {
+    const uint64_t want = __ballot(idle && r == 0);
+    if (idle) {
+      sub = next + (uint32_t)__popcll(want & rowsBefore);
+      on = sub < numSub;
+      if (on) unpack_task(sh.frontier[sub], b, e, me);
+      splits = 0;
+      idle = false;
+    }
+    next += (uint32_t)__popcll(want);
+    if (!__any(on)) break;
+    const uint32_t n = on ? e - b : 0u;
+    const bool in = r < n, inner = n > c.T;
+    Item v;
+    v.a = v.b = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (in) v = sIt[b + r];
+    const float ce[3] = {item_center(v, 0), item_center(v, 1), item_center(v, 2)};
+    const float vlo[3] = {v.a.x, v.a.y, v.a.z}, vhi[3] = {v.b.x, v.b.y, v.b.z};
+    float blo[3], bhi[3], clo[3], chi[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int32_t k = enc_cmp(ce[d]);
+      blo[d] = dec_f(row_all<0>(in ? enc_cmp(vlo[d]) : INT32_MAX));
+      bhi[d] = dec_f(row_all<1>(in ? enc_cmp(vhi[d]) : INT32_MIN));
+      clo[d] = dec_f(row_all<0>(in ? k : INT32_MAX));
+      chi[d] = dec_f(row_all<1>(in ? k : INT32_MIN));
+    }
+    // a lane per bin, one dimension after the other in the row's bins
+    float cost[3];
+    int myBin[3];
+    float leafCost = 0.f;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      int4 *w4 = reinterpret_cast<int4 *>(bins + r * kBinWords);
+      w4[0] = make_int4(bin_init(0), bin_init(1), bin_init(2), bin_init(3));
+      w4[1] = make_int4(bin_init(4), bin_init(5), 0, 0);
+      sync_wave_lds();
+      myBin[d] = sah_bin(ce[d], clo[d], chi[d], nb, c.binEps);
+      if (in && inner) {
+        int32_t *w = bins + myBin[d] * kBinWords;
+        for (int k = 0; k < 3; k++) {
+          atomicMin(&w[k], enc_f(vlo[k]));
+          atomicMax(&w[3 + k], enc_f(vhi[k]));
+        }
+        atomicAdd(&w[6], 1);
+      }
+      sync_wave_lds();
+      const int4 p = w4[0], q = w4[1];
+      sync_wave_lds();
+      const int32_t wlo[3] = {p.x, p.y, p.z}, whi[3] = {p.w, q.x, q.y};
+      float llo[3], lhi[3], rlo[3], rhi[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        llo[k] = dec_f(row_before<0>(wlo[k]));
+        lhi[k] = dec_f(row_before<1>(whi[k]));
+        rlo[k] = dec_f(row_from<0>(wlo[k]));
+        rhi[k] = dec_f(row_from<1>(whi[k]));
+      }
+      const uint32_t lCnt = (uint32_t)row_before<2>(q.z), rCnt = (uint32_t)row_from<2>(q.z);
+      const float rTerm = box_measure(rlo, rhi, c.elh != 0) * (float)rCnt;
+      const float s = box_measure(llo, lhi, c.elh != 0) * (float)lCnt + rTerm;
+      cost[d] = (lCnt > 0 && rCnt > 0 && s == s) ? s : INFINITY;
+      if (d == 0) leafCost = __shfl(rTerm, (int)row0, kWave);
+    }
+    // (as sah_decide_wave: the first minimum, the leaf first)
+    int mode = kModeLeaf, bin = 0;
+    auto pick = [&](float best, bool who) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const float m = __int_as_float(row_all<0>(__float_as_int(cost[d])));
+        const uint64_t at = __ballot(cost[d] == m) & rowMask;
+        if (who && m < best) {
+          best = m;
+          mode = d;
+          bin = (int)(__builtin_ctzll(at) - row0);
+        }
+      }
+    };
+    pick(leafCost < INFINITY ? leafCost : INFINITY, inner);
+    const bool over = inner && mode == kModeLeaf && n > c.cap;
+    if (__any(over)) {
+      pick(INFINITY, over);
+      if (over && mode == kModeLeaf) mode = kModeMiddle;
+    }
+    const bool split = on && mode != kModeLeaf;
+    if (on && !split && in) c.primIDs[gb + b + r] = item_id(v);
+    const int binAt = mode == 2 ? myBin[2] : (mode == 1 ? myBin[1] : myBin[0]);
+    const bool left = in && (mode == kModeMiddle ? r < n / 2 : binAt < bin);
+    const uint64_t mL = __ballot(left) & rowMask, mR = __ballot(in && !left) & rowMask;
+    const uint32_t nL = (uint32_t)__popcll(mL);
+    if (in && split) sIt[left ? b + mbcnt(mL) : e - 1 - mbcnt(mR)] = v;
+    const uint64_t ms = __ballot(split && r == 0);
+    const uint32_t pair = numPairs + (uint32_t)__popcll(ms & rowsBefore);
+    numPairs += (uint32_t)__popcll(ms);
+    if (on && r < 8) {
+      const uint64_t oc = split ? pack_oc(1 + 2 * pair, 0) : pack_oc(gb + b, n);
+      uint32_t w = __float_as_uint(blo[0]);
+      w = r == 1 ? __float_as_uint(blo[1]) : w;
+      w = r == 2 ? __float_as_uint(blo[2]) : w;
+      w = r == 3 ? __float_as_uint(bhi[0]) : w;
+      w = r == 4 ? __float_as_uint(bhi[1]) : w;
+      w = r == 5 ? __float_as_uint(bhi[2]) : w;
+      w = r == 6 ? (uint32_t)oc : w;
+      w = r == 7 ? (uint32_t)(oc >> 32) : w;
+      reinterpret_cast<uint32_t *>(loc + me)[r] = w;
+    }
+    if (split) {
+      if (r == 0) {
+        sh.pair[pair] = (uint16_t)(sub | splits << 8);
+        stack[sp] = pack_task(b + nL, e, 2 + 2 * pair);
+      }
+      sp++;
+      splits++;
+      e = b + nL;
+      me = 1 + 2 * pair;
+    }
+    sync_wave_lds();
+    if (on && !split) {
+      if (sp) {
+        unpack_task(stack[--sp], b, e, me);
+      } else {
+        on = false;
+        idle = true;
+        if (r == 0) sh.before[sub] = splits;
+      }
+    }
+  }
+  // splits of the subtrees before, two subtrees to a lane
+  sync_wave_lds();
+  const uint32_t s0 = 2 * lane < numSub ? sh.before[2 * lane] : 0u;
+  const uint32_t s1 = 2 * lane + 1 < numSub ? sh.before[2 * lane + 1] : 0u;
+  const uint32_t incl = (uint32_t)dpp_scan_i<2, true>((int32_t)(s0 + s1));
+  sync_wave_lds();
+  if (2 * lane < numSub) sh.before[2 * lane] = incl - s0 - s1;
+  if (2 * lane + 1 < numSub) sh.before[2 * lane + 1] = incl - s1;
+  if (lane == kWave - 1) sh.before[numSub] = incl;
+  sync_wave_lds();
+  for (uint32_t p = lane; p < numPairs; p += kWave) {
+    const uint32_t w = sh.pair[p], f = w & 255u;
+    place[p] = (uint16_t)(p < above ? p + sh.before[w] : sh.at[f] + sh.before[f] + (w >> 8));
+  }
+  return numPairs;
+}
+
 __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, Item *sIt,
-                              int32_t *sBins, uint32_t *sFr, uint32_t *sMe) {
+                              int32_t *sBins, SmallShare &sh) {
   const uint32_t lane = lane_id();
   const Item *gItems = c.items[sg.buf];
   const uint32_t gb = sg.begin;
@@ -770,15 +995,24 @@ __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx,
     return;
   }
   for (uint32_t i = lane; i < m; i += kWave) sIt[i] = gItems[gb + i];
+  const bool rows = nb <= (int)kRow;
+  uint32_t numSub = 0;
   int sp = 1;
-  if (lane == 0) { sFr[0] = m << 16; sMe[0] = 0; }
+  if (lane == 0) sh.stack[0] = pack_task(0u, m, 0u);
   sync_wave_lds();
   while (sp > 0) {
     --sp;
-    const uint32_t f = sFr[sp];
-    const uint32_t me = sMe[sp];
-    const uint32_t b = f & 0xffffu, e = f >> 16;
+    uint32_t b, e, me;
+    unpack_task((uint32_t)__builtin_amdgcn_readfirstlane((int)sh.stack[sp]), b, e, me);
     const uint32_t n = e - b;
+    if (rows && n <= kRow && n > c.T) {
+      if (lane == 0) {
+        sh.frontier[numSub] = pack_task(b, e, me);
+        sh.at[numSub] = (uint16_t)(nLocal / 2);
+      }
+      numSub++;
+      continue;
+    }
     // bounds on enc_cmp integers (fused integer DPP reductions)
     int32_t ble[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, bhe[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
     int32_t cle[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, che[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
@@ -846,31 +1080,35 @@ __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx,
     nLocal += 2;
     store_node_wave(loc + me, blo, bhi, pack_oc(child, 0));
     if (lane == 0) {
-      sFr[sp] = mid | (e << 16);
-      sMe[sp] = child + 1;
-      sFr[sp + 1] = b | (mid << 16);
-      sMe[sp + 1] = child;
+      sh.pair[child / 2] = (uint16_t)numSub;
+      sh.stack[sp] = pack_task(mid, e, child + 1);
+      sh.stack[sp + 1] = pack_task(b, mid, child);
     }
     sp += 2;
     sync_wave_lds();
   }
+  sync_wave_lds();
+  nLocal = 1 + 2 * small_rows(c, gb, sIt, sBins, sh, numSub, nLocal / 2, pair_places(c, sg));
   if (lane == 0) c.smallCount[segIdx] = nLocal;
 }
 
-// LDS (dynamic, sized by the bin count): items | bins | two stacks
+// LDS (dynamic, sized by the bin count): items | bins (of one node, or of one
+// dimension of four) | the rest
+__host__ __device__ constexpr int small_bin_words(int nb) {
+  return nb > (int)kRow ? 3 * nb * kBinWords : (3 * nb > 4 * (int)kRow ? 3 * nb : 4 * (int)kRow) * kBinWords;
+}
 __host__ __device__ constexpr size_t small_lds_bytes(int nb) {
-  return sizeof(Item) * kSmall + sizeof(int32_t) * 3 * (size_t)nb * kBinWords + 2 * sizeof(uint32_t) * (kSmall + 2);
+  return sizeof(Item) * kSmall + sizeof(int32_t) * small_bin_words(nb) + sizeof(SmallShare);
 }
 
 __global__ __launch_bounds__(kWave) void k_small(Ctx c) {
   extern __shared__ __align__(16) unsigned char smem[];
   Item *sIt = reinterpret_cast<Item *>(smem);
   int32_t *sBins = reinterpret_cast<int32_t *>(smem + sizeof(Item) * kSmall);
-  uint32_t *sFr = reinterpret_cast<uint32_t *>(sBins + 3 * c.nb * kBinWords);
-  uint32_t *sMe = sFr + (kSmall + 2);
+  SmallShare &sh = *reinterpret_cast<SmallShare *>(sBins + small_bin_words(c.nb));
   const uint32_t nSmall = c.ctr->numSmall;
   for (uint32_t w = blockIdx.x; w < nSmall; w += gridDim.x) {
-    small_segment(c, c.small[w], w, sIt, sBins, sFr, sMe);
+    small_segment(c, c.small[w], w, sIt, sBins, sh);
     sync_wave_lds();
   }
 }
@@ -887,7 +1125,8 @@ __global__ __launch_bounds__(kWave) void k_small_emit(Ctx c, Node *out) {
   const uint32_t nSmall = c.ctr->numSmall;
   for (uint32_t w = blockIdx.x; w < nSmall; w += gridDim.x) {
     const SmallSeg sg = c.small[w];
-    copy_local_nodes(c.loc + 2 * (size_t)sg.begin, c.smallCount[w], sg.node, c.smallBase[w], out);
+    copy_local_nodes(c.loc + 2 * (size_t)sg.begin, c.smallCount[w], sg.node, c.smallBase[w], out,
+                     pair_places(c, sg));
   }
 }
 
