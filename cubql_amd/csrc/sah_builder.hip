@@ -827,7 +827,7 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
   const uint32_t above = numPairs;
   uint32_t next = 0, sub = 0, splits = 0, sp = 0;
   uint32_t b = 0, e = 0, me = 0;
-  bool on = false, idle = true;  // a node to do; a subtree wanted
+  bool on = false, idle = true;  // a node to split; a subtree wanted
   while (true) {
     const uint64_t want = __ballot(idle && r == 0);
     if (idle) {
@@ -835,25 +835,47 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
       on = sub < numSub;
       if (on) unpack_task(sh.frontier[sub], b, e, me);
       splits = 0;
-      idle = false;
     }
     next += (uint32_t)__popcll(want);
     if (!__any(on)) break;
     const uint32_t n = on ? e - b : 0u;
-    const bool in = r < n, inner = n > c.T;
+    const bool in = r < n;
     Item v;
     v.a = v.b = make_float4(0.f, 0.f, 0.f, 0.f);
     if (in) v = sIt[b + r];
     const float ce[3] = {item_center(v, 0), item_center(v, 1), item_center(v, 2)};
     const float vlo[3] = {v.a.x, v.a.y, v.a.z}, vhi[3] = {v.b.x, v.b.y, v.b.z};
-    float blo[3], bhi[3], clo[3], chi[3];
+    float clo[3], chi[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const int32_t k = enc_cmp(ce[d]);
-      blo[d] = dec_f(row_all<0>(in ? enc_cmp(vlo[d]) : INT32_MAX));
-      bhi[d] = dec_f(row_all<1>(in ? enc_cmp(vhi[d]) : INT32_MIN));
       clo[d] = dec_f(row_all<0>(in ? k : INT32_MAX));
       chi[d] = dec_f(row_all<1>(in ? k : INT32_MIN));
+    }
+    // a word per lane of the node at `at`, and of the next one in lanes 8-15
+    auto store_nodes = [&](uint32_t at, uint32_t lanes, const float (&lo)[3], const float (&hi)[3],
+                           uint64_t oc) {
+      const uint32_t k = r & 7u;
+      uint32_t w = __float_as_uint(lo[0]);
+      w = k == 1 ? __float_as_uint(lo[1]) : w;
+      w = k == 2 ? __float_as_uint(lo[2]) : w;
+      w = k == 3 ? __float_as_uint(hi[0]) : w;
+      w = k == 4 ? __float_as_uint(hi[1]) : w;
+      w = k == 5 ? __float_as_uint(hi[2]) : w;
+      w = k == 6 ? (uint32_t)oc : w;
+      w = k == 7 ? (uint32_t)(oc >> 32) : w;
+      if (r < lanes) reinterpret_cast<uint32_t *>(loc + at)[r] = w;
+    };
+    if (want) {
+      // (a subtree's root: a leaf until it is split)
+      float lo[3], hi[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        lo[d] = dec_f(row_all<0>(in ? enc_cmp(vlo[d]) : INT32_MAX));
+        hi[d] = dec_f(row_all<1>(in ? enc_cmp(vhi[d]) : INT32_MIN));
+      }
+      store_nodes(me, idle && on ? 8u : 0u, lo, hi, pack_oc(gb + b, n));
+      idle = false;
     }
     // a lane per bin, one dimension after the other in the row's bins
     float cost[3];
@@ -866,7 +888,7 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
       w4[1] = make_int4(bin_init(4), bin_init(5), 0, 0);
       sync_wave_lds();
       myBin[d] = sah_bin(ce[d], clo[d], chi[d], nb, c.binEps);
-      if (in && inner) {
+      if (in) {
         int32_t *w = bins + myBin[d] * kBinWords;
         for (int k = 0; k < 3; k++) {
           atomicMin(&w[k], enc_f(vlo[k]));
@@ -906,46 +928,54 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
         }
       }
     };
-    pick(leafCost < INFINITY ? leafCost : INFINITY, inner);
-    const bool over = inner && mode == kModeLeaf && n > c.cap;
+    pick(leafCost < INFINITY ? leafCost : INFINITY, on);
+    const bool over = on && mode == kModeLeaf && n > c.cap;
     if (__any(over)) {
       pick(INFINITY, over);
       if (over && mode == kModeLeaf) mode = kModeMiddle;
     }
     const bool split = on && mode != kModeLeaf;
-    if (on && !split && in) c.primIDs[gb + b + r] = item_id(v);
     const int binAt = mode == 2 ? myBin[2] : (mode == 1 ? myBin[1] : myBin[0]);
-    const bool left = in && (mode == kModeMiddle ? r < n / 2 : binAt < bin);
-    const uint64_t mL = __ballot(left) & rowMask, mR = __ballot(in && !left) & rowMask;
-    const uint32_t nL = (uint32_t)__popcll(mL);
-    if (in && split) sIt[left ? b + mbcnt(mL) : e - 1 - mbcnt(mR)] = v;
+    const bool left = in && (mode == kModeMiddle ? r < n / 2 : binAt < bin), right = in && !left;
+    const uint64_t mL = __ballot(left) & rowMask, mR = __ballot(right) & rowMask;
+    const uint32_t nL = (uint32_t)__popcll(mL), nR = n - nL;
+    const uint32_t to = !split ? b + r : left ? b + mbcnt(mL) : e - 1 - mbcnt(mR);
+    if (in && split) sIt[to] = v;
+    if (in && (!split || (left ? nL : nR) <= c.T)) c.primIDs[gb + to] = item_id(v);
     const uint64_t ms = __ballot(split && r == 0);
     const uint32_t pair = numPairs + (uint32_t)__popcll(ms & rowsBefore);
     numPairs += (uint32_t)__popcll(ms);
-    if (on && r < 8) {
-      const uint64_t oc = split ? pack_oc(1 + 2 * pair, 0) : pack_oc(gb + b, n);
-      uint32_t w = __float_as_uint(blo[0]);
-      w = r == 1 ? __float_as_uint(blo[1]) : w;
-      w = r == 2 ? __float_as_uint(blo[2]) : w;
-      w = r == 3 ? __float_as_uint(bhi[0]) : w;
-      w = r == 4 ? __float_as_uint(bhi[1]) : w;
-      w = r == 5 ? __float_as_uint(bhi[2]) : w;
-      w = r == 6 ? (uint32_t)oc : w;
-      w = r == 7 ? (uint32_t)(oc >> 32) : w;
-      reinterpret_cast<uint32_t *>(loc + me)[r] = w;
+    // both children as leaves: lanes 0-7 the left one, 8-15 the right one
+    const bool second = r >= 8;
+    float lo[3], hi[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int32_t l = enc_cmp(vlo[d]), h = enc_cmp(vhi[d]);
+      const int32_t ll = row_all<0>(left ? l : INT32_MAX), lh = row_all<1>(left ? h : INT32_MIN);
+      const int32_t rl = row_all<0>(right ? l : INT32_MAX), rh = row_all<1>(right ? h : INT32_MIN);
+      lo[d] = dec_f(second ? rl : ll);
+      hi[d] = dec_f(second ? rh : lh);
     }
+    store_nodes(1 + 2 * pair, split ? 16u : 0u, lo, hi,
+                second ? pack_oc(gb + b + nL, nR) : pack_oc(gb + b, nL));
+    bool more = false;
     if (split) {
+      const uint32_t mid = b + nL, child = 1 + 2 * pair;
       if (r == 0) {
+        loc[me].oc = pack_oc(child, 0);
         sh.pair[pair] = (uint16_t)(sub | splits << 8);
-        stack[sp] = pack_task(b + nL, e, 2 + 2 * pair);
+        if (nR > c.T) stack[sp] = pack_task(mid, e, child + 1);
       }
-      sp++;
       splits++;
-      e = b + nL;
-      me = 1 + 2 * pair;
+      if (nR > c.T) sp++;
+      if (nL > c.T) {
+        e = mid;
+        me = child;
+        more = true;
+      }
     }
     sync_wave_lds();
-    if (on && !split) {
+    if (on && !more) {
       if (sp) {
         unpack_task(stack[--sp], b, e, me);
       } else {
@@ -955,8 +985,8 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
       }
     }
   }
-  // splits of the subtrees before, two subtrees to a lane
   sync_wave_lds();
+  // splits of the subtrees before, two subtrees to a lane
   const uint32_t s0 = 2 * lane < numSub ? sh.before[2 * lane] : 0u;
   const uint32_t s1 = 2 * lane + 1 < numSub ? sh.before[2 * lane + 1] : 0u;
   const uint32_t incl = (uint32_t)dpp_scan_i<2, true>((int32_t)(s0 + s1));
