@@ -21,7 +21,7 @@
 //     write one partial per tile (no global atomics); one workgroup per node
 //     reduces the partials and one wave evaluates all 3 x numBins candidate
 //     planes at once (prefix/suffix unions as wave scans); the partition is
-//     a single-pass decoupled look-back over 2048-prim tiles;
+//     a single-pass decoupled look-back over 1024-prim tiles;
 //   * nodes of <= 256 prims are finished by one wave each in LDS, which also
 //     computes their boxes, so no refit pass is needed;
 //   * the level loop runs on the device; the host checks for completion every
@@ -39,9 +39,11 @@ namespace cubql {
 namespace sah {
 
 constexpr int kBlock = 256;
-constexpr int kItems = 8;
-constexpr int kTile = kBlock * kItems;  // partition tile: 2048 prims
-constexpr int kBinTile = 4 * kTile;     // binning tile: 8192 prims
+// (8 items hold 198 registers, and the partition's workgroups of a level no
+// longer run at once: 1.31M prims 2.12 ms, 2.07 with 4, 2.09 with 2)
+constexpr int kItems = 4;
+constexpr int kTile = kBlock * kItems;  // partition tile: 1024 prims
+constexpr int kBinTile = 8 * kTile;     // binning tile: 8192 prims
 constexpr int kSmall = 256;             // max prims of a wave-finished node
 constexpr int kMaxBins = 64;            // one lane per bin
 constexpr int kBinWords = 8;            // lo xyz, hi xyz (encoded), count, pad
@@ -271,7 +273,9 @@ __device__ int sah_decide_wave(const int32_t *bins, int nb, uint32_t n, uint32_t
   auto pick = [&](float thr, int &bin) -> int {
     float best = thr;
     int dim = kModeLeaf;
-    for (int p = 0; p < nSets; p++) {
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      if (p >= nSets) break;
       // (costs are +0 .. +inf: their bit patterns order like the values)
       const float m = __int_as_float(wave_min_i32(__float_as_int(cost[p])));
       if (m < best) {
