@@ -1806,6 +1806,264 @@ __global__ __launch_bounds__(kWave) void k_small(Ctx c, int pp) {
   }
 }
 
+// The same trees by a workgroup per segment, for builds with too few segments
+// to fill the chip, where one wave's chain of pieces is the time.  All items
+// are in LDS; the nodes of more than 64 prims are split level by level, a wave
+// each, from one buffer into the other, and then the waves take the pieces of
+// up to 64.  Nothing is numbered on the way: the children of a node of range
+// [b, e) split at `mid` are the pair at loc[2 mid], and a piece keeps its own
+// pairs at loc[2 (b + 1)] and after, which no other node uses.  place[] then
+// gives each pair its number in the order in which one wave would have made it
+// (0xffff: none), for k_wide_emit.  3001 points: 96 us by waves, 30 us so.
+constexpr int kWideBlock = 512;
+// (uniform points, by waves and by workgroups: 1000 203 and 131 us a build, 100K
+// 333 and 262, 700K 418 and 385, 1.5M 515 and 525, 10M 1575 and 1983; boxes of a
+// mesh: 100K 578 and 451, 2M 923 and 912)
+constexpr uint32_t kWideMax = 1u << 20;
+constexpr uint16_t kNoPair = 0xffff;
+
+struct WideShare {
+  float4 it[2][kMedium];
+  uint32_t open[2][16], numOpen[2], numUnits;  // (nodes of more than 64 prims: at most 15 a level)
+  uint32_t unit[kMedium];    // pieces: b, e, buffer
+  uint16_t unitMe[kMedium];  //   and node
+  uint16_t kid[2 * kMedium]; // per node: where it is split, 0 if it is a piece
+  uint16_t pairs[kMedium];   // per piece, by its begin: its pairs, and the
+  uint16_t base[kMedium];    //   number of its first one
+};
+static_assert(kMedium <= 1024 && kMedium / 65 < 16, "wide small-phase packing");
+__device__ __forceinline__ uint32_t wide_pack(uint32_t b, uint32_t e, uint32_t me) { return b | e << 10 | me << 21; }
+
+__device__ __forceinline__ uint16_t *pair_places(const Ctx &c, const SmallSeg &sg) {
+  // (where its items were, which are in LDS by then)
+  return reinterpret_cast<uint16_t *>(c.items[sg.buf] + sg.pbeg);
+}
+
+// splits the node `me` of range [b, e), which is in it[cur], into it[cur ^ 1]
+template <bool PTS>
+__device__ void wide_split(const Ctx &c, WideShare &sh, uint32_t cur, uint32_t gb, uint32_t b, uint32_t e,
+                           uint32_t me) {
+  const uint32_t lane = lane_id();
+  const float4 *src = sh.it[cur];
+  float4 *dst = sh.it[cur ^ 1u];
+  int32_t cb[6], bb[6];
+  bounds_init(cb);
+  bounds_init(bb);
+#pragma unroll 4
+  for (uint32_t i = b + lane; i < e; i += kWave) {
+    const float4 v = src[i];
+    const int32_t ex = enc_cmp(v.x), ey = enc_cmp(v.y), ez = enc_cmp(v.z);
+    bounds_add(cb, ex, ey, ez, ex, ey, ez);
+    if (!PTS) {
+      const cubql_box3f bx = load_box(c.boxes, __float_as_uint(v.w));
+      bounds_add(bb, enc_cmp(bx.lower[0]), enc_cmp(bx.lower[1]), enc_cmp(bx.lower[2]), enc_cmp(bx.upper[0]),
+                 enc_cmp(bx.upper[1]), enc_cmp(bx.upper[2]));
+    }
+  }
+  bounds_wave(cb);
+  if (!PTS) bounds_wave(bb);
+  float clo[3], chi[3], lo[3], hi[3];
+  for (int d = 0; d < 3; d++) {
+    clo[d] = dec_f(cb[d]); chi[d] = dec_f(cb[d + 3]);
+    lo[d] = PTS ? clo[d] : dec_f(bb[d]);
+    hi[d] = PTS ? chi[d] : dec_f(bb[d + 3]);
+  }
+  int dim;
+  float pos;
+  choose_split(clo, chi, dim, pos);
+  uint32_t nL = 0, nR = 0;
+  for (uint32_t i0 = b; i0 < e; i0 += kWave) {
+    const uint32_t i = i0 + lane;
+    const bool act = i < e;
+    const float4 v = src[act ? i : b];
+    const bool isL = act && coord(v, dim) < pos;
+    const uint64_t mL = __ballot(isL), mR = __ballot(act && !isL);
+    if (act) dst[isL ? b + nL + mbcnt(mL) : e - 1 - (nR + mbcnt(mR))] = v;
+    nL += (uint32_t)__popcll(mL);
+    nR += (uint32_t)__popcll(mR);
+  }
+  // (one-sided: the middle of the global range, spatialMedian.h:107)
+  const uint32_t mid = nL != 0 && nR != 0 ? b + nL : (b + e) >> 1;
+  store_node_wave(c.loc + 2 * (size_t)gb + me, lo, hi, pack_oc(2 * mid, 0));
+  if (lane < 2) {
+    const uint32_t cb0 = lane ? mid : b, ce0 = lane ? e : mid, child = 2 * mid + lane;
+    if (ce0 - cb0 > (uint32_t)kWave && ce0 - cb0 > c.T) {
+      sh.open[cur ^ 1u][atomicAdd(&sh.numOpen[cur ^ 1u], 1u)] = wide_pack(cb0, ce0, child);
+    } else {
+      const uint32_t u = atomicAdd(&sh.numUnits, 1u);
+      sh.unit[u] = cb0 | ce0 << 10 | (cur ^ 1u) << 21;
+      sh.unitMe[u] = (uint16_t)child;
+      sh.kid[child] = 0;
+    }
+  }
+  if (lane == 0) sh.kid[me] = (uint16_t)mid;
+}
+
+// Numbers of the pairs, by one thread, in the order of small_segment and
+// small_sub: a node's own, its pieces of up to kSmall prims depth first, left
+// first, and then the last of the larger ones.  Returns the number of pairs.
+__device__ uint32_t wide_number(WideShare &sh, uint32_t m, uint32_t T, uint16_t *place) {
+  uint32_t *stack = reinterpret_cast<uint32_t *>(sh.it[0]);  // (the items are done with)
+  uint32_t *bigs = stack + kMedium + 2;
+  uint32_t r = 0, numBig = 0;
+  auto sub = [&](uint32_t b0, uint32_t e0, uint32_t me0) {
+    uint32_t sp = 0, b = b0, e = e0, me = me0;
+    while (true) {
+      const uint32_t q = sh.kid[me];
+      if (q) {
+        place[q] = (uint16_t)r++;
+        stack[sp++] = wide_pack(q, e, 2 * q + 1);
+        e = q;
+        me = 2 * q;
+        continue;
+      }
+      sh.base[b] = (uint16_t)r;
+      r += sh.pairs[b];
+      if (!sp) break;
+      const uint32_t f = stack[--sp];
+      b = f & 1023u;
+      e = f >> 10 & 2047u;
+      me = f >> 21;
+    }
+  };
+  if (m <= (uint32_t)kSmall || m <= T) {
+    sub(0u, m, 0u);
+    return r;
+  }
+  bigs[numBig++] = wide_pack(0u, m, 0u);
+  while (numBig) {
+    const uint32_t f = bigs[--numBig], b = f & 1023u, e = f >> 10 & 2047u, q = sh.kid[f >> 21];
+    place[q] = (uint16_t)r++;
+    for (uint32_t side = 0; side < 2; side++) {
+      const uint32_t cb = side ? q : b, ce = side ? e : q;
+      if (ce - cb <= (uint32_t)kSmall || ce - cb <= T) sub(cb, ce, 2 * q + side);
+      else bigs[numBig++] = wide_pack(cb, ce, 2 * q + side);
+    }
+  }
+  return r;
+}
+
+template <bool PTS>
+__device__ void wide_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, WideShare &sh) {
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  const uint32_t gb = sg.begin, m = sg.end - sg.begin;
+  const float4 *items = c.items[sg.buf] + sg.pbeg;
+  Node *loc = c.loc + 2 * (size_t)gb;
+  if (m > (uint32_t)kWave && m <= c.T) {
+    // a leaf
+    if (wave == 0) {
+      uint32_t nLocal = 1;
+      small_sub<PTS>(c, items, sg.rev != 0, gb, m, 0u, nLocal, loc, sh.it[0], sh.unit);
+      if (lane == 0) c.smallCount[segIdx] = 1;
+    }
+    return;
+  }
+  for (uint32_t i = tid; i < m; i += kWideBlock) sh.it[0][i] = items[sg.rev ? m - 1 - i : i];
+  if (tid == 0) {
+    const bool split = m > (uint32_t)kWave;
+    sh.open[0][0] = wide_pack(0u, m, 0u);
+    sh.numOpen[0] = split ? 1u : 0u;
+    sh.numOpen[1] = 0u;
+    sh.numUnits = split ? 0u : 1u;
+    sh.unit[0] = m << 10;
+    sh.unitMe[0] = 0;
+    sh.kid[0] = 0;
+  }
+  __syncthreads();
+  for (uint32_t cur = 0;; cur ^= 1u) {
+    const uint32_t n = sh.numOpen[cur];
+    if (!n) break;
+    for (uint32_t t = wave; t < n; t += kWideBlock / kWave) {
+      const uint32_t f = sh.open[cur][t];
+      wide_split<PTS>(c, sh, cur, gb, f & 1023u, f >> 10 & 2047u, f >> 21);
+    }
+    __syncthreads();
+    if (tid == 0) sh.numOpen[cur] = 0u;
+    __syncthreads();
+  }
+  const uint32_t numUnits = sh.numUnits;
+  for (uint32_t u = wave; u < numUnits; u += kWideBlock / kWave) {
+    const uint32_t f = sh.unit[u], b = f & 1023u, e = f >> 10 & 2047u, n = e - b;
+    const float4 *src = sh.it[f >> 21] + b;
+    uint32_t nLocal = 2 * (b + 1);
+    if (n <= (uint32_t)kWave) {
+      const float4 v = lane < n ? src[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+      cubql_box3f bx{};
+      if (!PTS && lane < n) bx = load_box(c.boxes, __float_as_uint(v.w));
+      reg_subtree<PTS>(c, gb + b, n, v.x, v.y, v.z, __float_as_uint(v.w), bx.lower[0], bx.lower[1], bx.lower[2],
+                       bx.upper[0], bx.upper[1], bx.upper[2], sh.unitMe[u], nLocal, loc);
+    } else {
+      // a leaf of more prims
+      int32_t bb[6];
+      bounds_init(bb);
+      for (uint32_t i = lane; i < n; i += kWave) {
+        const float4 v = src[i];
+        c.primIDs[gb + b + i] = __float_as_uint(v.w);
+        cubql_box3f bx;
+        if (PTS) {
+          bx.lower[0] = bx.upper[0] = v.x; bx.lower[1] = bx.upper[1] = v.y; bx.lower[2] = bx.upper[2] = v.z;
+        } else {
+          bx = load_box(c.boxes, __float_as_uint(v.w));
+        }
+        bounds_add(bb, enc_cmp(bx.lower[0]), enc_cmp(bx.lower[1]), enc_cmp(bx.lower[2]), enc_cmp(bx.upper[0]),
+                   enc_cmp(bx.upper[1]), enc_cmp(bx.upper[2]));
+      }
+      bounds_wave(bb);
+      const float lo[3] = {dec_f(bb[0]), dec_f(bb[1]), dec_f(bb[2])}, hi[3] = {dec_f(bb[3]), dec_f(bb[4]), dec_f(bb[5])};
+      store_node_wave(loc + sh.unitMe[u], lo, hi, pack_oc(gb + b, n));
+    }
+    if (lane == 0) sh.pairs[b] = (uint16_t)((nLocal - 2 * (b + 1)) / 2);
+  }
+  __syncthreads();
+  uint16_t *place = pair_places(c, sg);
+  if (tid == 0) c.smallCount[segIdx] = 1 + 2 * wide_number(sh, m, c.T, place);
+  __syncthreads();
+  for (uint32_t u = wave; u < numUnits; u += kWideBlock / kWave) {
+    const uint32_t f = sh.unit[u], b = f & 1023u, n = (f >> 10 & 2047u) - b;
+    for (uint32_t j = lane; j + 1 < n; j += kWave)
+      place[b + 1 + j] = j < sh.pairs[b] ? (uint16_t)(sh.base[b] + j) : kNoPair;
+  }
+}
+
+__global__ __launch_bounds__(kWideBlock) void k_wide(Ctx c, int pp) {
+  __shared__ WideShare sh;
+  if (c.ctr->numLarge[pp] != 0 || c.ctr->spinFault != 0) return;
+  const bool pts = c.ctr->allPoints != 0;
+  const uint32_t nSmall = c.ctr->numSmall;
+  for (uint32_t w = blockIdx.x; w < nSmall; w += gridDim.x) {
+    const SmallSeg sg = c.small[w];
+    if (pts) wide_segment<true>(c, sg, w, sh);
+    else wide_segment<false>(c, sg, w, sh);
+    __syncthreads();
+  }
+}
+
+// (a workgroup per segment)
+__global__ __launch_bounds__(256) void k_wide_emit(Ctx c, Node *out) {
+  const uint32_t nSmall = c.ctr->numSmall;
+  for (uint32_t w = blockIdx.x; w < nSmall; w += gridDim.x) {
+    const SmallSeg sg = c.small[w];
+    const uint4 *src = reinterpret_cast<const uint4 *>(c.loc + 2 * (size_t)sg.begin);
+    const uint16_t *place = pair_places(c, sg);
+    const uint32_t base = c.smallBase[w], n = c.smallCount[w] == 1 ? 1u : 2 * (sg.end - sg.begin);
+    for (uint32_t j = threadIdx.x; j < n; j += 256) {
+      const uint32_t at = j < 2 ? (uint32_t)kNoPair : place[j / 2];
+      if (j != 0 && at == kNoPair) continue;
+      const uint4 a = src[2 * j];
+      uint4 b = src[2 * j + 1];
+      const uint64_t oc = ((uint64_t)b.w << 32) | b.z;
+      if (oc_count(oc) == 0) {
+        const uint64_t g = pack_oc(base + 2 * (uint32_t)place[oc_offset(oc) / 2], 0);
+        b.z = (uint32_t)g;
+        b.w = (uint32_t)(g >> 32);
+      }
+      uint4 *d = reinterpret_cast<uint4 *>(out + (j == 0 ? sg.node : base + 2 * at + (j & 1u)));
+      d[0] = a;
+      d[1] = b;
+    }
+  }
+}
+
 // Exclusive scan of (count-1) over small segments: global id of local node
 // j >= 1 of segment s is smallBase[s] + j - 1.
 // global ids of the small segments' local nodes (the final node count goes
@@ -1954,6 +2212,7 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
   // -> 241 us a build, 800, which take no pass, 223 -> 173, against four passes
   // always).
   int batch = levels ? std::max(std::min(kPassesPerSync, (levels + 1) / 2 + 1), (levels + 1) / 2) : 0;
+  const bool wide = n <= kWideMax;
   bool firstBatch = true;
   int specPass = -1, smallSlot = -1;
   uint32_t specGrid = 0;
@@ -1983,7 +2242,8 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
       }
       specGrid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(bound, (uint64_t)n + 1));
       smallSlot = prof_begin(s);
-      k_small<<<specGrid, kWave, 0, s>>>(c, pass & 1);
+      if (wide) k_wide<<<specGrid, kWideBlock, 0, s>>>(c, pass & 1);
+      else k_small<<<specGrid, kWave, 0, s>>>(c, pass & 1);
       prof_end(smallSlot, s, "sm_small");
       // (status tag beyond every pass's)
       k_small_scan<<<div_up(specGrid, kCountScanTile), 1024, 0, s>>>(c, maxPasses + 2, pass & 1);
@@ -2013,7 +2273,8 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
     // workgroup per segment (the dispatcher balances the uneven segment
     // costs far better than a fixed round-robin over resident waves)
     smallSlot = prof_begin(s);
-    k_small<<<std::max<uint32_t>(1u, numSmall), kWave, 0, s>>>(c, pass & 1);
+    if (wide) k_wide<<<std::max<uint32_t>(1u, numSmall), kWideBlock, 0, s>>>(c, pass & 1);
+    else k_small<<<std::max<uint32_t>(1u, numSmall), kWave, 0, s>>>(c, pass & 1);
     prof_end(smallSlot, s, "sm_small");
     k_small_scan<<<std::max<uint32_t>(1u, div_up(numSmall, kCountScanTile)), 1024, 0, s>>>(c, maxPasses + 2, pass & 1);
     if (hipGetLastError() != hipSuccess) return fail((set_error("small-phase launch failed"), CUBQL_ERR_HIP));
@@ -2046,7 +2307,8 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
   if (numNodes) {
     k_copy_top<<<std::max<uint32_t>(1u, std::min<uint32_t>(div_up(topCount, 256), 1024)), 256, 0, s>>>(
         c.nodes, nodes, topCount);
-    if (numSmall) k_small_emit<<<div_up(numSmall, 4), 256, 0, s>>>(c, nodes);
+    if (numSmall && wide) k_wide_emit<<<numSmall, 256, 0, s>>>(c, nodes);
+    else if (numSmall) k_small_emit<<<div_up(numSmall, 4), 256, 0, s>>>(c, nodes);
     // (point input: the emit already wrote the pass-phase boxes; two node
     // lists a pass, each refit after the deeper ones)
     if (numTop && !hc0.allPoints)
