@@ -31,6 +31,26 @@ __device__ inline void choose_split(const float lo[3], const float hi[3], int &d
   pos = (l + h) / 2.f;
 }
 
+// The 24 bytes of a node's box as three 8-byte words (a node is 16-byte
+// aligned), stored and loaded at agent scope.
+__device__ __forceinline__ void store_box_agent(Node *nd, const float (&lo)[3], const float (&hi)[3]) {
+  uint64_t *w = reinterpret_cast<uint64_t *>(nd);
+  const float v[6] = {lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]};
+#pragma unroll
+  for (int j = 0; j < 3; j++)
+    __hip_atomic_store(w + j, (uint64_t)__float_as_uint(v[2 * j]) | ((uint64_t)__float_as_uint(v[2 * j + 1]) << 32),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_box_agent(const Node *nd, float (&lo)[3], float (&hi)[3]) {
+  const uint64_t *w = reinterpret_cast<const uint64_t *>(nd);
+  uint64_t v[3];
+#pragma unroll
+  for (int j = 0; j < 3; j++) v[j] = __hip_atomic_load(w + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  lo[0] = __uint_as_float((uint32_t)v[0]); lo[1] = __uint_as_float((uint32_t)(v[0] >> 32));
+  lo[2] = __uint_as_float((uint32_t)v[1]); hi[0] = __uint_as_float((uint32_t)(v[1] >> 32));
+  hi[1] = __uint_as_float((uint32_t)v[2]); hi[2] = __uint_as_float((uint32_t)(v[2] >> 32));
+}
+
 // One wave copies a finished small segment's cnt local nodes to the final
 // array: local node 0 to `root`, local node j >= 1 to base + j - 1, with an
 // inner node's child offset (a local id) rebased the same way.  With place,

@@ -308,11 +308,8 @@ static void refit_launch(const RCtx &c, Node *nodes, const uint32_t *primIDs, in
 // Numbering: node 0 is the root and node 1 unused (radix.h:585-586); the
 // children of the s-th split node (in position order) are nodes 2 + 2s and
 // 3 + 2s; the pairs of the middle-split subtrees follow all of those, each
-// subtree's in level order.  Boxes are refitted bottom up in buckets: the
-// inner nodes of middle-split subtrees first, deepest first, then the split
-// nodes in decreasing order of the common key-prefix length of their range,
-// which grows strictly from a node to its split children, so every child
-// is final before its parent.
+// subtree's in level order.  Leaves get their boxes when they are written, and
+// k_karras_climb fits the inner nodes above them.
 
 // Readers of the sorted keys for the radix-tree search: from the
 // workgroup's LDS copy of positions [lo, hi) (a read outside sets `miss`
@@ -378,24 +375,17 @@ __device__ __forceinline__ void karras_node(R &rd, I n, I i, uint32_t &first, ui
   last = (uint32_t)(i < j ? j : i);
 }
 
-template <typename K>
-__device__ __forceinline__ int key_prefix(K a, K b) {
-  return sizeof(K) == 8 ? __clzll((unsigned long long)(a ^ b)) : __clz((uint32_t)(a ^ b));
-}
-
 // Shape of the middle-split subtree of m prims with leaves <= T (each inner
 // node of s prims has children of floor(s/2) and ceil(s/2)): the sizes at
 // depth d are q = m >> d or q + 1 (m mod 2^d of them), so every node above
 // depth D = min{d : q_d <= T} is inner, at depth D exactly the nodes of
 // T + 1 prims are (when q_D == T), and deeper nodes are leaves.
 struct MidShape {
-  uint32_t D, q, r, T;  // depth D, q_D, m mod 2^D, the leaf threshold
-  // inner nodes at depth t
-  __host__ __device__ uint32_t at(uint32_t t) const { return t < D ? 1u << t : (t == D && q == T) ? r : 0u; }
+  uint32_t D, q, r;  // depth D, q_D, m mod 2^D
 };
 
 __host__ __device__ inline MidShape mid_shape(uint32_t m, uint32_t T) {
-  MidShape ms{0u, m, 0u, T};
+  MidShape ms{0u, m, 0u};
   while (ms.q > T) ms.q = m >> ++ms.D;
   ms.r = ms.D ? m & ((1u << ms.D) - 1u) : 0u;
   return ms;
@@ -407,14 +397,8 @@ __host__ __device__ inline uint32_t mid_inner(uint32_t m, uint32_t T) {
   return (ms.D ? (1u << ms.D) - 1u : 0u) + (ms.q == T ? ms.r : 0u);
 }
 
-// Refit buckets: split nodes by the prefix length of their range (< key
-// bits), inner nodes of middle-split subtrees by key bits + 1 + depth; the
-// last bin counts the middle-split subtree roots.
-constexpr int kDeltaBins = 128;
-constexpr int kBinEqRoots = kDeltaBins - 1;
 // radix-tree nodes per workgroup of the hierarchy kernels (kKThreads
-// threads, kKPer nodes each, strided); bucket slots are assigned per such
-// block
+// threads, kKPer nodes each, strided)
 constexpr int kKThreads = 1024;
 constexpr int kKPer = 2;
 constexpr uint32_t kKBlock = kKThreads * kKPer;
@@ -456,35 +440,28 @@ __device__ __forceinline__ void range_box(const cubql_box3f *boxes, const uint32
 }
 
 // The per-node outputs of the radix-tree pass: the node record, whether it
-// is a split node (more than T prims, two different keys), the inner nodes
-// of the middle-split subtrees under it, and its refit-bucket counts
-// (add(bin, count): into LDS in the block kernel, into the block's row in
-// global memory for the deferred nodes).
-template <typename K, typename Add>
-__device__ __forceinline__ void karras_emit_counts(const K *keys, uint32_t T, uint32_t i, uint32_t first,
-                                                   uint32_t last, uint32_t g, int dn, KNode *kn,
-                                                   uint32_t *splitFlag, uint32_t *eqPairs, Add &&add) {
-  constexpr int kBits = 8 * (int)sizeof(K);
+// is a split node (more than T prims, two different keys), and the inner nodes
+// of the middle-split subtrees under it.  Returns the number of those subtrees.
+template <typename K>
+__device__ __forceinline__ uint32_t karras_emit_counts(const K *keys, uint32_t T, uint32_t i, uint32_t first,
+                                                       uint32_t last, uint32_t g, KNode *kn, uint32_t *splitFlag,
+                                                       uint32_t *eqPairs) {
   kn[i] = KNode{first, last, g, 0u};
   const bool split = last - first + 1 > T && keys[first] != keys[last];
   splitFlag[i] = split ? 1u : 0u;
-  uint32_t eq = 0;
+  uint32_t eq = 0, roots = 0;
   if (split) {
-    // (split nodes: the keys of the range differ, so dn < key bits)
-    add(dn, 1u);
     const uint32_t cb[2] = {first, g + 1}, ce[2] = {g, last};
     for (int side = 0; side < 2; side++) {
       const uint32_t m = ce[side] - cb[side] + 1;
       if (m > T && keys[cb[side]] == keys[ce[side]]) {
-        const MidShape ms = mid_shape(m, T);
-        for (uint32_t t = 0; t <= ms.D; t++)
-          if (const uint32_t c = ms.at(t)) add(kBits + 1 + (int)t, c);
         eq += mid_inner(m, T);
-        add(kBinEqRoots, 1u);
+        roots++;
       }
     }
   }
   eqPairs[i] = eq;
+  return roots;
 }
 
 // keys a workgroup of k_karras stages in LDS: its nodes and kKWin on each
@@ -494,16 +471,16 @@ constexpr int kKWin = 1024;
 
 template <typename K>
 __global__ __launch_bounds__(kKThreads) void k_karras(const K *keys, const uint32_t *nPtr, uint32_t T, KNode *kn,
-                                                   uint32_t *splitFlag, uint32_t *eqPairs, uint32_t *blockHist,
-                                                   uint32_t numKBlocks, uint32_t *farList, uint32_t *farCount) {
-  __shared__ uint32_t sh[kDeltaBins];
+                                                   uint32_t *splitFlag, uint32_t *eqPairs, uint32_t *numEqRoots,
+                                                   uint32_t *farList, uint32_t *farCount) {
+  __shared__ uint32_t sRoots;
   __shared__ K sKeys[kKBlock + 2 * kKWin];
   const uint32_t n = *nPtr;
   const int64_t N = n;
   const int64_t b0 = (int64_t)blockIdx.x * kKBlock;
   const int64_t wlo = b0 - kKWin < 0 ? 0 : b0 - kKWin;
   const int64_t whi = b0 + kKBlock + kKWin > N ? N : b0 + kKBlock + kKWin;
-  for (int b = threadIdx.x; b < kDeltaBins; b += kKThreads) sh[b] = 0;
+  if (threadIdx.x == 0) sRoots = 0;
   for (int64_t j = wlo + threadIdx.x; j < whi; j += kKThreads) sKeys[j - wlo] = keys[j];
   __syncthreads();
   for (int r = 0; r < kKPer; r++) {
@@ -527,11 +504,11 @@ __global__ __launch_bounds__(kKThreads) void k_karras(const K *keys, const uint3
       if (lk.miss) farList[base + (uint32_t)__popcll(far & ((1ull << lane_id()) - 1ull))] = (uint32_t)i;
     }
     if (lk.miss) continue;
-    karras_emit_counts<K>(keys, T, (uint32_t)i, first, last, g, dn, kn, splitFlag, eqPairs,
-                          [&](int bin, uint32_t c) { atomicAdd(&sh[bin], c); });
+    const uint32_t roots = karras_emit_counts<K>(keys, T, (uint32_t)i, first, last, g, kn, splitFlag, eqPairs);
+    if (roots) atomicAdd(&sRoots, roots);
   }
   __syncthreads();
-  for (int b = threadIdx.x; b < kDeltaBins; b += kKThreads) blockHist[(size_t)b * numKBlocks + blockIdx.x] = sh[b];
+  if (threadIdx.x == 0 && sRoots) atomicAdd(numEqRoots, sRoots);
 }
 
 // Largest t in [0, tmax] with delta(i, i + t d) > thr, for one wave (all
@@ -564,8 +541,7 @@ __device__ __forceinline__ int64_t wave_last_true(const K *keys, int64_t n, int6
 template <typename K>
 __global__ __launch_bounds__(256) void k_karras_far(const K *keys, const uint32_t *nPtr, uint32_t T,
                                                     const uint32_t *farList, const uint32_t *farCount, KNode *kn,
-                                                    uint32_t *splitFlag, uint32_t *eqPairs, uint32_t *blockHist,
-                                                    uint32_t numKBlocks) {
+                                                    uint32_t *splitFlag, uint32_t *eqPairs, uint32_t *numEqRoots) {
   const int64_t N = *nPtr;
   const uint32_t cnt = *farCount;
   const uint32_t nw = gridDim.x * (256 / kWave);
@@ -582,29 +558,10 @@ __global__ __launch_bounds__(256) void k_karras_far(const K *keys, const uint32_
     const uint32_t g = (uint32_t)(i + sp * d + (d < 0 ? -1 : 0));
     const uint32_t first = (uint32_t)(i < j ? i : j), last = (uint32_t)(i < j ? j : i);
     if (lane_id() == 0) {
-      uint32_t *row = blockHist + (size_t)(i / kKBlock);
-      karras_emit_counts<K>(keys, T, (uint32_t)i, first, last, g, dn, kn, splitFlag, eqPairs,
-                            [&](int bin, uint32_t c) { atomicAdd(&row[(size_t)bin * numKBlocks], c); });
+      const uint32_t roots = karras_emit_counts<K>(keys, T, (uint32_t)i, first, last, g, kn, splitFlag, eqPairs);
+      if (roots) atomicAdd(numEqRoots, roots);
     }
   }
-}
-
-// One workgroup per bin: exclusive scan of the bin's row over the blocks
-// (in place), the bin's total to binTotal[bin].
-__global__ __launch_bounds__(1024) void k_karras_binscan(uint32_t *blockHist, uint32_t numKBlocks,
-                                                         uint32_t *binTotal) {
-  __shared__ uint32_t ss[1024 / kWave + 1];
-  uint32_t *row = blockHist + (size_t)blockIdx.x * numKBlocks;
-  uint32_t run = 0;
-  for (uint32_t b0 = 0; b0 < numKBlocks; b0 += 1024) {
-    const uint32_t k = b0 + threadIdx.x;
-    const uint32_t v = k < numKBlocks ? row[k] : 0u;
-    uint32_t tot;
-    const uint32_t ex = block_excl_scan<1024>(v, ss, &tot);
-    if (k < numKBlocks) row[k] = run + ex;
-    run += tot;
-  }
-  if (threadIdx.x == 0) binTotal[blockIdx.x] = run;
 }
 
 // Exclusive scans of two per-node counts over the n - 1 radix-tree nodes
@@ -695,17 +652,16 @@ __global__ void k_karras_root_eq(const uint32_t *nPtr, EqRoot *roots) { roots[0]
 
 // Children of every split node (one thread per split node, from the list
 // of split nodes): leaves with their boxes, split nodes (their position),
-// roots of middle-split subtrees (claimed with one atomic per wave).  Each
-// split node's refit bucket is its prefix length: dnKey[s] = dn, dnVal[s]
-// = s, sorted by key afterwards.
+// roots of middle-split subtrees (claimed with one atomic per wave).  up[s] is
+// the node whose children the pair s (nodes 2 + 2s and 3 + 2s) is; arrive[] is
+// cleared for k_karras_climb.
 template <typename K>
 __global__ __launch_bounds__(kBlock) void k_karras_emit(const K *keys, const cubql_box3f *boxes,
                                                         const uint32_t *primIDs, uint32_t T,
                                                         const KNode *kn, const uint32_t *splitList,
                                                         uint32_t numSplit, const uint32_t *slot,
                                                         const uint32_t *eqPairs, const uint32_t *eqBase,
-                                                        uint32_t *dnKey, uint32_t *dnVal, uint32_t *pos,
-                                                        Node *nodes, EqRoot *eqRoots, uint32_t *eqRootCursor) {
+                                                        uint32_t *up, uint32_t *arrive, Node *nodes, EqRoot *eqRoots, uint32_t *eqRootCursor) {
   const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
   const bool active = s < numSplit;
   uint32_t eqCount = 0;
@@ -720,10 +676,9 @@ __global__ __launch_bounds__(kBlock) void k_karras_emit(const K *keys, const cub
       for (int d = 0; d < 3; d++) { nd.lo[d] = INFINITY; nd.hi[d] = -INFINITY; }
       nd.oc = pack_oc(2, 0);
       nodes[0] = nd;
-      pos[0] = 0;
+      up[0] = 0;
     }
-    dnKey[s] = (uint32_t)key_prefix(keys[k.first], keys[k.last]);
-    dnVal[s] = s;
+    arrive[s] = 0;
     uint32_t eqPair = eqPairs[i] ? 2 + 2 * numSplit + 2 * eqBase[i] : 0u;
     const uint32_t cb[2] = {k.first, k.gamma + 1}, ce[2] = {k.gamma, k.last};
     for (int side = 0; side < 2; side++) {
@@ -745,7 +700,7 @@ __global__ __launch_bounds__(kBlock) void k_karras_emit(const K *keys, const cub
         for (int d = 0; d < 3; d++) { nd.lo[d] = INFINITY; nd.hi[d] = -INFINITY; }
         nd.oc = pack_oc(2 + 2 * cs, 0);
         nodes[base + side] = nd;
-        pos[cs] = base + side;
+        up[cs] = base + side;
       }
     }
   }
@@ -767,123 +722,151 @@ __global__ __launch_bounds__(kBlock) void k_karras_emit(const K *keys, const cub
 // node before k holds q or q + 1 prims).  Each inner node writes itself,
 // its leaf children with their boxes, and its position into its depth's
 // bucket (slots claimed by one atomic per wave and depth).
-__global__ __launch_bounds__(256) void k_karras_equal(const cubql_box3f *boxes, const uint32_t *primIDs, uint32_t T, const EqRoot *roots, uint32_t nr, int kBits,
-                                                      const uint32_t *bucketStart, uint32_t *bucketCursor,
-                                                      uint32_t *bucket, Node *nodes) {
-  const uint32_t lane = lane_id();
+__global__ __launch_bounds__(256) void k_karras_equal(const cubql_box3f *boxes, const uint32_t *primIDs, uint32_t T,
+                                                      const EqRoot *roots, uint32_t nr, uint32_t *up,
+                                                      uint32_t *arrive, Node *nodes) {
   for (uint32_t r = blockIdx.x; r < nr; r += gridDim.x) {
     const EqRoot er = roots[r];
     const MidShape ms = mid_shape(er.size, T);
     const uint32_t full = (1u << ms.D) - 1u;  // inner nodes above depth D
     const uint32_t items = full + (ms.q == T ? full + 1u : 0u);
     const uint32_t stride = gridDim.y * 256;
-    // every lane of a wave runs the same number of rounds (the wave-wide
-    // slot claim below needs all of them)
-    for (uint32_t w0 = blockIdx.y * 256 + (threadIdx.x & ~(kWave - 1u)); w0 < items; w0 += stride) {
-      const uint32_t w = w0 + lane;
-      bool inner = false;
-      uint32_t d = 0, pos = 0, pair = 0, b = 0, sz = 0;
-      if (w < items) {
-        uint32_t k;
-        if (w < full) {
-          d = 31u - (uint32_t)__clz(w + 1);
-          k = w + 1 - (1u << d);
+    for (uint32_t w = blockIdx.y * 256 + threadIdx.x; w < items; w += stride) {
+      const uint32_t d = w < full ? 31u - (uint32_t)__clz(w + 1) : ms.D;
+      const uint32_t k = w < full ? w + 1 - (1u << d) : w - full;
+      // range of node (d, k) from the root's halvings along k's bits
+      uint32_t b = 0, sz = er.size;
+      for (int j = (int)d - 1; j >= 0; j--) {
+        const uint32_t h = sz >> 1;
+        if ((k >> j) & 1u) {
+          b += h;
+          sz -= h;
         } else {
-          d = ms.D;
-          k = w - full;
-        }
-        // range of node (d, k) from the root's halvings along k's bits
-        sz = er.size;
-        for (int j = (int)d - 1; j >= 0; j--) {
-          const uint32_t h = sz >> 1;
-          if ((k >> j) & 1u) {
-            b += h;
-            sz -= h;
-          } else {
-            sz = h;
-          }
-        }
-        inner = sz > T;  // else a leaf at depth D, written by its parent
-        if (inner) {
-          const uint32_t I = d < ms.D ? w : full + (b - k * ms.q);
-          pos = d == 0 ? er.pos : er.pairBase + 2 * ((1u << (d - 1)) - 1u + (k >> 1)) + (k & 1u);
-          pair = er.pairBase + 2 * I;
-          Node nd;
-          for (int dd = 0; dd < 3; dd++) { nd.lo[dd] = INFINITY; nd.hi[dd] = -INFINITY; }
-          nd.oc = pack_oc(pair, 0);
-          nodes[pos] = nd;
-          const uint32_t h = sz >> 1;
-          const uint32_t cs[2] = {h, sz - h}, cbeg[2] = {b, b + h};
-          for (int side = 0; side < 2; side++)
-            if (cs[side] <= T) {
-              Node lf;
-              range_box(boxes, primIDs, er.begin + cbeg[side], cs[side], lf);
-              lf.oc = pack_oc(er.begin + cbeg[side], cs[side]);
-              nodes[pair + side] = lf;
-            }
+          sz = h;
         }
       }
-      // bucket slots: one atomic per distinct depth in the wave
-      uint64_t rem = __ballot(inner);
-      while (rem) {
-        const uint32_t leader = (uint32_t)__builtin_ctzll(rem);
-        const uint32_t dl = (uint32_t)__shfl((int)d, (int)leader, kWave);
-        const uint64_t grp = __ballot(inner && d == dl);
-        uint32_t slot0 = 0;
-        if (lane == leader) slot0 = atomicAdd(&bucketCursor[kBits + 1 + dl], (uint32_t)__popcll(grp));
-        slot0 = (uint32_t)__shfl((int)slot0, (int)leader, kWave);
-        if (inner && d == dl)
-          bucket[bucketStart[kBits + 1 + dl] + slot0 + (uint32_t)__popcll(grp & ((1ull << lane) - 1ull))] = pos;
-        rem &= ~grp;
-      }
+      if (sz <= T) continue;  // a leaf at depth D, written by its parent
+      const uint32_t I = d < ms.D ? w : full + (b - k * ms.q);
+      const uint32_t pos = d == 0 ? er.pos : er.pairBase + 2 * ((1u << (d - 1)) - 1u + (k >> 1)) + (k & 1u);
+      const uint32_t pair = er.pairBase + 2 * I;
+      Node nd;
+      for (int dd = 0; dd < 3; dd++) { nd.lo[dd] = INFINITY; nd.hi[dd] = -INFINITY; }
+      nd.oc = pack_oc(pair, 0);
+      nodes[pos] = nd;
+      up[(pair - 2) / 2] = pos;
+      arrive[(pair - 2) / 2] = 0;
+      const uint32_t h = sz >> 1;
+      const uint32_t cs[2] = {h, sz - h}, cbeg[2] = {b, b + h};
+      for (int side = 0; side < 2; side++)
+        if (cs[side] <= T) {
+          Node lf;
+          range_box(boxes, primIDs, er.begin + cbeg[side], cs[side], lf);
+          lf.oc = pack_oc(er.begin + cbeg[side], cs[side]);
+          nodes[pair + side] = lf;
+        }
     }
   }
 }
 
-// Refit of one bucket's inner nodes from their children, which are final
-// (leaves carry their boxes; inner children were refitted in an earlier
-// bucket).  Entries are split-node slots (node pos[s], children 2 + 2s) or,
-// for middle-split buckets, node positions.
-__device__ __forceinline__ void karras_refit_one(uint32_t e, bool slots, const uint32_t *pos, Node *nodes) {
-  uint32_t p, c0;
-  if (slots) {
-    p = pos[e];
-    c0 = 2 + 2 * e;
-  } else {
-    p = e;
-    c0 = (uint32_t)oc_offset(nodes[p].oc);
-  }
-  const Node l = nodes[c0], r = nodes[c0 + 1];
-  Node *me = &nodes[p];
-  for (int d = 0; d < 3; d++) {
-    me->lo[d] = fminf(l.lo[d], r.lo[d]);
-    me->hi[d] = fmaxf(l.hi[d], r.hi[d]);
+// The box [lo, hi] of inner node `node` stored, and those of the nodes above it
+// for as long as this thread is the last to come: past a sibling that is a
+// leaf, and of two inner siblings the second to arrive.  Boxes are handed over
+// as in refit.hip.
+__device__ __forceinline__ void karras_climb(Node *nodes, const uint32_t *up, uint32_t *arrive, uint32_t node,
+                                             float (&lo)[3], float (&hi)[3]) {
+  while (true) {
+    store_box_agent(&nodes[node], lo, hi);
+    if (node == 0) return;
+    const uint32_t sib = node ^ 1u, pair = (node - 2) / 2;  // (pairs begin at even nodes)
+    const Node s = nodes[sib];
+    float sl[3] = {s.lo[0], s.lo[1], s.lo[2]}, sh[3] = {s.hi[0], s.hi[1], s.hi[2]};
+    if (!oc_count(s.oc)) {
+      // this node's box has reached the coherence point before its arrival counts
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (__hip_atomic_fetch_add(&arrive[pair], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
+      asm volatile("" ::: "memory");
+      load_box_agent(&nodes[sib], sl, sh);
+    }
+    const bool left = (node & 1u) == 0;
+    for (int d = 0; d < 3; d++) {
+      lo[d] = left ? fminf(lo[d], sl[d]) : fminf(sl[d], lo[d]);
+      hi[d] = left ? fmaxf(hi[d], sh[d]) : fmaxf(sh[d], hi[d]);
+    }
+    node = up[pair];
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_karras_refit(const uint32_t *list, uint32_t begin, uint32_t count,
-                                                         bool slots, const uint32_t *pos, Node *nodes) {
-  const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-  if (t < count) karras_refit_one(list[begin + t], slots, pos, nodes);
-}
-
-// The narrow buckets in one workgroup, in order; its barriers order them
-// (one CU: a bucket's node writes are seen by the later buckets' reads).
-// Split-node buckets (slots) are ranges of the slots sorted by prefix
-// length; middle-split buckets are ranges of node positions.
-struct RefitRange {
-  uint32_t begin, count, slots, pad;
-};
-constexpr int kRefitTopBuckets = kDeltaBins;
-__global__ __launch_bounds__(1024) void k_karras_refit_top(const uint32_t *slotList, const uint32_t *posList,
-                                                           const RefitRange *ranges, int numRanges,
-                                                           const uint32_t *pos, Node *nodes) {
-  for (int r = 0; r < numRanges; r++) {
-    const RefitRange rr = ranges[r];
-    const uint32_t *list = rr.slots ? slotList : posList;
-    for (uint32_t t = threadIdx.x; t < rr.count; t += 1024)
-      karras_refit_one(list[rr.begin + t], rr.slots != 0, pos, nodes);
-    __syncthreads();
+// Boxes of the inner nodes, from the pairs of two leaves up.  Pairs are in
+// position order, so a workgroup's kClimb pairs hold whole subtrees: those are
+// climbed in LDS (a pair's leaves count as arrived), and what is left at the
+// subtrees' tops goes on through memory.  Bound by the latency of the climbs,
+// in memory 5 us a level.  3M prims, leaves of 8: 44 us, 132 us all in memory,
+// 140 us with the nodes sorted by prefix length and a launch for each.
+constexpr uint32_t kClimb = 1024;
+__global__ __launch_bounds__(kClimb) void k_karras_climb(Node *nodes, const uint32_t *up, uint32_t *arrive,
+                                                         uint32_t numPairs) {
+  __shared__ float sBox[6][2 * kClimb];  // of the pairs' two nodes
+  __shared__ uint32_t sSeen[kClimb];     // which of them are there
+  __shared__ uint32_t sUp[kClimb];
+  const uint32_t t0 = blockIdx.x * kClimb, i = threadIdx.x, t = t0 + i;
+  const uint32_t cnt = min(kClimb, numPairs - t0);
+  uint32_t leaves = 0;
+  float lo[3], hi[3];
+  if (i < cnt) {
+    const Node c[2] = {nodes[2 + 2 * (size_t)t], nodes[3 + 2 * (size_t)t]};
+#pragma unroll
+    for (uint32_t side = 0; side < 2; side++)
+      if (oc_count(c[side].oc)) {
+        leaves |= 1u << side;
+        for (int d = 0; d < 3; d++) {
+          sBox[d][2 * i + side] = c[side].lo[d];
+          sBox[3 + d][2 * i + side] = c[side].hi[d];
+        }
+      }
+    for (int d = 0; d < 3; d++) {
+      lo[d] = fminf(c[0].lo[d], c[1].lo[d]);
+      hi[d] = fmaxf(c[0].hi[d], c[1].hi[d]);
+    }
+    sUp[i] = up[t];
+  }
+  sSeen[i] = leaves;
+  __syncthreads();
+  uint32_t q = i, node = 0;
+  bool climbing = leaves == 3u, out = false;
+  while (climbing) {
+    node = sUp[q];
+    q = (node - 2) / 2 - t0;
+    out = node == 0 || q >= cnt;
+    if (out) break;
+    const uint32_t side = node & 1u;
+    for (int d = 0; d < 3; d++) {
+      nodes[node].lo[d] = lo[d];
+      nodes[node].hi[d] = hi[d];
+      sBox[d][2 * q + side] = lo[d];
+      sBox[3 + d][2 * q + side] = hi[d];
+    }
+    // (a wave's LDS accesses run in program order)
+    asm volatile("" ::: "memory");
+    climbing = ((atomicOr(&sSeen[q], 1u << side) >> (side ^ 1u)) & 1u) != 0;
+    asm volatile("" ::: "memory");
+    if (climbing)
+      for (int d = 0; d < 3; d++) {
+        const float sl = sBox[d][2 * q + (side ^ 1u)], sh = sBox[3 + d][2 * q + (side ^ 1u)];
+        lo[d] = side == 0 ? fminf(lo[d], sl) : fminf(sl, lo[d]);
+        hi[d] = side == 0 ? fmaxf(hi[d], sh) : fmaxf(sh, hi[d]);
+      }
+  }
+  __syncthreads();
+  if (out) karras_climb(nodes, up, arrive, node, lo, hi);
+  // a pair that one inner node has come to, and the other has not
+  const uint32_t inner = sSeen[i] & ~leaves;
+  if (inner && sSeen[i] != 3u) {
+    const uint32_t side = inner >> 1;
+    for (int d = 0; d < 3; d++) {
+      lo[d] = sBox[d][2 * i + side];
+      hi[d] = sBox[3 + d][2 * i + side];
+    }
+    karras_climb(nodes, up, arrive, 2 + 2 * t + side, lo, hi);
   }
 }
 
@@ -942,20 +925,16 @@ int build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, in
       return fail((set_error("id copy failed"), CUBQL_ERR_HIP));
   }
   // hierarchy in one pass over the radix-tree nodes, one host check for the
-  // node count, then the refit by prefix length
+  // node count, then the boxes of the inner nodes
   int hs = prof_begin(s);
-  constexpr int kBits = 8 * (int)sizeof(K);
   const uint32_t scanTiles = div_up(std::max(n, 1u), kCountScanTile);
   const uint32_t numKBlocks = div_up(std::max(n, 1u), kKBlock);
-  enum { M_SPLIT = 0, M_EQPAIRS = 1, M_FAR = 2, M_ROOTEQ = 3, M_ERR = 4, M_EQCURSOR = 5, M_WORDS = 8 };
+  enum { M_SPLIT = 0, M_EQPAIRS = 1, M_FAR = 2, M_ROOTEQ = 3, M_ERR = 4, M_EQCURSOR = 5, M_EQROOTS = 6, M_WORDS = 8 };
   KNode *kn = nullptr;
   uint32_t *splitFlag = nullptr, *slotArr = nullptr, *eqPairs = nullptr, *eqBase = nullptr, *misc = nullptr;
-  uint32_t *hist = nullptr, *bStart = nullptr, *bCursor = nullptr, *bucket = nullptr, *pos = nullptr;
-  uint32_t *splitList = nullptr, *dnKey = nullptr, *dnVal = nullptr, *dnKeyB = nullptr, *dnValB = nullptr;
-  uint32_t *blockHist = nullptr;
+  uint32_t *splitList = nullptr, *up = nullptr, *arrive = nullptr;
   uint64_t *kStatus = nullptr;
   EqRoot *eqRoots = nullptr;
-  RefitRange *topRanges = nullptr;
   ScratchArena hscr(mem, s);
   const size_t n1 = std::max(n, 1u);
   CUBQL_CHECK(hscr.reserve(&kn, n1));
@@ -963,43 +942,33 @@ int build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, in
   CUBQL_CHECK(hscr.reserve(&slotArr, n1));
   CUBQL_CHECK(hscr.reserve(&eqPairs, n1));
   CUBQL_CHECK(hscr.reserve(&eqBase, n1));
-  CUBQL_CHECK(hscr.reserve(&pos, n1));
-  CUBQL_CHECK(hscr.reserve(&bucket, n1));  // middle-split inner nodes (< n)
+  CUBQL_CHECK(hscr.reserve(&up, n1));
   CUBQL_CHECK(hscr.reserve(&splitList, n1));
-  CUBQL_CHECK(hscr.reserve(&dnKey, n1));
-  CUBQL_CHECK(hscr.reserve(&dnVal, n1));
-  CUBQL_CHECK(hscr.reserve(&dnKeyB, n1));
-  CUBQL_CHECK(hscr.reserve(&dnValB, n1));
+  CUBQL_CHECK(hscr.reserve(&arrive, n1));
   CUBQL_CHECK(hscr.reserve(&eqRoots, n1));
-  CUBQL_CHECK(hscr.reserve(&blockHist, (size_t)kDeltaBins * numKBlocks));
   CUBQL_CHECK(hscr.reserve(&kStatus, 2 * (size_t)scanTiles));
-  CUBQL_CHECK(hscr.reserve(&misc, M_WORDS + 3 * kDeltaBins));
-  CUBQL_CHECK(hscr.reserve(&topRanges, kRefitTopBuckets));
+  CUBQL_CHECK(hscr.reserve(&misc, M_WORDS));
   uint32_t *farList = nullptr;
   CUBQL_CHECK(hscr.reserve(&farList, n1));
   if (hscr.commit() != CUBQL_OK) return fail(CUBQL_ERR_ALLOC);
-  hist = misc + M_WORDS;
-  bStart = hist + kDeltaBins;
-  bCursor = bStart + kDeltaBins;
-  if (fill_u32(misc, 0u, M_WORDS + 3 * kDeltaBins, s) != CUBQL_OK ||
+  if (fill_u32(misc, 0u, M_WORDS, s) != CUBQL_OK ||
       fill_u32((uint32_t *)kStatus, 0u, 4 * (size_t)scanTiles, s) != CUBQL_OK)
     return fail(CUBQL_ERR_HIP);
   // the valid count is on the device only: the grids are sized by n and
   // the kernels stop at the count
   const uint32_t *nv = &c.ctr[C_NUMVALID];
   k_karras_info<K><<<1, 1, 0, s>>>(kRes, nv, T, misc);
-  k_karras<K><<<numKBlocks, kKThreads, 0, s>>>(kRes, nv, T, kn, splitFlag, eqPairs, blockHist, numKBlocks, farList,
+  k_karras<K><<<numKBlocks, kKThreads, 0, s>>>(kRes, nv, T, kn, splitFlag, eqPairs, misc + M_EQROOTS, farList,
                                                misc + M_FAR);
-  k_karras_far<K><<<1024, 256, 0, s>>>(kRes, nv, T, farList, misc + M_FAR, kn, splitFlag, eqPairs, blockHist,
-                                       numKBlocks);
-  k_karras_binscan<<<kDeltaBins, 1024, 0, s>>>(blockHist, numKBlocks, hist);
+  k_karras_far<K><<<1024, 256, 0, s>>>(kRes, nv, T, farList, misc + M_FAR, kn, splitFlag, eqPairs,
+                                       misc + M_EQROOTS);
   k_karras_scan2<<<scanTiles, 1024, 0, s>>>(splitFlag, eqPairs, slotArr, eqBase, splitList, nv, kStatus,
                                             kStatus + scanTiles,
                                             misc + M_SPLIT, misc + M_EQPAIRS, misc + M_ERR);
   if (hipGetLastError() != hipSuccess) return fail((set_error("hierarchy launch failed"), CUBQL_ERR_HIP));
-  std::vector<uint32_t> hm(M_WORDS + kDeltaBins);
+  uint32_t hm[M_WORDS];
   uint32_t numValid = 0, spinWord = 0;
-  if (hipMemcpyAsync(hm.data(), misc, sizeof(uint32_t) * hm.size(), hipMemcpyDeviceToHost, s) != hipSuccess ||
+  if (hipMemcpyAsync(hm, misc, sizeof(hm), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipMemcpyAsync(&numValid, nv, sizeof(uint32_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipMemcpyAsync(&spinWord, &c.ctr[C_SPIN], sizeof(uint32_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
@@ -1008,46 +977,18 @@ int build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, in
   prof_set(hs, 40.0 * numValid, numValid);
   if (hm[M_ERR] || spinWord)
     return fail((set_error("radix build: a look-back wait exceeded its bound"), CUBQL_ERR_INTERNAL));
-  uint32_t *hh = hm.data() + M_WORDS;
   const bool rootEq = hm[M_ROOTEQ] != 0;
   const bool rootLeaf = numValid <= T;
-  uint32_t numSplit = hm[M_SPLIT], eqInner = hm[M_EQPAIRS], numEqRoots = hh[kBinEqRoots];
+  uint32_t numSplit = hm[M_SPLIT], eqInner = hm[M_EQPAIRS], numEqRoots = hm[M_EQROOTS];
   if (rootEq) {
-    // no split node: the refit buckets are those of the one subtree
+    // no split node: one subtree, if any
     numSplit = 0;
     numEqRoots = rootLeaf ? 0 : 1;
     eqInner = rootLeaf ? 0 : mid_inner(numValid, T);
-    std::fill(hh, hh + kDeltaBins, 0u);
-    if (!rootLeaf) {
-      const MidShape ms = mid_shape(numValid, T);
-      for (uint32_t t = 0; t <= ms.D; t++) hh[kBits + 1 + t] = ms.at(t);
-    }
   }
-  hh[kBinEqRoots] = 0;  // not a refit bucket
   const uint64_t nodes64 = numValid == 0 ? 0 : 2 + 2 * (uint64_t)numSplit + 2 * (uint64_t)eqInner;
   if (nodes64 > 0xffffffffull) return fail((set_error("radix build: node count overflows"), CUBQL_ERR_INTERNAL));
   const uint32_t numNodes = (uint32_t)nodes64;
-  // bucket starts: split-node buckets are ranges of the slots sorted by
-  // prefix length (ascending); middle-split buckets are ranges of `bucket`
-  std::vector<uint32_t> hStart(kDeltaBins, 0);
-  for (int d = 0, runS = 0, runE = 0; d < kDeltaBins; d++) {
-    if (d < kBits) {
-      hStart[d] = (uint32_t)runS;
-      runS += (int)hh[d];
-    } else {
-      hStart[d] = (uint32_t)runE;
-      runE += (int)hh[d];
-    }
-  }
-  // refit order: middle-split buckets deepest first, then split-node
-  // buckets by decreasing prefix length; the narrow tail (every bucket
-  // after the last wide one) goes to one workgroup
-  constexpr uint32_t kRefitTopMax = 4096;
-  std::vector<RefitRange> order;
-  for (int d = kDeltaBins - 1; d >= 0; d--)
-    if (hh[d]) order.push_back(RefitRange{hStart[d], hh[d], d < kBits ? 1u : 0u, 0u});
-  size_t topFrom = order.size();
-  while (topFrom > 0 && order[topFrom - 1].count <= kRefitTopMax) topFrom--;
   Node *nodes = nullptr;
   int es = prof_begin(s);
   st = mem_alloc(mem, (void **)&nodes, std::max<size_t>(numNodes, 2) * sizeof(Node), s);
@@ -1056,36 +997,22 @@ int build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, in
     mem_free(mem, nodes, s);
     return fail(e);
   };
-  uint32_t *slotsByDn = dnVal;
   // node 1 stays unused (zero), as in the reference (radix.h:585-586)
   if (fill_u32((uint32_t *)(nodes + 1), 0u, sizeof(Node) / 4, s) != CUBQL_OK) return failN(CUBQL_ERR_HIP);
   if (numValid) {
-    if (hipMemcpyAsync(bStart, hStart.data(), sizeof(uint32_t) * kDeltaBins, hipMemcpyHostToDevice, s) != hipSuccess ||
-        (order.size() > topFrom &&
-         hipMemcpyAsync(topRanges, order.data() + topFrom, sizeof(RefitRange) * (order.size() - topFrom),
-                        hipMemcpyHostToDevice, s) != hipSuccess))
-      return failN((set_error("bucket upload failed"), CUBQL_ERR_HIP));
     if (rootLeaf) {
       k_karras_leaf_root<<<1, 256, 0, s>>>(boxes, primIDs, nv, nodes);
     } else if (rootEq) {
       k_karras_root_eq<<<1, 1, 0, s>>>(nv, eqRoots);
     } else {
       k_karras_emit<K><<<div_up(numSplit, kBlock), kBlock, 0, s>>>(kRes, boxes, primIDs, T, kn, splitList, numSplit,
-                                                                   slotArr, eqPairs, eqBase, dnKey, dnVal, pos,
-                                                                   nodes, eqRoots, misc + M_EQCURSOR);
-      // split nodes into prefix-length order (one 8-bit pass; lengths < 64).
-      // No host check follows, so its look-back waits are the unbounded
-      // kind (every tile waited on is held by a running workgroup).
-      uint32_t *kOut = nullptr;
-      st = radix_sort_pairs_dev_u32(dnKey, dnVal, dnKeyB, dnValB, misc + M_SPLIT, numSplit, 8, s, mem, &kOut,
-                                    &slotsByDn, nullptr);
-      if (st) return failN(st);
+                                                                   slotArr, eqPairs, eqBase, up, arrive, nodes,
+                                                                   eqRoots, misc + M_EQCURSOR);
     }
     if (numEqRoots) {
       // a few workgroups per subtree when there are few subtrees
       const uint32_t gx = std::min(numEqRoots, 16384u), gy = std::min(64u, std::max(1u, 1024u / numEqRoots));
-      k_karras_equal<<<dim3(gx, gy), 256, 0, s>>>(boxes, primIDs, T, eqRoots, numEqRoots, kBits, bStart,
-                                                  bCursor, bucket, nodes);
+      k_karras_equal<<<dim3(gx, gy), 256, 0, s>>>(boxes, primIDs, T, eqRoots, numEqRoots, up, arrive, nodes);
     }
     if (hipGetLastError() != hipSuccess) return failN((set_error("hierarchy emit launch failed"), CUBQL_ERR_HIP));
   }
@@ -1097,13 +1024,8 @@ int build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, in
   bvh->numPrims = numValid;
   int rs = prof_begin(s);
   if (numValid && !rootLeaf) {
-    for (size_t r = 0; r < topFrom; r++)
-      k_karras_refit<<<div_up(order[r].count, kBlock), kBlock, 0, s>>>(order[r].slots ? slotsByDn : bucket,
-                                                                        order[r].begin, order[r].count,
-                                                                        order[r].slots != 0, pos, nodes);
-    if (order.size() > topFrom)
-      k_karras_refit_top<<<1, 1024, 0, s>>>(slotsByDn, bucket, topRanges, (int)(order.size() - topFrom), pos,
-                                            nodes);
+    const uint32_t pairs = numSplit + eqInner;
+    k_karras_climb<<<div_up(pairs, kClimb), kClimb, 0, s>>>(nodes, up, arrive, pairs);
   }
   st = hipGetLastError() == hipSuccess ? CUBQL_OK : (set_error("refit launch failed"), CUBQL_ERR_HIP);
   prof_end(rs, s, "refit");

@@ -15,6 +15,8 @@
 // whole L2 instead.  1M boxes, leaf 4: 3265 us with
 // fences, 88 us now.  Two leaves under one parent, the most common pair, are
 // one thread's work and need no arrival.
+#include "block_ops.h"
+#include "build_common.h"
 #include "common.h"
 #include "refit.h"
 
@@ -70,26 +72,6 @@ __device__ __forceinline__ void leaf_box(const cubql_box3f *boxes, const uint32_
   }
 }
 
-// The 24 bytes of a node's box as three 8-byte words (a node is 16-byte
-// aligned), stored and loaded at agent scope.
-__device__ __forceinline__ void store_box(Node *nd, const float (&lo)[3], const float (&hi)[3]) {
-  uint64_t *w = reinterpret_cast<uint64_t *>(nd);
-  const float v[6] = {lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]};
-#pragma unroll
-  for (int j = 0; j < 3; j++)
-    __hip_atomic_store(w + j, (uint64_t)__float_as_uint(v[2 * j]) | ((uint64_t)__float_as_uint(v[2 * j + 1]) << 32),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void load_node_box(const Node *nd, float (&lo)[3], float (&hi)[3]) {
-  const uint64_t *w = reinterpret_cast<const uint64_t *>(nd);
-  uint64_t v[3];
-#pragma unroll
-  for (int j = 0; j < 3; j++) v[j] = __hip_atomic_load(w + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  lo[0] = __uint_as_float((uint32_t)v[0]); lo[1] = __uint_as_float((uint32_t)(v[0] >> 32));
-  lo[2] = __uint_as_float((uint32_t)v[1]); hi[0] = __uint_as_float((uint32_t)(v[1] >> 32));
-  hi[1] = __uint_as_float((uint32_t)v[2]); hi[2] = __uint_as_float((uint32_t)(v[2] >> 32));
-}
-
 __global__ __launch_bounds__(256) void k_refit(Node *nodes, uint32_t numNodes, const uint32_t *primIDs,
                                                const cubql_box3f *boxes, const uint32_t *parent, uint32_t *arrive) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < numNodes; i += gridDim.x * blockDim.x) {
@@ -122,7 +104,7 @@ __global__ __launch_bounds__(256) void k_refit(Node *nodes, uint32_t numNodes, c
       }
     }
     while (true) {
-      store_box(&nodes[node], lo, hi);
+      store_box_agent(&nodes[node], lo, hi);
       const uint32_t p = parent[node];
       if (p == 0xffffffffu) break;
       const uint32_t left = (uint32_t)oc_offset(nodes[p].oc);
@@ -134,7 +116,7 @@ __global__ __launch_bounds__(256) void k_refit(Node *nodes, uint32_t numNodes, c
       // the sibling's box, combined in child order
       const bool isLeft = node == left;
       float sl[3], sh[3];
-      load_node_box(&nodes[isLeft ? left + 1 : left], sl, sh);
+      load_box_agent(&nodes[isLeft ? left + 1 : left], sl, sh);
       for (int d = 0; d < 3; d++) {
         lo[d] = isLeft ? fminf(lo[d], sl[d]) : fminf(sl[d], lo[d]);
         hi[d] = isLeft ? fmaxf(hi[d], sh[d]) : fmaxf(sh[d], hi[d]);
