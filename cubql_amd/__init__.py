@@ -207,10 +207,15 @@ class TorchMemory:
 
         def _malloc(pp, size, stream, user):
             try:
-                st = (torch.cuda.ExternalStream(stream, device=self.device) if stream
-                      else torch.cuda.default_stream(self.device))
-                with torch.cuda.stream(st):
+                # (entering a stream takes as long as the allocation: 3001
+                # points, three blocks, a build and a query: 202 us, 187 without)
+                if torch.cuda.current_stream(self.device).cuda_stream == (stream or 0):
                     t = torch.empty(int(size), dtype=torch.uint8, device=self.device)
+                else:
+                    st = (torch.cuda.ExternalStream(stream, device=self.device) if stream
+                          else torch.cuda.default_stream(self.device))
+                    with torch.cuda.stream(st):
+                        t = torch.empty(int(size), dtype=torch.uint8, device=self.device)
                 self.live[t.data_ptr()] = t
                 pp[0] = t.data_ptr()
                 return 0
