@@ -780,10 +780,10 @@ __global__ __launch_bounds__(1024) void k_emit(Ctx c, int level) {
 // whatever its size, and most splits are of few prims.  So the wave splits
 // nodes one by one only while they have more than kRow prims; the subtrees
 // under those, kept in order in frontier[], are then built four at a time, one
-// in each row of 16 lanes, a prim and a bin to a lane (bin counts up to 16).
+// in each row of 16 lanes, a prim and one, two or four bins to a lane.
 // Splits are given pairs as they come; their places in depth-first order are
 // left for k_small_emit.  1.31M prims, leaves of 4: 1330 us with one node at a
-// time, 588 us so.
+// time, 588 us so; with 32 bins 1470 and 669 us.
 constexpr uint32_t kRow = 16;
 
 struct SmallShare {
@@ -823,6 +823,12 @@ template <int OP>
 __device__ __forceinline__ int32_t row_from(int32_t v) {
   return row_step<OP, 0x108>(row_step<OP, 0x104>(row_step<OP, 0x102>(row_step<OP, 0x101>(v))));
 }
+// union of the lanes after (exclusive)
+template <int OP>
+__device__ __forceinline__ int32_t row_after(int32_t v) {
+  constexpr int32_t I = OP == 0 ? INT32_MAX : (OP == 1 ? INT32_MIN : 0);
+  return row_from<OP>(__builtin_amdgcn_update_dpp(I, v, 0x101, 0xF, 0xF, false));
+}
 // of the whole row, in every lane (row_ror)
 template <int OP>
 __device__ __forceinline__ int32_t row_all(int32_t v) {
@@ -842,13 +848,14 @@ __device__ __forceinline__ uint16_t *pair_places(const Ctx &c, const SmallSeg &s
 // of the segment's pairs.  numPairs: pairs of the splits above.  Returns the
 // number of the segment's pairs.  (Every lane stays in the loop: a row without a
 // subtree computes on identities.)
+template <int PER>
 __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sBins, SmallShare &sh, uint32_t numSub,
                                uint32_t numPairs, uint16_t *place) {
   const uint32_t lane = lane_id(), r = lane & 15u, row0 = lane & 48u;
   const uint64_t rowMask = 0xffffull << row0, rowsBefore = (1ull << row0) - 1;
   const int nb = c.nb;
   Node *loc = c.loc + 2 * (size_t)gb;
-  int32_t *bins = sBins + row0 * kBinWords;
+  int32_t *bins = sBins + row0 * PER * kBinWords;  // (bins PER r .. PER r + PER - 1 are lane r's)
   uint32_t *stack = sh.stack + row0;  // right siblings: at most kRow - 1
   const uint32_t above = numPairs;
   uint32_t next = 0, sub = 0, splits = 0, sp = 0;
@@ -905,13 +912,16 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
     }
     // a lane per bin, one dimension after the other in the row's bins
     float cost[3];
-    int myBin[3];
+    int myBin[3], costBin[3];
     float leafCost = 0.f;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-      int4 *w4 = reinterpret_cast<int4 *>(bins + r * kBinWords);
-      w4[0] = make_int4(bin_init(0), bin_init(1), bin_init(2), bin_init(3));
-      w4[1] = make_int4(bin_init(4), bin_init(5), 0, 0);
+      int4 *w4 = reinterpret_cast<int4 *>(bins + r * PER * kBinWords);
+#pragma unroll
+      for (int k = 0; k < PER; k++) {
+        w4[2 * k] = make_int4(bin_init(0), bin_init(1), bin_init(2), bin_init(3));
+        w4[2 * k + 1] = make_int4(bin_init(4), bin_init(5), 0, 0);
+      }
       sync_wave_lds();
       myBin[d] = sah_bin(ce[d], clo[d], chi[d], nb, c.binEps);
       if (in) {
@@ -923,22 +933,66 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
         atomicAdd(&w[6], 1);
       }
       sync_wave_lds();
-      const int4 p = w4[0], q = w4[1];
-      sync_wave_lds();
-      const int32_t wlo[3] = {p.x, p.y, p.z}, whi[3] = {p.w, q.x, q.y};
-      float llo[3], lhi[3], rlo[3], rhi[3];
+      int32_t w[PER][7];  // lo, hi, count
 #pragma unroll
-      for (int k = 0; k < 3; k++) {
-        llo[k] = dec_f(row_before<0>(wlo[k]));
-        lhi[k] = dec_f(row_before<1>(whi[k]));
-        rlo[k] = dec_f(row_from<0>(wlo[k]));
-        rhi[k] = dec_f(row_from<1>(whi[k]));
+      for (int k = 0; k < PER; k++) {
+        const int4 p = w4[2 * k], q = w4[2 * k + 1];
+        w[k][0] = p.x; w[k][1] = p.y; w[k][2] = p.z; w[k][3] = p.w; w[k][4] = q.x; w[k][5] = q.y; w[k][6] = q.z;
       }
-      const uint32_t lCnt = (uint32_t)row_before<2>(q.z), rCnt = (uint32_t)row_from<2>(q.z);
-      const float rTerm = box_measure(rlo, rhi, c.elh != 0) * (float)rCnt;
-      const float s = box_measure(llo, lhi, c.elh != 0) * (float)lCnt + rTerm;
-      cost[d] = (lCnt > 0 && rCnt > 0 && s == s) ? s : INFINITY;
-      if (d == 0) leafCost = __shfl(rTerm, (int)row0, kWave);
+      sync_wave_lds();
+      // unions of the bins before the lane's, and from each of its bins on
+      int32_t before[7], from[PER][7];
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        int32_t lo = w[0][j], hi = w[0][3 + j];
+#pragma unroll
+        for (int k = 1; k < PER; k++) {
+          lo = min(lo, w[k][j]);
+          hi = max(hi, w[k][3 + j]);
+        }
+        before[j] = row_before<0>(lo);
+        before[3 + j] = row_before<1>(hi);
+        from[PER - 1][j] = PER == 1 ? row_from<0>(lo) : min(w[PER - 1][j], row_after<0>(lo));
+        from[PER - 1][3 + j] = PER == 1 ? row_from<1>(hi) : max(w[PER - 1][3 + j], row_after<1>(hi));
+      }
+      int32_t cnt = 0;
+#pragma unroll
+      for (int k = 0; k < PER; k++) cnt += w[k][6];
+      before[6] = row_before<2>(cnt);
+      from[PER - 1][6] = PER == 1 ? row_from<2>(cnt) : w[PER - 1][6] + row_after<2>(cnt);
+#pragma unroll
+      for (int k = PER - 2; k >= 0; k--) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+          from[k][j] = min(from[k + 1][j], w[k][j]);
+          from[k][3 + j] = max(from[k + 1][3 + j], w[k][3 + j]);
+        }
+        from[k][6] = from[k + 1][6] + w[k][6];
+      }
+      cost[d] = INFINITY;
+      costBin[d] = 0;
+#pragma unroll
+      for (int k = 0; k < PER; k++) {
+        float llo[3], lhi[3], rlo[3], rhi[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+          llo[j] = dec_f(before[j]);
+          lhi[j] = dec_f(before[3 + j]);
+          rlo[j] = dec_f(from[k][j]);
+          rhi[j] = dec_f(from[k][3 + j]);
+          before[j] = min(before[j], w[k][j]);
+          before[3 + j] = max(before[3 + j], w[k][3 + j]);
+        }
+        const uint32_t lCnt = (uint32_t)before[6], rCnt = (uint32_t)from[k][6];
+        before[6] += w[k][6];
+        const float rTerm = box_measure(rlo, rhi, c.elh != 0) * (float)rCnt;
+        const float s = box_measure(llo, lhi, c.elh != 0) * (float)lCnt + rTerm;
+        if (lCnt > 0 && rCnt > 0 && s < cost[d]) {
+          cost[d] = s;
+          costBin[d] = (int)r * PER + k;
+        }
+        if (d == 0 && k == 0) leafCost = __shfl(rTerm, (int)row0, kWave);
+      }
     }
     // (as sah_decide_wave: the first minimum, the leaf first)
     int mode = kModeLeaf, bin = 0;
@@ -947,10 +1001,12 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
       for (int d = 0; d < 3; d++) {
         const float m = __int_as_float(row_all<0>(__float_as_int(cost[d])));
         const uint64_t at = __ballot(cost[d] == m) & rowMask;
+        const int first = PER == 1 ? (int)(__builtin_ctzll(at) - row0)
+                                   : __shfl(costBin[d], (int)__builtin_ctzll(at), kWave);
         if (who && m < best) {
           best = m;
           mode = d;
-          bin = (int)(__builtin_ctzll(at) - row0);
+          bin = first;
         }
       }
     };
@@ -1028,6 +1084,7 @@ __device__ uint32_t small_rows(const Ctx &c, uint32_t gb, Item *sIt, int32_t *sB
   return numPairs;
 }
 
+template <int PER>
 __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, Item *sIt,
                               int32_t *sBins, SmallShare &sh) {
   const uint32_t lane = lane_id();
@@ -1051,7 +1108,6 @@ __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx,
     return;
   }
   for (uint32_t i = lane; i < m; i += kWave) sIt[i] = gItems[gb + i];
-  const bool rows = nb <= (int)kRow;
   uint32_t numSub = 0;
   int sp = 1;
   if (lane == 0) sh.stack[0] = pack_task(0u, m, 0u);
@@ -1061,7 +1117,7 @@ __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx,
     uint32_t b, e, me;
     unpack_task((uint32_t)__builtin_amdgcn_readfirstlane((int)sh.stack[sp]), b, e, me);
     const uint32_t n = e - b;
-    if (rows && n <= kRow && n > c.T) {
+    if (n <= kRow && n > c.T) {
       if (lane == 0) {
         sh.frontier[numSub] = pack_task(b, e, me);
         sh.at[numSub] = (uint16_t)(nLocal / 2);
@@ -1144,27 +1200,31 @@ __device__ void small_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx,
     sync_wave_lds();
   }
   sync_wave_lds();
-  nLocal = 1 + 2 * small_rows(c, gb, sIt, sBins, sh, numSub, nLocal / 2, pair_places(c, sg));
+  nLocal = 1 + 2 * small_rows<PER>(c, gb, sIt, sBins, sh, numSub, nLocal / 2, pair_places(c, sg));
   if (lane == 0) c.smallCount[segIdx] = nLocal;
 }
 
+// Bins of a lane of a row: 16, 32 or 64 bins in a row.
+inline int bins_per_lane(int nb) { return nb <= 16 ? 1 : (nb <= 32 ? 2 : 4); }
+
 // LDS (dynamic, sized by the bin count): items | bins (of one node, or of one
 // dimension of four) | the rest
-__host__ __device__ constexpr int small_bin_words(int nb) {
-  return nb > (int)kRow ? 3 * nb * kBinWords : (3 * nb > 4 * (int)kRow ? 3 * nb : 4 * (int)kRow) * kBinWords;
+__host__ __device__ constexpr int small_bin_words(int nb, int per) {
+  return (3 * nb > 4 * (int)kRow * per ? 3 * nb : 4 * (int)kRow * per) * kBinWords;
 }
-__host__ __device__ constexpr size_t small_lds_bytes(int nb) {
-  return sizeof(Item) * kSmall + sizeof(int32_t) * small_bin_words(nb) + sizeof(SmallShare);
+inline size_t small_lds_bytes(int nb) {
+  return sizeof(Item) * kSmall + sizeof(int32_t) * small_bin_words(nb, bins_per_lane(nb)) + sizeof(SmallShare);
 }
 
+template <int PER>
 __global__ __launch_bounds__(kWave) void k_small(Ctx c) {
   extern __shared__ __align__(16) unsigned char smem[];
   Item *sIt = reinterpret_cast<Item *>(smem);
   int32_t *sBins = reinterpret_cast<int32_t *>(smem + sizeof(Item) * kSmall);
-  SmallShare &sh = *reinterpret_cast<SmallShare *>(sBins + small_bin_words(c.nb));
+  SmallShare &sh = *reinterpret_cast<SmallShare *>(sBins + small_bin_words(c.nb, PER));
   const uint32_t nSmall = c.ctr->numSmall;
   for (uint32_t w = blockIdx.x; w < nSmall; w += gridDim.x) {
-    small_segment(c, c.small[w], w, sIt, sBins, sh);
+    small_segment<PER>(c, c.small[w], w, sIt, sBins, sh);
     sync_wave_lds();
   }
 }
@@ -1321,7 +1381,9 @@ int sah_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T
   int smallSlot = -1;
   if (numSmall) {
     smallSlot = prof_begin(s);
-    k_small<<<smallGrid, kWave, small_lds_bytes(numBins), s>>>(c);
+    const int per = bins_per_lane(numBins);
+    const auto small = per == 1 ? k_small<1> : (per == 2 ? k_small<2> : k_small<4>);
+    small<<<smallGrid, kWave, small_lds_bytes(numBins), s>>>(c);
     prof_end(smallSlot, s, "sah_small");
     // (status tag beyond every level's)
     k_small_scan<<<div_up(numSmall, kCountScanTile), 1024, 0, s>>>(c, maxLevels + 2);
