@@ -244,9 +244,9 @@ __device__ __forceinline__ float split_cost(const int32_t *bins, int nb, int d, 
 // n = prims of the node.  Returns the split dim, kModeLeaf or kModeMiddle.
 __device__ int sah_decide_wave(const int32_t *bins, int nb, uint32_t n, uint32_t cap, bool elh, int &splitBin) {
   const uint32_t lane = lane_id();
-  float cost[3];     // candidate sets in (dim, bin) order; lane order within each
-  int passDim[3];    // first dim of each candidate set (-1: unused)
-  int nSets;
+  // candidate sets in (dim, bin) order, lane order within each: with at most 32
+  // bins dims 0 and 1, then dim 2
+  float cost[3] = {INFINITY, INFINITY, INFINITY};
   float leafCost;
   if (nb <= 32) {
     const uint32_t bl = lane & 31u, half = lane >> 5;
@@ -255,8 +255,6 @@ __device__ int sah_decide_wave(const int32_t *bins, int nb, uint32_t n, uint32_t
                                 elh, &leaf0);
     cost[1] = split_cost<false>(bins, nb, 2, bl, half == 0 && bl < (uint32_t)nb, (int)(nb - 1 - bl) & 63, elh,
                                 &leaf1);
-    passDim[0] = 0; passDim[1] = 2; passDim[2] = -1;
-    nSets = 2;
     leafCost = __shfl(leaf0, 0, kWave);
   } else {
     const bool inBin = lane < (uint32_t)nb;
@@ -264,9 +262,7 @@ __device__ int sah_decide_wave(const int32_t *bins, int nb, uint32_t n, uint32_t
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       cost[d] = split_cost<true>(bins, nb, d, lane, inBin, inBin ? nb - 1 - (int)lane : (int)lane, elh, &lt[d]);
-      passDim[d] = d;
     }
-    nSets = 3;
     leafCost = __shfl(lt[0], 0, kWave);
   }
   // rAreas[0] * rCount: the union of all bins is the node box
@@ -275,17 +271,16 @@ __device__ int sah_decide_wave(const int32_t *bins, int nb, uint32_t n, uint32_t
     int dim = kModeLeaf;
 #pragma unroll
     for (int p = 0; p < 3; p++) {
-      if (p >= nSets) break;
       // (costs are +0 .. +inf: their bit patterns order like the values)
       const float m = __int_as_float(wave_min_i32(__float_as_int(cost[p])));
       if (m < best) {
         best = m;
         const uint32_t idx = (uint32_t)__builtin_ctzll(__ballot(cost[p] == m));
         if (nb <= 32) {
-          dim = passDim[p] + (int)(idx >> 5);
+          dim = p == 0 ? (int)(idx >> 5) : 2;
           bin = (int)(idx & 31u);
         } else {
-          dim = passDim[p];
+          dim = p;
           bin = (int)idx;
         }
       }
@@ -464,7 +459,35 @@ __device__ __forceinline__ void seg_cb(const Seg &g, float (&lo)[3], float (&hi)
   for (int d = 0; d < 3; d++) { lo[d] = dec_f(g.cb[d]); hi[d] = dec_f(g.cb[d + 3]); }
 }
 
-// Bin: one LDS bin set per binning tile, written out as that tile's partial.
+// Evaluates SAH for open node s from its bins, by one wave: records the decision
+// and the node's box (the union of its bins); leaves are final here.
+__device__ __forceinline__ void decide_node(const Ctx &c, const int32_t *bins, const Seg &g, uint32_t s) {
+  const uint32_t n = g.end - g.begin;
+  const int nb = c.nb;
+  int bin = 0;
+  const int mode = sah_decide_wave(bins, nb, n, c.cap, c.elh != 0, bin);
+  // node box = union of the dimension-0 bins
+  float lo[3], hi[3];
+  const bool inBin = lane_id() < (uint32_t)nb;
+  const int32_t *w = bins + (inBin ? lane_id() : 0) * kBinWords;
+  for (int k = 0; k < 3; k++) {
+    lo[k] = dec_f(wave_min_i32(inBin ? w[k] : INT32_MAX));
+    hi[k] = dec_f(wave_max_i32(inBin ? w[3 + k] : INT32_MIN));
+  }
+  if (lane_id() == 0) {
+    c.segMode[s] = mode;
+    c.segBin[s] = bin;
+    if (mode >= 0) {
+      c.segLo[s] = dec_f(g.cb[mode]);
+      c.segHi[s] = dec_f(g.cb[mode + 3]);
+    }
+  }
+  store_node_wave(&c.nodes[g.node], lo, hi, mode == kModeLeaf ? pack_oc(g.begin, n) : 0ull);
+}
+
+// Bin: one LDS bin set per binning tile, written out as that tile's partial; a
+// node of one tile is decided here and has no partial (16 levels of 1.31M prims:
+// 100 us of the build).
 // Bound by LDS.  1.31M prims, the first level: 136 us with 21 atomics per prim
 // from 256 threads, 42 us with bin_add_read from 512 (all levels 1349 -> 535
 // us).  (Tiles of 4096 or 2048 prims: 3% and 6% of the build slower, through
@@ -491,15 +514,18 @@ __global__ __launch_bounds__(kBinBlock) void k_bin(Ctx c, int level) {
     const uint32_t e0 = min(b0 + (uint32_t)kBinTile, g.end);
     for (uint32_t i = b0 + threadIdx.x; i < e0; i += kBinBlock) bin_add_read(sBins, nb, c.binEps, src[i], clo, chi);
     sync_block_lds();
-    int32_t *out = c.partial + (size_t)bt * W;
-    for (int w = threadIdx.x; w < W; w += kBinBlock) out[w] = sBins[w];
+    if (c.binStart[s + 1] - c.binStart[s] == 1) {
+      if (threadIdx.x < kWave) decide_node(c, sBins, c.segs[par][s], s);
+    } else {
+      int32_t *out = c.partial + (size_t)bt * W;
+      for (int w = threadIdx.x; w < W; w += kBinBlock) out[w] = sBins[w];
+    }
     sync_block_lds();
   }
 }
 
-// Select: reduce a node's partials, evaluate SAH, record the decision and
-// the node's box (the union of its bins); leaves are final here.  Bound by the
-// latency of the partials, eight in flight (the root of 1.31M prims, 160 of
+// Select: reduce the partials of a node of several tiles and decide it.  Bound
+// by the latency of the partials, eight in flight (the root of 1.31M prims, 160 of
 // them: 93 us one after the other, 32 us so).
 __global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
   __shared__ int32_t sBins[3 * kMaxBins * kBinWords];
@@ -509,6 +535,7 @@ __global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
   const int W = 3 * nb * kBinWords;
   for (uint32_t s = blockIdx.x; s < nSeg; s += gridDim.x) {
     const uint32_t tb = c.binStart[s], te = c.binStart[s + 1];
+    if (te - tb == 1) continue;
     for (int w = threadIdx.x; w < W; w += kBlock) {
       const int k = w & (kBinWords - 1);
       int32_t acc = bin_init(w);
@@ -526,29 +553,7 @@ __global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
       sBins[w] = acc;
     }
     sync_block_lds();
-    if (threadIdx.x < kWave) {
-      const Seg g = c.segs[par][s];
-      const uint32_t n = g.end - g.begin;
-      int bin = 0;
-      const int mode = sah_decide_wave(sBins, nb, n, c.cap, c.elh != 0, bin);
-      // node box = union of the dimension-0 bins
-      float lo[3], hi[3];
-      const bool inBin = lane_id() < (uint32_t)nb;
-      const int32_t *w = sBins + (inBin ? lane_id() : 0) * kBinWords;
-      for (int k = 0; k < 3; k++) {
-        lo[k] = dec_f(wave_min_i32(inBin ? w[k] : INT32_MAX));
-        hi[k] = dec_f(wave_max_i32(inBin ? w[3 + k] : INT32_MIN));
-      }
-      if (lane_id() == 0) {
-        c.segMode[s] = mode;
-        c.segBin[s] = bin;
-        if (mode >= 0) {
-          c.segLo[s] = dec_f(g.cb[mode]);
-          c.segHi[s] = dec_f(g.cb[mode + 3]);
-        }
-      }
-      store_node_wave(&c.nodes[g.node], lo, hi, mode == kModeLeaf ? pack_oc(g.begin, n) : 0ull);
-    }
+    if (threadIdx.x < kWave) decide_node(c, sBins, c.segs[par][s], s);
     sync_block_lds();
   }
 }
