@@ -17,7 +17,7 @@
 //     open node owning a contiguous range (left side stable, right side
 //     reversed), so the tree and primIDs are a deterministic function of the
 //     input;
-//   * large nodes: binning tiles of 8192 prims build their bins in LDS and
+//   * large nodes: binning tiles of up to 8192 prims build their bins in LDS and
 //     write one partial per tile (no global atomics); one workgroup per node
 //     reduces the partials and one wave evaluates all 3 x numBins candidate
 //     planes at once (prefix/suffix unions as wave scans); the partition is
@@ -43,7 +43,10 @@ constexpr int kBlock = 256;
 // longer run at once: 1.31M prims 2.12 ms, 2.07 with 4, 2.09 with 2)
 constexpr int kItems = 4;
 constexpr int kTile = kBlock * kItems;  // partition tile: 1024 prims
-constexpr int kBinTile = 8 * kTile;     // binning tile: 8192 prims
+// Binning tile: a workgroup per CU at the root, up to 8192 prims (the sums over
+// smaller ones cost more than they save: 1.31M prims 1.92 ms with 6144, 2.01 with
+// 4096; 200K 981 us with 8192, 871 with 1024; 20K 565 and 513).
+constexpr uint32_t kBinTileMax = 8 * kTile;
 constexpr int kSmall = 256;             // max prims of a wave-finished node
 constexpr int kMaxBins = 64;            // one lane per bin
 constexpr int kBinWords = 8;            // lo xyz, hi xyz (encoded), count, pad
@@ -109,6 +112,7 @@ struct Ctx {
   int32_t *segBin;
   float *segLo, *segHi;  // centroid bounds of the split dim
   uint64_t *tileStatus;
+  uint32_t binTile;    // prims of a binning tile
   int32_t *partial;    // [binTiles][3*nb*kBinWords]
   SmallSeg *small;
   Node *loc;
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(1024) void k_count_scan(Ctx c, uint32_t numBlocks) 
       k->numLarge[0] = 1;
       c.tileStart[0] = 0;
       c.binStart[0] = 0;
-      level_plan_totals(c, 0u, 1u, div_up(run, kTile), div_up(run, kBinTile), run);
+      level_plan_totals(c, 0u, 1u, div_up(run, kTile), div_up(run, c.binTile), run);
     } else {
       if (run > 0) {
         c.small[0] = SmallSeg{0, run, 0, 0};
@@ -487,11 +491,9 @@ __device__ __forceinline__ void decide_node(const Ctx &c, const int32_t *bins, c
 
 // Bin: one LDS bin set per binning tile, written out as that tile's partial; a
 // node of one tile is decided here and has no partial (16 levels of 1.31M prims:
-// 100 us of the build).
-// Bound by LDS.  1.31M prims, the first level: 136 us with 21 atomics per prim
+// 100 us of the build).  Bound by LDS.  1.31M prims, the first level: 136 us with 21 atomics per prim
 // from 256 threads, 42 us with bin_add_read from 512 (all levels 1349 -> 535
-// us).  (Tiles of 4096 or 2048 prims: 3% and 6% of the build slower, through
-// the sums over them.)
+// us).
 constexpr int kBinBlock = 512;
 __global__ __launch_bounds__(kBinBlock) void k_bin(Ctx c, int level) {
   __shared__ __align__(16) int32_t sBins[3 * kMaxBins * kBinWords];
@@ -510,8 +512,8 @@ __global__ __launch_bounds__(kBinBlock) void k_bin(Ctx c, int level) {
     const Seg g = c.segs[par][s];
     float clo[3], chi[3];
     seg_cb(g, clo, chi);
-    const uint32_t b0 = g.begin + (bt - c.binStart[s]) * kBinTile;
-    const uint32_t e0 = min(b0 + (uint32_t)kBinTile, g.end);
+    const uint32_t b0 = g.begin + (bt - c.binStart[s]) * c.binTile;
+    const uint32_t e0 = min(b0 + c.binTile, g.end);
     for (uint32_t i = b0 + threadIdx.x; i < e0; i += kBinBlock) bin_add_read(sBins, nb, c.binEps, src[i], clo, chi);
     sync_block_lds();
     if (c.binStart[s + 1] - c.binStart[s] == 1) {
@@ -525,23 +527,28 @@ __global__ __launch_bounds__(kBinBlock) void k_bin(Ctx c, int level) {
 }
 
 // Select: reduce the partials of a node of several tiles and decide it.  Bound
-// by the latency of the partials, eight in flight (the root of 1.31M prims, 160 of
-// them: 93 us one after the other, 32 us so).
-__global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
+// by the latency of the partials: eight in flight, and up to eight parts of them
+// at once (the root of 1.31M prims, 160 partials: 93 us one after the other, 32 us
+// with eight in flight; all levels 1.3% of the build less with the parts).
+constexpr int kSelectBlock = 512;
+__global__ __launch_bounds__(kSelectBlock) void k_select(Ctx c, int level) {
   __shared__ int32_t sBins[3 * kMaxBins * kBinWords];
   const int par = level & 1;
   const uint32_t nSeg = c.ctr->numLarge[par];
-  const int nb = c.nb;
-  const int W = 3 * nb * kBinWords;
+  const uint32_t W = 3 * (uint32_t)c.nb * kBinWords;
   for (uint32_t s = blockIdx.x; s < nSeg; s += gridDim.x) {
-    const uint32_t tb = c.binStart[s], te = c.binStart[s + 1];
-    if (te - tb == 1) continue;
-    for (int w = threadIdx.x; w < W; w += kBlock) {
-      const int k = w & (kBinWords - 1);
-      int32_t acc = bin_init(w);
-      const int32_t *p = c.partial + (size_t)tb * W + w;
+    const uint32_t tb = c.binStart[s], tiles = c.binStart[s + 1] - tb;
+    if (tiles == 1) continue;
+    const uint32_t parts = min(8u, div_up(tiles, 8)), per = div_up(tiles, parts);
+    for (uint32_t w = threadIdx.x; w < W; w += kSelectBlock) sBins[w] = bin_init((int)w);
+    sync_block_lds();
+    for (uint32_t i = threadIdx.x; i < W * parts; i += kSelectBlock) {
+      const uint32_t part = i / W, w = i - part * W, k = w & (kBinWords - 1);
+      uint32_t t = part * per;
+      const uint32_t te = min(t + per, tiles);
+      int32_t acc = bin_init((int)w);
+      const int32_t *p = c.partial + (size_t)(tb + t) * W + w;
       auto add = [&](int32_t v) { acc = k < 3 ? min(acc, v) : (k < 6 ? max(acc, v) : acc + v); };
-      uint32_t t = tb;
       for (; t + 8 <= te; t += 8, p += 8 * (size_t)W) {
         int32_t v[8];
 #pragma unroll
@@ -550,7 +557,9 @@ __global__ __launch_bounds__(kBlock) void k_select(Ctx c, int level) {
         for (int u = 0; u < 8; u++) add(v[u]);
       }
       for (; t < te; t++, p += W) add(*p);
-      sBins[w] = acc;
+      if (k < 3) atomicMin(&sBins[w], acc);
+      else if (k < 6) atomicMax(&sBins[w], acc);
+      else atomicAdd(&sBins[w], acc);
     }
     sync_block_lds();
     if (threadIdx.x < kWave) decide_node(c, sBins, c.segs[par][s], s);
@@ -693,7 +702,7 @@ __global__ __launch_bounds__(1024) void k_emit(Ctx c, int level) {
         if (large[side]) {
           v[1]++;
           v[3] += div_up(sz, kTile);
-          v[4] += div_up(sz, kBinTile);
+          v[4] += div_up(sz, c.binTile);
           v[5] += sz;
         } else {
           v[2]++;
@@ -756,7 +765,7 @@ __global__ __launch_bounds__(1024) void k_emit(Ctx c, int level) {
         c.tileStart[li] = ti;
         c.binStart[li] = bi;
         ti += div_up(ce[side] - cb[side], kTile);
-        bi += div_up(ce[side] - cb[side], kBinTile);
+        bi += div_up(ce[side] - cb[side], c.binTile);
         li++;
       } else {
         c.small[smallBase + si] = SmallSeg{cb[side], ce[side], child + side, (uint32_t)(par ^ 1)};
@@ -1285,7 +1294,8 @@ int sah_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T
   const uint32_t numBlocks = div_up(n, kTile);
   c.maxLarge = n / (kSmall + 1) + 2;
   const uint32_t maxTiles = div_up(n, kTile) + c.maxLarge + 1;
-  const uint32_t maxBinTiles = div_up(n, kBinTile) + c.maxLarge + 1;
+  c.binTile = std::max<uint32_t>(kTile, std::min<uint32_t>(kBinTileMax, div_up(div_up(n, 256u), kTile) * kTile));
+  const uint32_t maxBinTiles = div_up(n, c.binTile) + c.maxLarge + 1;
   const size_t binW = 3 * (size_t)numBins * kBinWords;
   const uint32_t maxLevels = 4096;
   CUBQL_CHECK(scr.reserve(&c.items[0], n));
@@ -1356,7 +1366,7 @@ int sah_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T
       k_bin<<<binGrid, kBinBlock, 0, s>>>(c, level);
       prof_end(pb, s, "sah_bin");
       if (pb >= 0) binSlots.push_back({pb, level});
-      k_select<<<selGrid, kBlock, 0, s>>>(c, level);
+      k_select<<<selGrid, kSelectBlock, 0, s>>>(c, level);
       int pp = prof_begin(s);
       k_partition<<<partGrid, kBlock, 0, s>>>(c, level);
       prof_end(pp, s, "sah_partition");
