@@ -1815,7 +1815,9 @@ __global__ __launch_bounds__(kWave) void k_small(Ctx c, int pp) {
 // pairs at loc[2 (b + 1)] and after, which no other node uses.  place[] then
 // gives each pair its number in the order in which one wave would have made it
 // (0xffff: none), for k_wide_emit.  3001 points: 96 us by waves, 30 us so.
-constexpr int kWideBlock = 512;
+// (16 waves up to 2^17 prims, 8 above, where a CU holds several workgroups: 100K
+// points 310 us a build and query with 16, 316 with 8; a build of 1M 553 and 518)
+constexpr uint32_t kWideLarge = 1u << 17;
 // (uniform points, by waves and by workgroups: 1000 203 and 131 us a build, 100K
 // 333 and 262, 700K 418 and 385, 1.5M 515 and 525, 10M 1575 and 1983; boxes of a
 // mesh: 100K 578 and 451, 2M 923 and 912)
@@ -1943,7 +1945,7 @@ __device__ uint32_t wide_number(WideShare &sh, uint32_t m, uint32_t T, uint16_t 
   return r;
 }
 
-template <bool PTS>
+template <bool PTS, int BLOCK>
 __device__ void wide_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, WideShare &sh) {
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   const uint32_t gb = sg.begin, m = sg.end - sg.begin;
@@ -1958,7 +1960,7 @@ __device__ void wide_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, 
     }
     return;
   }
-  for (uint32_t i = tid; i < m; i += kWideBlock) sh.it[0][i] = items[sg.rev ? m - 1 - i : i];
+  for (uint32_t i = tid; i < m; i += BLOCK) sh.it[0][i] = items[sg.rev ? m - 1 - i : i];
   if (tid == 0) {
     const bool split = m > (uint32_t)kWave;
     sh.open[0][0] = wide_pack(0u, m, 0u);
@@ -1973,7 +1975,7 @@ __device__ void wide_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, 
   for (uint32_t cur = 0;; cur ^= 1u) {
     const uint32_t n = sh.numOpen[cur];
     if (!n) break;
-    for (uint32_t t = wave; t < n; t += kWideBlock / kWave) {
+    for (uint32_t t = wave; t < n; t += BLOCK / kWave) {
       const uint32_t f = sh.open[cur][t];
       wide_split<PTS>(c, sh, cur, gb, f & 1023u, f >> 10 & 2047u, f >> 21);
     }
@@ -1982,7 +1984,7 @@ __device__ void wide_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, 
     __syncthreads();
   }
   const uint32_t numUnits = sh.numUnits;
-  for (uint32_t u = wave; u < numUnits; u += kWideBlock / kWave) {
+  for (uint32_t u = wave; u < numUnits; u += BLOCK / kWave) {
     const uint32_t f = sh.unit[u], b = f & 1023u, e = f >> 10 & 2047u, n = e - b;
     const float4 *src = sh.it[f >> 21] + b;
     uint32_t nLocal = 2 * (b + 1);
@@ -2018,22 +2020,23 @@ __device__ void wide_segment(const Ctx &c, const SmallSeg &sg, uint32_t segIdx, 
   uint16_t *place = pair_places(c, sg);
   if (tid == 0) c.smallCount[segIdx] = 1 + 2 * wide_number(sh, m, c.T, place);
   __syncthreads();
-  for (uint32_t u = wave; u < numUnits; u += kWideBlock / kWave) {
+  for (uint32_t u = wave; u < numUnits; u += BLOCK / kWave) {
     const uint32_t f = sh.unit[u], b = f & 1023u, n = (f >> 10 & 2047u) - b;
     for (uint32_t j = lane; j + 1 < n; j += kWave)
       place[b + 1 + j] = j < sh.pairs[b] ? (uint16_t)(sh.base[b] + j) : kNoPair;
   }
 }
 
-__global__ __launch_bounds__(kWideBlock) void k_wide(Ctx c, int pp) {
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_wide(Ctx c, int pp) {
   __shared__ WideShare sh;
   if (c.ctr->numLarge[pp] != 0 || c.ctr->spinFault != 0) return;
   const bool pts = c.ctr->allPoints != 0;
   const uint32_t nSmall = c.ctr->numSmall;
   for (uint32_t w = blockIdx.x; w < nSmall; w += gridDim.x) {
     const SmallSeg sg = c.small[w];
-    if (pts) wide_segment<true>(c, sg, w, sh);
-    else wide_segment<false>(c, sg, w, sh);
+    if (pts) wide_segment<true, BLOCK>(c, sg, w, sh);
+    else wide_segment<false, BLOCK>(c, sg, w, sh);
     __syncthreads();
   }
 }
@@ -2213,6 +2216,8 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
   // always).
   int batch = levels ? std::max(std::min(kPassesPerSync, (levels + 1) / 2 + 1), (levels + 1) / 2) : 0;
   const bool wide = n <= kWideMax;
+  const auto wideKernel = n <= kWideLarge ? k_wide<1024> : k_wide<512>;
+  const int wideBlock = n <= kWideLarge ? 1024 : 512;
   bool firstBatch = true;
   int specPass = -1, smallSlot = -1;
   uint32_t specGrid = 0;
@@ -2242,7 +2247,7 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
       }
       specGrid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(bound, (uint64_t)n + 1));
       smallSlot = prof_begin(s);
-      if (wide) k_wide<<<specGrid, kWideBlock, 0, s>>>(c, pass & 1);
+      if (wide) wideKernel<<<specGrid, wideBlock, 0, s>>>(c, pass & 1);
       else k_small<<<specGrid, kWave, 0, s>>>(c, pass & 1);
       prof_end(smallSlot, s, "sm_small");
       // (status tag beyond every pass's)
@@ -2273,7 +2278,7 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
     // workgroup per segment (the dispatcher balances the uneven segment
     // costs far better than a fixed round-robin over resident waves)
     smallSlot = prof_begin(s);
-    if (wide) k_wide<<<std::max<uint32_t>(1u, numSmall), kWideBlock, 0, s>>>(c, pass & 1);
+    if (wide) wideKernel<<<std::max<uint32_t>(1u, numSmall), wideBlock, 0, s>>>(c, pass & 1);
     else k_small<<<std::max<uint32_t>(1u, numSmall), kWave, 0, s>>>(c, pass & 1);
     prof_end(smallSlot, s, "sm_small");
     k_small_scan<<<std::max<uint32_t>(1u, div_up(numSmall, kCountScanTile)), 1024, 0, s>>>(c, maxPasses + 2, pass & 1);

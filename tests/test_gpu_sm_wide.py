@@ -1,5 +1,6 @@
 """Spatial-median builds whose small nodes are finished by a workgroup each,
-on both sides of the size (2^20 prims) where waves take over: leaves from one
+on both sides of the sizes where the workgroup changes (2^17 prims) and where
+waves take over (2^20): leaves from one
 prim to larger than a segment, pieces of 64 and 65 prims, points, boxes,
 clusters, and copies (one-sided splits all the way down).  The tree equals the
 oracle's, and its nodes are numbered without a gap, children after parents."""
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kind", ["points", "boxes", "clustered", "copies"])
 @pytest.mark.parametrize("n,T", [(1, 1), (64, 8), (65, 1), (65, 64), (257, 70), (1000, 1), (1024, 300), (1025, 4),
-                                 (3001, 8), (3001, 2000), (70000, 3), (1 << 20, 8), ((1 << 20) + 1, 8)])
+                                 (3001, 8), (3001, 2000), (70000, 3), (1 << 17, 8),
+                                 ((1 << 17) + 1, 8), (1 << 20, 8), ((1 << 20) + 1, 8)])
 def test_wide_small_nodes(oracle_mod, kind, n, T):
     import cubql_amd as cq
     print(f"[gpu] median build {kind}, {n} prims, T {T}", flush=True)
