@@ -56,7 +56,25 @@ def test_refit_moved_boxes(cq, n, leaf):
         assert np.array_equal(nodes["lo"][i], lo[i]) and np.array_equal(nodes["hi"][i], hi[i]), i
 
 
-@pytest.mark.parametrize("depth", [1, 2, 300])
+@pytest.mark.parametrize("builder", ["radixBuilder", "rebinRadixBuilder", "sahBuilder"])
+@pytest.mark.parametrize("n", [255, 513, 20001])
+def test_refit_numberings(cq, builder, n):
+    """Spans of nodes that hold whole subtrees, parts of them, or neither."""
+    print(f"[gpu] refit {builder}, {n} boxes", flush=True)
+    rng = np.random.default_rng(n)
+    c = rng.random((n, 3), dtype=np.float32)
+    build = getattr(cq.cuda, builder)
+    bvh = build(torch.from_numpy(np.hstack([c, c])).cuda(), cq.BuildConfig(makeLeafThreshold=1))
+    boxes = np.hstack([c - np.float32(0.3), c + rng.random((n, 3), dtype=np.float32)])
+    cq.refit(bvh, torch.from_numpy(boxes).cuda())
+    torch.cuda.synchronize()
+    nodes, prims = cq.nodes_to_numpy(bvh), bvh.prim_ids_tensor().cpu().numpy().view(np.uint32)
+    lo, hi = _expected(nodes, prims, boxes)
+    for i in lo:
+        assert np.array_equal(nodes["lo"][i], lo[i]) and np.array_equal(nodes["hi"][i], hi[i]), i
+
+
+@pytest.mark.parametrize("depth", [1, 2, 300, 1000])
 def test_refit_chain(cq, depth):
     from test_gpu_deep import _chain
     print(f"[gpu] refit chain of depth {depth}", flush=True)
