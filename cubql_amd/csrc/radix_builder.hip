@@ -280,6 +280,12 @@ __global__ __launch_bounds__(1024) void k_rrefit_top(RCtx c, Node *nodes, const 
   }
 }
 
+// Levels above which the generic climb takes the place of a pass per level.
+// (Clusters, 64 levels and more: 1M prims 4.69 ms a build by levels and 3.90 by
+// the climb, 5M 7.21 and 6.21; uniform, 8 to 16 levels: 1M 0.54 and 0.57, 5M 1.00
+// and 1.15.)
+constexpr int kRefitLevelsMax = 24;
+
 // host: refit levels [0, levels) given their node counts
 static void refit_launch(const RCtx &c, Node *nodes, const uint32_t *primIDs, int levels,
                          const std::vector<uint32_t> &hc, int numCU, hipStream_t s) {
@@ -1518,7 +1524,17 @@ int rebin_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t
   bvh->primIDs = primIDs;
   bvh->numPrims = numValid;
   int rs = prof_begin(s);
-  refit_launch(c, nodes, primIDs, level, hc, numCU, s);
+  if (level > kRefitLevelsMax) {
+    st = refit_tree(bvh, boxes, s, mem);
+    if (st) {
+      mem_free(mem, nodes, s);
+      bvh->nodes = nullptr;
+      bvh->primIDs = nullptr;
+      return fail(st);
+    }
+  } else {
+    refit_launch(c, nodes, primIDs, level, hc, numCU, s);
+  }
   st = hipGetLastError() == hipSuccess ? CUBQL_OK : (set_error("refit launch failed"), CUBQL_ERR_HIP);
   prof_end(rs, s, "refit");
   prof_set(rs, 24.0 * numValid + 64.0 * numNodes, numNodes);
