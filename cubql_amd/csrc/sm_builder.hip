@@ -2096,16 +2096,29 @@ __global__ void k_copy_top(const Node *src, Node *dst, uint32_t n) {
 
 // Bounds of the pass-phase inner nodes, node list by node list (two a
 // pass: a pass's split children before its segments), deepest first.
-__global__ void k_refit_top(Ctx c, Node *nodes, int level) {
+__device__ __forceinline__ void refit_top_node(Node *nodes, uint32_t i) {
+  Node *nd = &nodes[i];
+  const uint64_t off = oc_offset(nd->oc);
+  const Node l = nodes[off], r = nodes[off + 1];
+  for (int d = 0; d < 3; d++) {
+    nd->lo[d] = fminf(l.lo[d], r.lo[d]);
+    nd->hi[d] = fmaxf(l.hi[d], r.hi[d]);
+  }
+}
+__global__ void k_refit_list(Ctx c, Node *nodes, int level) {
   const uint32_t b = c.levelStart[level], e = c.levelStart[level + 1];
-  for (uint32_t i = b + blockIdx.x * blockDim.x + threadIdx.x; i < e; i += gridDim.x * blockDim.x) {
-    Node *nd = &nodes[c.topNodes[i]];
-    uint64_t off = oc_offset(nd->oc);
-    const Node l = nodes[off], r = nodes[off + 1];
-    for (int d = 0; d < 3; d++) {
-      nd->lo[d] = fminf(l.lo[d], r.lo[d]);
-      nd->hi[d] = fmaxf(l.hi[d], r.hi[d]);
-    }
+  for (uint32_t i = b + blockIdx.x * blockDim.x + threadIdx.x; i < e; i += gridDim.x * blockDim.x)
+    refit_top_node(nodes, c.topNodes[i]);
+}
+// Lists [0, lists), of at most 2^(l + 1) nodes each, in one workgroup, whose
+// barriers order them: a launch a list takes longer than its work (100K boxes of a
+// mesh, eight lists: 423 us a build with launches, 381 so).
+constexpr int kRefitLists = 12;
+__global__ __launch_bounds__(1024) void k_refit_top(Ctx c, Node *nodes, int lists) {
+  for (int l = lists - 1; l >= 0; l--) {
+    const uint32_t e = c.levelStart[l + 1];
+    for (uint32_t i = c.levelStart[l] + threadIdx.x; i < e; i += 1024) refit_top_node(nodes, c.topNodes[i]);
+    __syncthreads();
   }
 }
 
@@ -2316,8 +2329,10 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
     else if (numSmall) k_small_emit<<<div_up(numSmall, 4), 256, 0, s>>>(c, nodes);
     // (point input: the emit already wrote the pass-phase boxes; two node
     // lists a pass, each refit after the deeper ones)
-    if (numTop && !hc0.allPoints)
-      for (int l = 2 * pass - 1; l >= 0; l--) k_refit_top<<<64, 256, 0, s>>>(c, nodes, l);
+    if (numTop && !hc0.allPoints) {
+      for (int l = 2 * pass - 1; l >= kRefitLists; l--) k_refit_list<<<64, 256, 0, s>>>(c, nodes, l);
+      k_refit_top<<<1, 1024, 0, s>>>(c, nodes, std::min(2 * pass, kRefitLists));
+    }
     if (hipGetLastError() != hipSuccess) {
       mem_free(mem, nodes, s);
       return fail((set_error("emit launch failed"), CUBQL_ERR_HIP));

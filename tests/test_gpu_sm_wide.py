@@ -11,7 +11,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind", ["points", "boxes", "clustered", "copies"])
+@pytest.mark.parametrize("kind", ["points", "boxes", "clustered", "clustered boxes", "copies"])
 @pytest.mark.parametrize("n,T", [(1, 1), (64, 8), (65, 1), (65, 64), (257, 70), (1000, 1), (1024, 300), (1025, 4),
                                  (3001, 8), (3001, 2000), (70000, 3), (1 << 17, 8),
                                  ((1 << 17) + 1, 8), (1 << 20, 8), ((1 << 20) + 1, 8)])
@@ -23,9 +23,12 @@ def test_wide_small_nodes(oracle_mod, kind, n, T):
     half = np.zeros_like(P)
     if kind == "boxes":
         half = rng.random((n, 3), dtype=np.float32) * np.float32(0.01)
-    elif kind == "clustered":
+    elif kind.startswith("clustered"):
+        # (more lists of inner nodes than one workgroup takes)
         P = P ** 8
         P[::97] *= 1000
+        if kind == "clustered boxes":
+            half = P * np.float32(0.01)
     elif kind == "copies":
         P = P[rng.integers(0, max(1, n // 200), n)]
     B = np.concatenate([P - half, P + half], axis=1).astype(np.float32)
