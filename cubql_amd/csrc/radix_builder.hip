@@ -24,7 +24,6 @@
 #include "radix_sort.h"
 #include "refit.h"
 
-#include <vector>
 
 namespace cubql {
 namespace rb {
@@ -288,7 +287,7 @@ constexpr int kRefitLevelsMax = 24;
 
 // host: refit levels [0, levels) given their node counts
 static void refit_launch(const RCtx &c, Node *nodes, const uint32_t *primIDs, int levels,
-                         const std::vector<uint32_t> &hc, int numCU, hipStream_t s) {
+                         const uint32_t *hc, int numCU, hipStream_t s) {
   int top = 0;  // levels [0, top) are narrow
   while (top < levels && hc[C_LEVEL0 + top] <= kRefitTopMax) top++;
   for (int l = levels - 1; l >= top; l--) {
@@ -633,10 +632,12 @@ __global__ void k_karras_info(const K *keys, const uint32_t *nPtr, const uint32_
   info[M_SPIN] = *spin;
 }
 
-// pinned host mirror of those words
+// pinned host mirror of those words, or of the counters
+constexpr size_t kCtrWords = C_LSTART0 + kMaxLevels + 8;
+static_assert((size_t)M_WORDS <= kCtrWords, "one buffer for both");
 static uint32_t *host_words() {
   static thread_local uint32_t *p = nullptr;
-  if (!p && hipHostMalloc((void **)&p, M_WORDS * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) p = nullptr;
+  if (!p && hipHostMalloc((void **)&p, kCtrWords * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) p = nullptr;
   return p;
 }
 
@@ -1466,7 +1467,8 @@ int rebin_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t
   const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(div_up(n, kBlock), (uint32_t)numCU * 8));
   int jobBits = 1;
   while ((1ull << jobBits) < (uint64_t)maxJobs) jobBits++;
-  std::vector<uint32_t> hc(C_LSTART0 + kMaxLevels + 8);
+  uint32_t *hc = host_words();
+  if (!hc) return fail((set_error("hipHostMalloc failed"), CUBQL_ERR_HIP));
   int level = 0, rounds = 0;
   int hs = prof_begin(s);
   while (true) {
@@ -1474,7 +1476,7 @@ int rebin_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t
     for (int i = 0; i < kLevelsPerSync && level < kMaxLevels; i++, level++)
       k_rlevel_rebin<<<grid, kBlock, 0, s>>>(c, keys, level);
     if (hipGetLastError() != hipSuccess) return fail((set_error("rebin level launch failed"), CUBQL_ERR_HIP));
-    if (hipMemcpyAsync(hc.data(), c.ctr, sizeof(uint32_t) * hc.size(), hipMemcpyDeviceToHost, s) != hipSuccess ||
+    if (hipMemcpyAsync(hc, c.ctr, sizeof(uint32_t) * kCtrWords, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return fail((set_error("rebin level sync failed"), CUBQL_ERR_HIP));
     int L = -1;
@@ -1514,7 +1516,7 @@ int rebin_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t
     k_thread_scan<<<div_up(numSmall, kCountScanTile), 1024, 0, s>>>(c);
   }
   if (hipGetLastError() != hipSuccess) return fail((set_error("thread phase launch failed"), CUBQL_ERR_HIP));
-  if (hipMemcpyAsync(hc.data(), c.ctr, sizeof(uint32_t) * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
+  if (hipMemcpyAsync(hc, c.ctr, sizeof(uint32_t) * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail((set_error("rebin sync failed"), CUBQL_ERR_HIP));
   if (hc[C_SPIN]) return fail((set_error("rebin build: a look-back wait exceeded its bound"), CUBQL_ERR_INTERNAL));
