@@ -22,8 +22,9 @@
 //     reduces the partials and one wave evaluates all 3 x numBins candidate
 //     planes at once (prefix/suffix unions as wave scans); the partition is
 //     a single-pass decoupled look-back over 1024-prim tiles;
-//   * nodes of <= 256 prims are finished by one wave each in LDS, which also
-//     computes their boxes, so no refit pass is needed;
+//   * nodes of <= 256 prims are finished by one wave each in LDS, subtrees of
+//     <= 16 prims four at a time; it also computes their boxes, so no refit
+//     pass is needed;
 //   * the level loop runs on the device; the host checks for completion every
 //     few levels.
 #include "block_ops.h"

@@ -19,7 +19,8 @@
 //     right reversed, per level), using decoupled look-back over 2048-item
 //     tiles; ranges that come out reversed carry a flag;
 //   * nodes of <= kMedium prims are finished by one wavefront each (pieces
-//     of <= kSmall prims in LDS), which also computes all their boxes;
+//     of <= kSmall prims in LDS), or in builds of up to kWideMax prims by a
+//     workgroup each, which also computes all their boxes;
 //   * the pass loop runs on the device: kernels read their work counts from
 //     device memory, the host checks for completion once per batch of
 //     passes.
