@@ -11,9 +11,9 @@
 //   4. top-down hierarchy: a range of <= T prims is a leaf, a range of equal
 //      keys is split in the middle, otherwise at the first key that has the
 //      highest differing bit of its first and last key set (findSplit,
-//      radix.h:446-482; createNodes radix.h:501-570), one launch per level,
-//      children allocated with one atomic per workgroup;
-//   5. exact bottom-up refit (refit.hip).
+//      radix.h:446-482; createNodes radix.h:501-570), found for every node at
+//      once (k_karras) and numbered by a scan;
+//   5. exact boxes from the leaves up (k_karras_climb).
 // 63-bit keys (21 bits per axis) are the reference default; 30-bit keys
 // (10 bits per axis) are its radix.h:34-38 variant.
 #include "block_ops.h"
