@@ -4,11 +4,11 @@
 // per thread (traversal/fixedBoxQuery.h:42-160, 215-230) with a per-prim
 // test of the prim's box against the query box: for every query box, the
 // prims whose boxes overlap it (closed boxes, math/box.h:208-212), in the
-// traversal's order (depth first, first child / lowest slot first).  One
+// traversal's order (depth first, first child / lowest slot first).  A
 // query per lane; binary and wide (W = 4, 8) trees.  Queries whose stack
 // would overflow rerun with a deeper one.
 //
-// Batches that are large for their tree (binary) run in spatial order
+// Large batches (kWalkMin), over a binary tree, run in spatial order
 // (query_order.h), a wave of queries walking together, and read leaf prims
 // from a copy of the prim boxes in primID-slot order.  1M boxes against
 // themselves, leaves of 4: 1305 us with one query per lane in input order, on
@@ -25,6 +25,10 @@
 
 namespace cubql {
 namespace bq {
+
+// batches below this size walk the tree a query per lane, in input order
+constexpr uint32_t kWalkMin = 3u << 17;
+static_assert(kWalkMin >= kQueryOrderMin, "the walk takes ordered queries");
 
 // prim boxes of a leaf that are read at once
 constexpr int kLeafBoxes = 4;
@@ -65,9 +69,10 @@ __device__ __forceinline__ bool query_one(const BVH &bvh, const cubql_box3f *pri
   return cubql_dev::for_each_leaf_in_box<STACK>(bvh, lo, hi, leaf);
 }
 
-// prim boxes in primID-slot order: lo, hi.x | hi.y, hi.z, primID
+// prim boxes in primID-slot order: lo, hi.x | hi.y, hi.z, primID; clears *ovf
 __global__ __launch_bounds__(256) void k_slot_boxes(const uint32_t *primIDs, uint32_t numPrims,
-                                                    const cubql_box3f *primBoxes, float4 *sboxes) {
+                                                    const cubql_box3f *primBoxes, float4 *sboxes, Overflow *ovf) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ovf = Overflow{0u, 0u};
   for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < numPrims; t += gridDim.x * 256) {
     const uint32_t i = primIDs[t];
     float lo[3], hi[3];
@@ -236,27 +241,35 @@ int run(const BVH &bvh, const cubql_box3f *primBoxes, const cubql_box3f *queries
   uint32_t *ovfList = nullptr;
   CUBQL_CHECK(scr.alloc(&ovf, 1));
   CUBQL_CHECK(scr.alloc(&ovfList, nq));
-  CUBQL_CHECK(fill_u32((uint32_t *)ovf, 0u, 2, s));
   const uint32_t *order = nullptr;
   float4 *sboxes = nullptr;
   if constexpr (std::is_same<BVH, cubql_bvh3f>::value) {
     // The shared walk pays while a wave's queries overlap mostly the same
-    // nodes, that is while the queries are about as dense as the prims.  1M
-    // prims, query boxes of the prims' size, us before and now: 1M queries
-    // 1262 / 666, 262144 387 / 484, 131072 292 / 551; with boxes six times as
-    // long 21314 / 2583, 5100 / 1779 and 3098 / 2050.
-    if (nq >= kQueryOrderMin && bvh.numPrims && (uint64_t)nq * 2 >= bvh.numPrims) {
+    // nodes, that is while the queries are about as dense as the prims, and once
+    // the batch outweighs the order and the copy (60 to 70 us).  Batches against
+    // themselves, us without the walk / with it:
+    //              140000      262144      300000      400000      1000000
+    //   uniform    275 / 291   356 / 340   407 / 340   588 / 373   1262 / 666
+    //   plane      137 / 178   179 / 198   209 / 211   289 / 226    657 / 388
+    //   Gaussian   159 / 200   202 / 224   226 / 231   279 / 261    591 / 435
+    //   sphere     128 / 195   172 / 211   195 / 227   270 / 247    597 / 387
+    //   (leaves of 4; uniform boxes three times as long: 2165 / 800 and 5414 / 1057 at
+    //   140000 and 400000; boxes that overlap next to nothing, a hundredth as long:
+    //   65 / 128 and 135 / 160, in a sphere 63 / 147 and 133 / 194)
+    // and 1M prims with half as many queries: uniform 770 / 544, sphere 317 / 319.
+    if (nq >= kWalkMin && bvh.numPrims && (uint64_t)nq * 2 >= bvh.numPrims) {
       char *w = nullptr;
       CUBQL_CHECK(scr.alloc(&w, query_order_ws_bytes(nq)));
       CUBQL_CHECK(scr.alloc(&sboxes, 2 * ((size_t)bvh.numPrims + bq::kLeafBoxes)));
       CUBQL_CHECK(query_order_ws(&bvh.nodes[0].bounds, &bvh, {(const float *)queries, nq, true}, s, w, &order));
     }
   }
+  if (!order) CUBQL_CHECK(fill_u32((uint32_t *)ovf, 0u, 2, s));
   int ps = prof_begin(s);
   if (order) {
     if constexpr (std::is_same<BVH, cubql_bvh3f>::value) {
       k_slot_boxes<<<std::max(1u, std::min(div_up(bvh.numPrims, 256u), 2048u)), 256, 0, s>>>(
-          bvh.primIDs, bvh.numPrims, primBoxes, sboxes);
+          bvh.primIDs, bvh.numPrims, primBoxes, sboxes, ovf);
       k_box_query_wave<<<div_up(nq, kBlock), kBlock, 0, s>>>(bvh, sboxes, queries, nq, outIDs ? maxOut : 0u,
                                                                 outIDs, counts, ovf, ovfList, order);
     }

@@ -37,9 +37,12 @@ size_t radix_sort_ws_bytes(uint32_t nMax, int keyBits);
 int radix_sort_pairs_ws_u32(uint32_t *kA, uint32_t *vA, uint32_t *kB, uint32_t *vB,
                             const uint32_t *nDev, uint32_t nMax, int keyBits, hipStream_t s,
                             void *ws, uint32_t **kRes, uint32_t **vRes);
-// The same with the values 0, 1, 2, ... (vA's contents are not read).
+// The same with the values 0, 1, 2, ... (vA's contents are not read).  skipLow: a
+// device word; where it is not 0, the low byte is not sorted by and the keys are
+// those in kB.
 int radix_sort_iota_ws_u32(uint32_t *kA, uint32_t *vA, uint32_t *kB, uint32_t *vB, const uint32_t *nDev,
-                           uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint32_t **kRes, uint32_t **vRes);
+                           uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint32_t **kRes, uint32_t **vRes,
+                           const uint32_t *skipLow = nullptr);
 int radix_sort_pairs_ws_u64(uint64_t *kA, uint32_t *vA, uint64_t *kB, uint32_t *vB,
                             const uint32_t *nDev, uint32_t nMax, int keyBits, hipStream_t s,
                             void *ws, uint64_t **kRes, uint32_t **vRes);

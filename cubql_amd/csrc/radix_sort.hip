@@ -28,13 +28,15 @@ __device__ __forceinline__ uint64_t st_word(uint32_t tag, uint32_t flag, uint32_
 }
 
 // Digit counts of every pass: a sub-histogram per wave in LDS, then one
-// global atomic per digit, pass and workgroup.
+// global atomic per digit, pass and workgroup.  skipLow: as in radix_sort.h.
 constexpr int kHistBlock = 256;
 constexpr int kHistWaves = kHistBlock / kWave;
 template <typename K>
-__global__ __launch_bounds__(kHistBlock) void k_hist(const K *keys, const uint32_t *nPtr, int passes,
-                                                     uint32_t *digitCount) {
+__global__ __launch_bounds__(kHistBlock) void k_hist(const K *keys, const K *keysB, const uint32_t *skipLow,
+                                                     const uint32_t *nPtr, int passes, uint32_t *digitCount) {
   extern __shared__ uint32_t h[];  // [kHistWaves][passes][kDigits]
+  const bool skip = skipLow && *skipLow;
+  if (skip) keys = keysB;
   const uint32_t n = *nPtr;
   const int words = passes * (int)kDigits;
   for (int i = threadIdx.x; i < kHistWaves * words; i += kHistBlock) h[i] = 0;
@@ -52,7 +54,7 @@ __global__ __launch_bounds__(kHistBlock) void k_hist(const K *keys, const uint32
 #pragma unroll
     for (int u = 0; u < U; u++) {
       if (i0 + u * kHistBlock < n)
-        for (int p = 0; p < passes; p++) atomicAdd(&hw[p * kDigits + ((uint32_t)(key[u] >> (8 * p)) & 255u)], 1u);
+        for (int p = skip ? 1 : 0; p < passes; p++) atomicAdd(&hw[p * kDigits + ((uint32_t)(key[u] >> (8 * p)) & 255u)], 1u);
     }
   }
   __syncthreads();
@@ -75,7 +77,8 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin,
                                                               K *__restrict__ kout, uint32_t *__restrict__ vout,
                                                               const uint32_t *nPtr, int shift, uint32_t tag,
                                                               const uint32_t *digitCount, uint64_t *status,
-                                                              uint32_t *ticket, uint32_t *err) {
+                                                              uint32_t *ticket, uint32_t *err,
+                                                              const uint32_t *skipLow) {
   constexpr int BLOCK = kBlock, NW = BLOCK / kWave;
   constexpr uint32_t TILE = BLOCK * ITEMS;
   static_assert(BLOCK >= (int)kDigits, "one thread per digit");
@@ -86,6 +89,8 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin,
   __shared__ uint32_t sTile;
   K *const sK = reinterpret_cast<K *>(sBuf);
   uint32_t *const sV = reinterpret_cast<uint32_t *>(sBuf);
+  const bool skip = skipLow && *skipLow;
+  if (skip && shift == 0) return;
   const uint32_t n = *nPtr;
   const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
   if (threadIdx.x == 0) sTile = atomicAdd(ticket, 1u);
@@ -105,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const K *__restrict__ kin,
 #pragma unroll
   for (int k = 0; k < ITEMS; k++) {
     const uint32_t i = tileBase + li0 + k * kWave;
-    val[k] = li0 + k * kWave < tileN ? (vin ? vin[i] : i) : 0u;
+    val[k] = li0 + k * kWave < tileN ? (vin && !skip ? vin[i] : i) : 0u;
   }
   uint32_t tot;
   const uint32_t digitBase = block_excl_scan<BLOCK, true>(dcount, ss[0], &tot);
@@ -215,7 +220,7 @@ size_t sort_ws_bytes(uint32_t nMax, int keyBits) {
 template <typename K>
 int sort_pairs_ws(K *kA, uint32_t *vA, K *kB, uint32_t *vB, const uint32_t *nDev, uint32_t nMax,
                   int keyBits, hipStream_t s, void *ws, K **kRes, uint32_t **vRes, uint32_t *err = nullptr,
-                  bool iota = false) {
+                  bool iota = false, const uint32_t *skipLow = nullptr) {
   const int passes = (keyBits + 7) / 8;
   const bool small = nMax < kSmallSort;
   const uint32_t maxTiles = std::max<uint32_t>(1u, div_up(nMax, kBlock * (small ? kSmallItems : kLargeItems<K>)));
@@ -225,14 +230,16 @@ int sort_pairs_ws(K *kA, uint32_t *vA, K *kB, uint32_t *vB, const uint32_t *nDev
   CUBQL_CHECK(fill_u32((uint32_t *)status, 0u, (size_t)maxTiles * kDigits * 2 + (size_t)passes * kDigits + 16, s));
   // (two workgroups a CU: the global atomics of more would queue up)
   const uint32_t histBlocks = std::max(1u, std::min(div_up(nMax, 4096), 512u));
-  k_hist<K><<<histBlocks, kHistBlock, (size_t)kHistWaves * passes * kDigits * 4, s>>>(kA, nDev, passes, digitCount);
+  k_hist<K><<<histBlocks, kHistBlock, (size_t)kHistWaves * passes * kDigits * 4, s>>>(kA, kB, skipLow, nDev, passes,
+                                                                                              digitCount);
   K *ki = kA, *ko = kB;
   uint32_t *vi = vA, *vo = vB;
   for (int p = 0; p < passes; p++) {
     int ps = prof_begin(s);
     const auto pass = small ? k_onesweep<K, kSmallItems> : k_onesweep<K, kLargeItems<K>>;
     pass<<<maxTiles, kBlock, 0, s>>>(ki, iota && p == 0 ? nullptr : vi, ko, vo, nDev, 8 * p, (uint32_t)(p + 1),
-                                     digitCount + p * kDigits, status, tickets + p, err);
+                                     digitCount + p * kDigits, status, tickets + p, err,
+                                     p < 2 ? skipLow : nullptr);
     prof_end(ps, s, "radix_onesweep");
     prof_set(ps, (double)nMax * 2.0 * (sizeof(K) + 4), nMax);
     std::swap(ki, ko);
@@ -263,8 +270,9 @@ int radix_sort_pairs_ws_u32(uint32_t *kA, uint32_t *vA, uint32_t *kB, uint32_t *
   return rs::sort_pairs_ws<uint32_t>(kA, vA, kB, vB, nDev, nMax, keyBits, s, ws, kRes, vRes);
 }
 int radix_sort_iota_ws_u32(uint32_t *kA, uint32_t *vA, uint32_t *kB, uint32_t *vB, const uint32_t *nDev,
-                           uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint32_t **kRes, uint32_t **vRes) {
-  return rs::sort_pairs_ws<uint32_t>(kA, vA, kB, vB, nDev, nMax, keyBits, s, ws, kRes, vRes, nullptr, true);
+                           uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint32_t **kRes, uint32_t **vRes,
+                           const uint32_t *skipLow) {
+  return rs::sort_pairs_ws<uint32_t>(kA, vA, kB, vB, nDev, nMax, keyBits, s, ws, kRes, vRes, nullptr, true, skipLow);
 }
 int radix_sort_pairs_ws_u64(uint64_t *kA, uint32_t *vA, uint64_t *kB, uint32_t *vB, const uint32_t *nDev,
                             uint32_t nMax, int keyBits, hipStream_t s, void *ws, uint64_t **kRes,
