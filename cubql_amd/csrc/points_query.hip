@@ -108,7 +108,9 @@ constexpr int kFcpLeafLanes = 24;
 // Closest points over a binary tree: a wave per qpw queries (wave_closest.h).
 // 10M queries of 10M points: 3.70 ms and 0.13 ms of reruns with one query per
 // lane on an 8-entry LDS stack, 1.47 ms here, bound by VALU issue.
-// Queries that lose a task to a full queue go to the deep kernel.
+// Queries that lose a task to a full queue run again in their wave, as in the
+// batched kernel: 3000 equal points, leaves of 16, 200K queries 4.37 ms with the
+// deep kernel for them, 1.02 so; 300K clustered queries 711 and 353 us.
 template <bool kSorted>
 __global__ __launch_bounds__(kBlock) void k_fcp(cubql_bvh3f bvh, const float *points, const float4 *spts,
                                                 const float *queries, uint32_t nq, uint32_t qpw, float sqrMax,
@@ -124,12 +126,28 @@ __global__ __launch_bounds__(kBlock) void k_fcp(cubql_bvh3f bvh, const float *po
   float3 q = make_float3(0.f, 0.f, 0.f);
   if (live) q = load_pt(queries, qi);
   const unsigned long long none = closest_none(sqrMax);
-  bool failed;
-  const unsigned long long best =
-      wave_closest<kFcpLeafLanes>(tasks[wave], bvh.nodes, live, bvh.nodes[0].offsetAndCountBits, q.x, q.y, q.z, none,
-                   LeafPoints<kSorted>{bvh.primIDs, points, spts}, &failed);
+  const uint64_t root = bvh.nodes[0].offsetAndCountBits;
+  unsigned long long best = none;
+  // Queries that lost a task run again, eight at a time and then alone (the
+  // queue holds more of each), and last in the deep kernel.
+  uint64_t lost = 0, todo = __ballot(live);
+  for (uint32_t together = kWave; todo; together /= 8) {
+    uint64_t again = 0;
+    while (todo) {
+      const bool on = ((todo >> lane) & 1u) && mbcnt(todo) < together;
+      bool failed;
+      const unsigned long long k =
+          wave_closest<kFcpLeafLanes>(tasks[wave], bvh.nodes, on, root, q.x, q.y, q.z, none,
+                                      LeafPoints<kSorted>{bvh.primIDs, points, spts}, &failed);
+      todo &= ~__ballot(on);
+      again |= __ballot(on && failed);
+      if (on) best = k;
+    }
+    if (together == 1) lost = again;
+    else todo = again;
+  }
   if (!live) return;
-  if (failed) {
+  if ((lost >> lane) & 1u) {
     ovfList[atomicAdd(&ovf->count, 1u)] = qi;
     return;
   }
