@@ -1538,8 +1538,11 @@ int rebin_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t
   bvh->primIDs = primIDs;
   bvh->numPrims = numValid;
   int rs = prof_begin(s);
-  if (level > kRefitLevelsMax) {
-    st = refit_tree(bvh, boxes, s, mem);
+  if (level > kRefitLevelsMax && numNodes) {
+    // (on the thread phase's nodes, which have been emitted: 64 n bytes, 8 to a node
+    // are needed)
+    uint32_t *const words = reinterpret_cast<uint32_t *>(c.loc);
+    st = refit_tree_ws(bvh, boxes, s, words, words + numNodes);
     if (st) {
       mem_free(mem, nodes, s);
       bvh->nodes = nullptr;

@@ -6,6 +6,8 @@ namespace cubql {
 // Recomputes every reachable node box of *bvh from the prim boxes.
 int refit_tree(cubql_bvh3f *bvh, const cubql_box3f *boxes, hipStream_t s,
                const cubql_mem_resource *mem);
+// The same on two arrays of numNodes words (numNodes > 0).
+int refit_tree_ws(cubql_bvh3f *bvh, const cubql_box3f *boxes, hipStream_t s, uint32_t *parent, uint32_t *arrive);
 // Spatial-median builder (sm_builder.hip); T = leaf threshold (>= 1).
 int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, hipStream_t s,
              const cubql_mem_resource *mem);

@@ -162,6 +162,15 @@ __global__ __launch_bounds__(kSpan) void k_refit(Node *nodes, uint32_t numNodes,
 
 }  // namespace rf
 
+int refit_tree_ws(cubql_bvh3f *bvh, const cubql_box3f *boxes, hipStream_t s, uint32_t *parent, uint32_t *arrive) {
+  uint32_t g = std::min<uint32_t>(div_up(bvh->numNodes, 256), 8192);
+  rf::k_parents<<<g, 256, 0, s>>>((const Node *)bvh->nodes, bvh->numNodes, parent, arrive);
+  rf::k_refit<<<div_up(bvh->numNodes, rf::kSpan), rf::kSpan, 0, s>>>((Node *)bvh->nodes, bvh->numNodes, bvh->primIDs,
+                                                                     boxes, parent, arrive);
+  CUBQL_LAUNCH_CHECK();
+  return CUBQL_OK;
+}
+
 int refit_tree(cubql_bvh3f *bvh, const cubql_box3f *boxes, hipStream_t s,
                const cubql_mem_resource *mem) {
   if (bvh->numNodes == 0) return CUBQL_OK;
@@ -169,11 +178,7 @@ int refit_tree(cubql_bvh3f *bvh, const cubql_box3f *boxes, hipStream_t s,
   uint32_t *parent = nullptr, *arrive = nullptr;
   CUBQL_CHECK(scr.alloc(&parent, bvh->numNodes));
   CUBQL_CHECK(scr.alloc(&arrive, bvh->numNodes));
-  uint32_t g = std::min<uint32_t>(div_up(bvh->numNodes, 256), 8192);
-  rf::k_parents<<<g, 256, 0, s>>>((const Node *)bvh->nodes, bvh->numNodes, parent, arrive);
-  rf::k_refit<<<div_up(bvh->numNodes, rf::kSpan), rf::kSpan, 0, s>>>((Node *)bvh->nodes, bvh->numNodes, bvh->primIDs, boxes, parent, arrive);
-  CUBQL_LAUNCH_CHECK();
-  return CUBQL_OK;
+  return refit_tree_ws(bvh, boxes, s, parent, arrive);
 }
 
 }  // namespace cubql
