@@ -176,8 +176,7 @@ def bench_batched(cq, dev, num_clouds: int, plain_budget_s: float, tune: bool):
     torch.cuda.synchronize()
     maxc = int(max(ss.max(), ts.max()))
     if tune:
-        # stack depths 8 and 16 run the traversal stack in LDS, 64 in scratch
-        cands = [(T, b, st) for T in (4, 8, 16) for b in (128, 256) for st in (8, 16, 64)]
+        cands = [(T, b, 64) for T in (4, 8, 16) for b in (128, 256)]
         params, times = tune_batch(src, so, tgt, to, cands, reps=2, max_cloud_size=maxc)
     else:
         params, times = cq.BatchParams(8, 256, 64, maxc), {}
@@ -221,8 +220,7 @@ def bench_batched(cq, dev, num_clouds: int, plain_budget_s: float, tune: bool):
     plain_ms = plain_ms_done if done == num_clouds else plain_ms_done / max(done / num_clouds, 1e-9)
     return {
         "clouds": num_clouds, "src_points": int(so_h[-1]), "tgt_points": int(to_h[-1]),
-        "params": {"leafSize": params.leafSize, "blockSize": params.blockSize,
-                   "stackDepth": params.stackDepth},
+        "params": {"leafSize": params.leafSize, "blockSize": params.blockSize},
         "tuning_ms": times,
         "batched_ms": batched_ms, "batched_mpoints_s": (so_h[-1] + to_h[-1]) / batched_ms / 1e3,
         "plain_ms": plain_ms, "plain_clouds_timed": done,

@@ -78,7 +78,8 @@ _FREE_CB = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_void_p)
 
 
 class BatchParams(C.Structure):
-    """cubql_batch_params: leafSize, blockSize (64/128/256), stackDepth (8/16/32/64), maxCloudSize."""
+    """cubql_batch_params: leafSize, blockSize (64/128/256), and stackDepth (8/16/32/64) and
+    maxCloudSize, which have no effect."""
     _fields_ = [("leafSize", C.c_int), ("blockSize", C.c_int), ("stackDepth", C.c_int),
                 ("maxCloudSize", C.c_uint32)]
 

@@ -1,4 +1,4 @@
-"""Autotuner for the batched path: leaf size, query block size, stack depth.
+"""Autotuner for the batched path: leaf size and query block size.
 
 Every candidate computes the same nearest neighbours and distances (the
 lowest-index rule makes results independent of the tree shape), so the
@@ -17,7 +17,8 @@ import torch
 
 from . import BatchParams, ChamferBatch
 
-DEFAULT_CANDIDATES = [(T, b, s) for T in (2, 4, 8, 16) for b in (64, 128, 256) for s in (32, 64)]
+# (leafSize, blockSize, stackDepth); the stack depth has no effect
+DEFAULT_CANDIDATES = [(T, b, 64) for T in (2, 4, 8, 16) for b in (64, 128, 256)]
 _cache = {}
 
 
