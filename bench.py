@@ -273,20 +273,39 @@ def _kernel_ms(cq, name, fn, reps=3):
     return st["ms"] / st["launches"] if st and st["launches"] else None
 
 
-def query_roofline(cq, stats, kernel_ms, io_bytes, prim_bytes, kernel):
-    """Visited-bytes roofline of a query kernel: per query, `io_bytes` of
-    query in and result out, the node bytes the traversal loaded (64 per
-    child pair expanded, 32 per node popped) and `prim_bytes` per prim
-    tested, all counted by an instrumented run of the same queries."""
+def lane_counts(stats, kernel_ms, io_bytes, prim_bytes, kernel):
+    """Per query of a batch: `io_bytes` of query in and result out, the node
+    bytes loaded (64 per child pair expanded, 32 per node popped) and the prims
+    tested by one lane walking alone, from an instrumented run; and the time of
+    the kernel."""
     nq = stats["queries"]
-    total = nq * io_bytes + stats["node_bytes"] + stats["prims"] * prim_bytes
+    return {"kernel": kernel, "avg_launch_ms": kernel_ms, "io_bytes_per_query": io_bytes,
+            "node_bytes_per_query": stats["node_bytes"] / nq, "prims_per_query": stats["prims"] / nq,
+            "prim_bytes": prim_bytes}
+
+
+def points_counts(stats, kernel_ms, io_bytes, prim_bytes, kernel):
+    """The same for a point kernel, whose lanes share their wave's subtrees and
+    read common node pairs once: it does not load what one lane alone would, so
+    the bytes and its time make no rate."""
+    return {**lane_counts(stats, kernel_ms, io_bytes, prim_bytes, kernel),
+            "note": "counts of one lane walking alone; the timed kernel shares a wave's subtrees, visits other "
+                    "nodes and is bound by instruction issue, so no rate is formed of the two"}
+
+
+def query_roofline(stats, kernel_ms, io_bytes, prim_bytes, kernel):
+    """Visited-bytes roofline of a kernel whose lanes walk as in the
+    instrumented run (triangles)."""
+    c = lane_counts(stats, kernel_ms, io_bytes, prim_bytes, kernel)
+    nq = stats["queries"]
+    total = nq * (io_bytes + c["node_bytes_per_query"] + c["prims_per_query"] * prim_bytes)
     gbs = total / (kernel_ms * 1e-3) / 1e9
     return {"bound": "hbm", "kernel": kernel, "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": gbs / HBM_PEAK_GBS, "avg_launch_ms": kernel_ms, "bytes_per_launch": total,
-            "bytes_per_query": total / nq, "node_bytes_per_query": stats["node_bytes"] / nq,
-            "prims_per_query": stats["prims"] / nq,
+            "bytes_per_query": total / nq, "node_bytes_per_query": c["node_bytes_per_query"],
+            "prims_per_query": c["prims_per_query"],
             "bytes_model": f"{io_bytes} B query+result, node bytes loaded, {prim_bytes} B per prim tested",
-            "note": "visited bytes, not HBM traffic: neighbouring (Morton-ordered) queries load the same "
+            "note": "visited bytes, not HBM traffic: neighbouring (spatially ordered) queries load the same "
                     "nodes, most of them from L2 or the MALL, so frac can pass 1"}
 
 
@@ -324,7 +343,7 @@ def bench_triangles(cq, dev, reps: int):
     stats = cq.query_stats(bvh, dQ, tris=dF, verts=dV)
     # query 12 B in, id + distance 8 B out; per triangle 4 B primID,
     # 12 B index triple and 3 x 12 B vertices
-    roof = query_roofline(cq, stats, kms, 20, 52, "fcp_triangles") if kms else None
+    roof = query_roofline(stats, kms, 20, 52, "fcp_triangles") if kms else None
     ids = out["r"][0]
     g = torch.ones(len(Q), device=dev)
     gq = torch.empty_like(dQ)
@@ -360,7 +379,7 @@ def bench_mixture(cq, dev, reps: int):
     kms = _kernel_ms(cq, "knn_points", fwd)
     stats = cq.query_stats(bvh, Q, data=P, k=16)
     # query 12 B in, 16 x (id + distance) + count out; 16 B per point tested
-    roof = query_roofline(cq, stats, kms, 12 + 8 * 16 + 4, 16, "knn_points<16>") if kms else None
+    counts = points_counts(stats, kms, 12 + 8 * 16 + 4, 16, "knn_points<16>") if kms else None
     ids = out["r"][0]
     g = torch.full((len(Q), 16), 1.0 / (len(Q) * 16), device=dev)
     gq = torch.empty_like(Q)
@@ -374,7 +393,7 @@ def bench_mixture(cq, dev, reps: int):
            "num_nodes": int(bvh.numNodes),
            "knn_ms": knn_ms, "knn_mqueries_s": len(Q) / knn_ms / 1e3,
            "backward_ms": bwd_ms, "fwd_bwd_mqueries_s": len(Q) / (knn_ms + bwd_ms) / 1e3,
-           "knn_roofline": roof}
+           "knn_counts": counts}
     bvh.free()
     return res
 
@@ -465,7 +484,7 @@ def bench_radix(cq, boxes, cfg, mem, N, steps, kern):
 
 def bench_queries(cq, P, Q, boxes, cfg, mem, N, nq, nk, build_ms):
     """10M closest-point and 1M kNN (k=8) queries on one tree, their
-    visited-bytes rooflines, and the whole build against HBM peak."""
+    traversal counts, and the whole build against HBM peak."""
     import torch
     bvh = cq.gpuBuilder(boxes, cfg, mem=mem)
     Qf, Qk = Q[:nq], Q[:nk]
@@ -473,10 +492,10 @@ def bench_queries(cq, P, Q, boxes, cfg, mem, N, nq, nk, build_ms):
     knn_ms = _time_cuda(lambda: cq.points.findKNN(bvh, P, Qk, 8), 3)
     fcp_kms = _kernel_ms(cq, "fcp_points", lambda: cq.points.findClosest(bvh, P, Qf))
     knn_kms = _kernel_ms(cq, "knn_points", lambda: cq.points.findKNN(bvh, P, Qk, 8))
-    query_rooflines = {
+    query_counts = {
         # query 12 B in, id + distance 8 B out; 4 B primID + 12 B point per prim
-        "fcp": query_roofline(cq, cq.query_stats(bvh, Qf, data=P, k=0), fcp_kms, 20, 16, "fcp_points"),
-        "knn8": query_roofline(cq, cq.query_stats(bvh, Qk, data=P, k=8), knn_kms, 12 + 8 * 8 + 4, 16,
+        "fcp": points_counts(cq.query_stats(bvh, Qf, data=P, k=0), fcp_kms, 20, 16, "fcp_points"),
+        "knn8": points_counts(cq.query_stats(bvh, Qk, data=P, k=8), knn_kms, 12 + 8 * 8 + 4, 16,
                                "knn_points<8>"),
     }
     num_nodes = bvh.numNodes
@@ -491,7 +510,7 @@ def bench_queries(cq, P, Q, boxes, cfg, mem, N, nq, nk, build_ms):
                           "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
                           "bytes_model": "64 B/prim (box read, primID, centroid, leaf box) + 32 B/node "
                                          "+ 20 B per prim and level in an open node"}
-    return fcp_ms, knn_ms, query_rooflines, num_nodes, build_roofline
+    return fcp_ms, knn_ms, query_counts, num_nodes, build_roofline
 
 
 def main():
@@ -574,12 +593,12 @@ def main():
     if "radix" in legs:
         radix = bench_radix(cq, boxes, cfg, mem, N, args.steps, kern)
     tris = mixture = batched = cpu = None
-    query_rooflines = None
+    query_counts = None
     fcp_ms = knn_ms = None
     nq, nk = args.fcp_queries, args.knn_queries
     num_nodes = build_roofline = None
     if "queries" in legs:
-        (fcp_ms, knn_ms, query_rooflines, num_nodes,
+        (fcp_ms, knn_ms, query_counts, num_nodes,
          build_roofline) = bench_queries(cq, P, Q, boxes, cfg, mem, N, nq, nk, ms_per_step)
         print(f"[bench] fcp {nq/fcp_ms/1e3:.1f} Mq/s, knn {nk/knn_ms/1e3:.1f} Mq/s", file=sys.stderr,
               flush=True)
@@ -632,7 +651,7 @@ def main():
         "radix_builds": radix,
         "fcp_mqueries_s": nq / fcp_ms / 1e3 if fcp_ms else None,
         "knn_mqueries_s": nk / knn_ms / 1e3 if knn_ms else None,
-        "query_rooflines": query_rooflines,
+        "query_counts": query_counts,
         "pcie_h2d_gbs": pcie_h2d_gbs,
         "triangle_mesh": tris,
         "gaussian_mixture": mixture,

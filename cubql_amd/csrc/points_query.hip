@@ -967,8 +967,10 @@ __device__ __forceinline__ void stats_flush(const cubql_dev::TraversalCounts &st
   }
 }
 
-// Instrumented closest-point (k == 0) or kNN queries with the deep stack:
-// per query, bytes of node data loaded and prims tested.
+// Instrumented closest-point (k == 0) or kNN queries with the deep stack: per
+// query, bytes of node data loaded and prims tested by one lane walking alone.
+// (k_fcp and k_knn_wave share a wave's subtrees and visit other nodes; k_knn, for
+// more than kKnnWaveMax neighbours, walks as here.)
 template <int K>
 __global__ __launch_bounds__(64) void k_points_stats(cubql_bvh3f bvh, const float *points, const float *queries,
                                                      uint32_t nq, int k, float sqrMax, unsigned long long *out) {
@@ -984,7 +986,6 @@ __global__ __launch_bounds__(64) void k_points_stats(cubql_bvh3f bvh, const floa
       int32_t ids[K];
       float ds[K];
       int found;
-      // the traversal k_knn runs, on the deep stack
       if constexpr (K <= kKnnSeededMax) {
         cubql_dev::PrivateStack<kDeepStack> stack;
         knn_seeded_on<K>(stack, bvh, points, nullptr, q, k, sqrMax, ids, ds, found, st);

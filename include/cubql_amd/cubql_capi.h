@@ -418,8 +418,10 @@ int cubql_profile_query(const char *kernel, uint64_t *launches, double *totalMs,
 /* Traversal statistics, the counterpart of the nodeDist / primCode counters
    of the reference's traversal-quality test (testing/bvh/buildQual.h:65-98,
    NUM_TRAVERSAL_STEPS): runs the same queries as cubql_fcp_points_f3
-   (k == 0), cubql_knn_points_f3 (1 <= k <= 64) or cubql_fcp_triangles_f3
-   with per-query counters and writes three device uint64 sums to d_out:
+   (k == 0), cubql_knn_points_f3 (1 <= k <= 64) or cubql_fcp_triangles_f3, one
+   lane walking alone for each (the point queries themselves share subtrees
+   between the lanes of a wave and visit other nodes), with per-query counters,
+   and writes three device uint64 sums to d_out:
    bytes of node data loaded (64 per child pair expanded, 32 per node popped
    from the stack), prims (points or triangles) tested, and queries.  A
    measurement aid: slower than the plain queries, results discarded. */
