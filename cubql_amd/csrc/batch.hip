@@ -414,7 +414,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
 void k_bquery(Side qs, Side ts, uint32_t qpw, int32_t *nn, float *d2, uint32_t *ovf) {
   __shared__ WaveTasksAux tasks[BLOCK / kWave];
   const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
-  // queries sorted by (cloud, Morton key): one contiguous run per XCD
+  // queries sorted by (cloud, Morton key): contiguous runs of them per XCD
   const uint64_t i = (uint64_t)(xcd_chunk(blockIdx.x, gridDim.x) * (BLOCK / kWave) + wave) * qpw + lane;
   const bool act = lane < qpw && i < qs.n;
   const uint32_t t = act ? (uint32_t)i : 0u;

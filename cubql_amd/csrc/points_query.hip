@@ -3,8 +3,10 @@
 // Replaces user kernels that call cuBQL::points::findClosest / findKNN once
 // per thread (queries/points/findClosest.h:181-226, queries/points/knn.h:
 // 75-116; sample launch: samples/s01_closestPoint_points_gpu/
-// closestPoint.cu:41-66).  One query per lane of a wave64; traversal from
-// include/cubql_amd/traversal.hip.h.  Result rule: among equal float32
+// closestPoint.cu:41-66).  Over binary trees a wave64 takes up to 64 queries and
+// its lanes share their subtrees (wave_closest.h, wave_knn.h); over wide trees, for
+// more than kKnnWaveMax neighbours and in the deep reruns a lane walks for one query
+// (include/cubql_amd/traversal.hip.h).  Result rule: among equal float32
 // distances the lowest primID wins (kNN lists are ordered by
 // (sqrDist, primID)).
 #include <mutex>
@@ -118,7 +120,7 @@ __global__ __launch_bounds__(kBlock) void k_fcp(cubql_bvh3f bvh, const float *po
                                                 const uint32_t *order) {
   __shared__ WaveTasks tasks[kBlock / kWave];
   const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
-  // Morton-ordered queries: one contiguous run of them per XCD
+  // spatially ordered queries: contiguous runs of them per XCD
   const uint32_t b = order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x;
   const uint64_t i = (uint64_t)(b * (kBlock / kWave) + wave) * qpw + lane;
   const bool live = lane < qpw && i < nq;
@@ -285,9 +287,8 @@ constexpr int kSeedSibs = 4;
 // pairs under sqrMax whatever the visiting order, and every leaf within the
 // radius is still visited exactly once.  One loop visits every leaf, so the
 // insertion code is inlined once.
-template <int K, bool kSorted = false, typename StackT, typename Stats = cubql_dev::NoStats>
-__device__ __forceinline__ bool knn_seeded_on(StackT &stack, const cubql_bvh3f &bvh, const float *points,
-                                              const float4 *spts, float3 q, int k, float sqrMax,
+template <int K, typename StackT, typename Stats = cubql_dev::NoStats>
+__device__ __forceinline__ bool knn_seeded_on(StackT &stack, const cubql_bvh3f &bvh, const float *points, float3 q, int k, float sqrMax,
                                               int32_t (&ids)[K], float (&ds)[K], int &found,
                                               Stats &&st = Stats()) {
   using namespace cubql_dev;
@@ -342,16 +343,8 @@ __device__ __forceinline__ bool knn_seeded_on(StackT &stack, const cubql_bvh3f &
       }
       if (!skip)
         for (uint32_t c = 0; c < cnt; c++) {
-          uint32_t pid;
-          float3 p;
-          if constexpr (kSorted) {
-            const float4 v = spts[off + c];
-            pid = __float_as_uint(v.w);
-            p = make_float3(v.x, v.y, v.z);
-          } else {
-            pid = bvh.primIDs[off + c];
-            p = load_pt(points, pid);
-          }
+          const uint32_t pid = bvh.primIDs[off + c];
+          const float3 p = load_pt(points, pid);
           st.prim();
           const float d = sqr_dist_pt(p.x, p.y, p.z, q.x, q.y, q.z);
           const int32_t id = (int32_t)pid;
@@ -470,7 +463,7 @@ __global__ __launch_bounds__(kBlock) void k_knn_wave(cubql_bvh3f bvh, const floa
                                                      const uint32_t *order) {
   __shared__ WaveKnn<K> share[kBlock / kWave];
   const uint32_t wave = threadIdx.x / kWave, lane = lane_id();
-  // spatially ordered queries: one contiguous run of them per XCD
+  // spatially ordered queries: contiguous runs of them per XCD
   const uint32_t b = order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x;
   const uint64_t i = (uint64_t)(b * (kBlock / kWave) + wave) * qpw + lane;
   const bool live = lane < qpw && i < nq;
@@ -541,7 +534,7 @@ __global__ __launch_bounds__(kBlock) void k_knn(BVH bvh, const float *points, co
                                                 float sqrMax, int32_t *outIds, float *outD,
                                                 int32_t *outFound, Overflow *ovf,
                                                 uint32_t *ovfList, const uint32_t *order) {
-  // spatially ordered queries: one contiguous run of them per XCD
+  // spatially ordered queries: contiguous runs of them per XCD
   const uint32_t i = (order ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x) * kBlock + threadIdx.x;
   if (i >= nq) return;
   const uint32_t qi = order ? order[i] : i;
@@ -579,7 +572,7 @@ __global__ __launch_bounds__(64) void k_knn_deep(BVH bvh, const float *points,
     bool done;
     if constexpr (std::is_same<BVH, cubql_bvh3f>::value && K <= kKnnSeededMax) {
       cubql_dev::PrivateStack<kDeepStack> stack;
-      done = knn_seeded_on<K>(stack, bvh, points, nullptr, q, k, sqrMax, ids, ds, found);
+      done = knn_seeded_on<K>(stack, bvh, points, q, k, sqrMax, ids, ds, found);
     } else {
       done = knn_one<K, kDeepStack>(bvh, points, nullptr, q, k, sqrMax, ids, ds, found);
     }
@@ -988,7 +981,7 @@ __global__ __launch_bounds__(64) void k_points_stats(cubql_bvh3f bvh, const floa
       int found;
       if constexpr (K <= kKnnSeededMax) {
         cubql_dev::PrivateStack<kDeepStack> stack;
-        knn_seeded_on<K>(stack, bvh, points, nullptr, q, k, sqrMax, ids, ds, found, st);
+        knn_seeded_on<K>(stack, bvh, points, q, k, sqrMax, ids, ds, found, st);
       } else {
         knn_one<K, kDeepStack>(bvh, points, nullptr, q, k, sqrMax, ids, ds, found, st);
       }

@@ -740,9 +740,9 @@ __global__ __launch_bounds__(kBlock) void k_karras_emit(const K *keys, const cub
 // the level-order inner node w when w < 2^D - 1, else node k = w - (2^D - 1)
 // of depth D, inner when it holds T + 1 prims; the depth-D inner nodes are
 // numbered by rank, which is their start offset minus k q (every depth-D
-// node before k holds q or q + 1 prims).  Each inner node writes itself,
-// its leaf children with their boxes, and its position into its depth's
-// bucket (slots claimed by one atomic per wave and depth).
+// node before k holds q or q + 1 prims).  Each inner node writes itself, its
+// leaf children with their boxes, and its position as the parent of its pair
+// (up[], with arrive[] cleared, for k_karras_climb).
 __global__ __launch_bounds__(256) void k_karras_equal(const cubql_box3f *boxes, const uint32_t *primIDs, uint32_t T,
                                                       const EqRoot *roots, uint32_t nr, uint32_t *up,
                                                       uint32_t *arrive, Node *nodes) {
