@@ -1,8 +1,10 @@
 // common.hip -- error state, memory resource and small utility kernels.
 #include <cstdarg>
 #include <mutex>
+#include <vector>
 
 #include "common.h"
+#include "host_words.h"
 
 namespace cubql {
 
@@ -68,6 +70,46 @@ int mem_free(const cubql_mem_resource *mem, void *ptr, hipStream_t s) {
     return CUBQL_ERR_HIP;
   }
   return CUBQL_OK;
+}
+
+// (Not destroyed at exit: a static destructor could run after the runtime's.)
+struct HostBlocks {
+  std::mutex mu;
+  std::vector<uint32_t *> free;
+};
+static HostBlocks &host_blocks() {
+  static HostBlocks *b = new HostBlocks;
+  return *b;
+}
+
+HostWords::HostWords() {
+  HostBlocks &b = host_blocks();
+  {
+    std::lock_guard<std::mutex> lk(b.mu);
+    if (!b.free.empty()) {
+      p_ = b.free.back();
+      b.free.pop_back();
+      return;
+    }
+  }
+  const hipError_t e = hipHostMalloc((void **)&p_, kWords * sizeof(uint32_t), hipHostMallocPortable);
+  if (e != hipSuccess) {
+    p_ = nullptr;
+    set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
+  }
+}
+
+HostWords::~HostWords() {
+  if (!p_) return;
+  HostBlocks &b = host_blocks();
+  {
+    std::lock_guard<std::mutex> lk(b.mu);
+    if (b.free.size() < kKept) {
+      b.free.push_back(p_);
+      return;
+    }
+  }
+  (void)hipHostFree(p_);
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint32_t v, size_t n) {

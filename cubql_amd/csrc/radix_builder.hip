@@ -20,6 +20,7 @@
 #include "build_common.h"
 #include "wave_ops.h"
 #include "common.h"
+#include "host_words.h"
 #include "profile.h"
 #include "radix_sort.h"
 #include "refit.h"
@@ -632,14 +633,8 @@ __global__ void k_karras_info(const K *keys, const uint32_t *nPtr, const uint32_
   info[M_SPIN] = *spin;
 }
 
-// pinned host mirror of those words, or of the counters
 constexpr size_t kCtrWords = C_LSTART0 + kMaxLevels + 8;
-static_assert((size_t)M_WORDS <= kCtrWords, "one buffer for both");
-static uint32_t *host_words() {
-  static thread_local uint32_t *p = nullptr;
-  if (!p && hipHostMalloc((void **)&p, kCtrWords * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) p = nullptr;
-  return p;
-}
+static_assert((size_t)M_WORDS <= HostWords::kWords && kCtrWords <= HostWords::kWords, "host mirror of either");
 
 // The root alone: one leaf of at most T prims (one workgroup) ...
 __global__ __launch_bounds__(256) void k_karras_leaf_root(const cubql_box3f *boxes, const uint32_t *primIDs,
@@ -986,8 +981,9 @@ int build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, in
                                             misc + M_SPLIT, misc + M_EQPAIRS, misc + M_ERR);
   k_karras_info<K><<<1, 1, 0, s>>>(kRes, nv, &c.ctr[C_SPIN], T, misc);
   if (hipGetLastError() != hipSuccess) return fail((set_error("hierarchy launch failed"), CUBQL_ERR_HIP));
-  const uint32_t *hm = host_words();
-  if (!hm) return fail((set_error("hipHostMalloc failed"), CUBQL_ERR_HIP));
+  const HostWords words;
+  const uint32_t *hm = words.get();
+  if (!hm) return fail(CUBQL_ERR_HIP);
   if (hipMemcpyAsync((void *)hm, misc, M_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail((set_error("hierarchy sync failed"), CUBQL_ERR_HIP));
@@ -1467,8 +1463,9 @@ int rebin_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t
   const uint32_t grid = std::max<uint32_t>(1u, std::min<uint32_t>(div_up(n, kBlock), (uint32_t)numCU * 8));
   int jobBits = 1;
   while ((1ull << jobBits) < (uint64_t)maxJobs) jobBits++;
-  uint32_t *hc = host_words();
-  if (!hc) return fail((set_error("hipHostMalloc failed"), CUBQL_ERR_HIP));
+  const HostWords hostWords;
+  uint32_t *hc = hostWords.get();
+  if (!hc) return fail(CUBQL_ERR_HIP);
   int level = 0, rounds = 0;
   int hs = prof_begin(s);
   while (true) {

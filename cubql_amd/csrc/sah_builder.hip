@@ -30,6 +30,7 @@
 #include "block_ops.h"
 #include "build_common.h"
 #include "common.h"
+#include "host_words.h"
 #include "profile.h"
 #include "wave_ops.h"
 
@@ -1268,13 +1269,7 @@ __global__ void k_copy_top(const Node *src, Node *dst, uint32_t n) {
 
 }  // namespace sah
 
-static_assert(sizeof(sah::Counters) <= 64 * sizeof(uint32_t), "host counter mirror");
-static uint32_t *sah_host_words() {
-  static thread_local uint32_t *p = nullptr;
-  if (!p && hipHostMalloc((void **)&p, 64 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
-    p = nullptr;
-  return p;
-}
+static_assert(sizeof(sah::Counters) <= HostWords::kWords * sizeof(uint32_t), "host counter mirror");
 
 int sah_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, uint32_t cap,
               int numBins, hipStream_t s, const cubql_mem_resource *mem, bool elh) {
@@ -1348,8 +1343,9 @@ int sah_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T
   }
   if (hipGetLastError() != hipSuccess) return fail((set_error("sah init launch failed"), CUBQL_ERR_HIP));
 
-  uint32_t *hw = sah_host_words();
-  if (!hw) return fail((set_error("hipHostMalloc failed"), CUBQL_ERR_HIP));
+  const HostWords words;
+  uint32_t *hw = words.get();
+  if (!hw) return fail(CUBQL_ERR_HIP);
   int dev = 0, numCU = 256;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&numCU, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)

@@ -26,6 +26,7 @@
 //     passes.
 #include "block_ops.h"
 #include "common.h"
+#include "host_words.h"
 #include "wave_ops.h"
 #include "build_common.h"
 #include "profile.h"
@@ -2125,15 +2126,8 @@ __global__ __launch_bounds__(1024) void k_refit_top(Ctx c, Node *nodes, int list
 
 }  // namespace sm
 
-// pinned host mirror for the few completion checks
-static_assert(sizeof(sm::Counters) <= 64 * sizeof(uint32_t), "host counter mirror");
-static uint32_t *host_words() {
-  static thread_local uint32_t *p = nullptr;
-  if (!p) {
-    if (hipHostMalloc((void **)&p, 64 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) p = nullptr;
-  }
-  return p;
-}
+// host mirror for the few completion checks
+static_assert(sizeof(sm::Counters) <= HostWords::kWords * sizeof(uint32_t), "host counter mirror");
 
 int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T, hipStream_t s,
              const cubql_mem_resource *mem) {
@@ -2199,8 +2193,9 @@ int sm_build(cubql_bvh3f *bvh, const cubql_box3f *boxes, uint32_t n, uint32_t T,
   k_write_items<<<numBlocks, kBlock, 0, s>>>(c);
   if (hipGetLastError() != hipSuccess) return fail((set_error("init launch failed"), CUBQL_ERR_HIP));
 
-  uint32_t *hw = host_words();
-  if (!hw) return fail((set_error("hipHostMalloc failed"), CUBQL_ERR_HIP));
+  const HostWords words;
+  uint32_t *hw = words.get();
+  if (!hw) return fail(CUBQL_ERR_HIP);
   int dev = 0, numCU = 256;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&numCU, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)

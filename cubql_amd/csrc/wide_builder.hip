@@ -18,6 +18,7 @@
 #include "block_ops.h"
 #include "build_common.h"
 #include "common.h"
+#include "host_words.h"
 
 namespace cubql {
 namespace wd {
@@ -117,14 +118,6 @@ __global__ void k_exec(const Node *nodes, uint32_t n, const uint32_t *flag, cons
 
 // Collapse `bin` into `out` (nodes allocated from `mem`; primIDs left to the
 // caller).  Blocks the host once to read the wide node count.
-// pinned host mirror of the node count and the fault word (a copy to pageable
-// memory waits by itself)
-static uint32_t *host_words() {
-  static thread_local uint32_t *p = nullptr;
-  if (!p && hipHostMalloc((void **)&p, 2 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) p = nullptr;
-  return p;
-}
-
 int collapse_wide(const cubql_bvh3f &bin, int width, cubql_wbvh3f *out, hipStream_t s,
                   const cubql_mem_resource *mem) {
   const uint32_t n = bin.numNodes;
@@ -151,11 +144,9 @@ int collapse_wide(const cubql_bvh3f &bin, int width, cubql_wbvh3f *out, hipStrea
   wd::k_flag<<<g, 256, 0, s>>>(nodes, n, parent, logW, flag);
   wd::k_scan<<<scanTiles, 1024, 0, s>>>(flag, wideId, n, status, total);
   CUBQL_LAUNCH_CHECK();
-  uint32_t *tw = host_words();
-  if (!tw) {
-    set_error("hipHostMalloc failed");
-    return CUBQL_ERR_HIP;
-  }
+  const HostWords words;
+  uint32_t *tw = words.get();
+  if (!tw) return CUBQL_ERR_HIP;
   CUBQL_HIP(hipMemcpyAsync(tw, total, 8, hipMemcpyDeviceToHost, s));
   CUBQL_HIP(hipStreamSynchronize(s));
   if (tw[1]) {
