@@ -12,9 +12,12 @@
 // (query_order.h), a wave of queries walking together, and read leaf prims
 // from a copy of the prim boxes in primID-slot order.  1M boxes against
 // themselves, leaves of 4: 1305 us with one query per lane in input order, on
-// a private stack and with a gather per prim; 538 us here and 65 us for the
-// order and the copy.  Bound by the latency of the wave's chain of scalar
-// loads (two rounds of waves, 400 loads each).
+// a private stack and with a gather per prim; 517 us here and 88 us for the
+// order and the copy.  Bound by the wave's chain of 381 scalar loads, each
+// waited for before the next address is known: a wave waits for memory 52% of
+// its time and to issue 23%, with all 8 waves to a SIMD.  The busiest unit is
+// the scalar one (12.5K instructions a wave: 0.33 ms at one a cycle for each
+// CU); the VALU issues for 0.22 ms.
 #include <type_traits>
 
 #include "common.h"
@@ -86,8 +89,8 @@ __global__ __launch_bounds__(256) void k_slot_boxes(const uint32_t *primIDs, uin
 // > 0 iff the boxes are apart: the largest gap over the axes.  a > b exactly
 // where a - b > 0, and where a difference is NaN the comparison is false and
 // the maximum passes it over.  Six subtractions and three maxima: six
-// comparisons would be joined by scalar instructions, and those, one a cycle
-// for the whole CU, bound this kernel (18.3K of them a wave, 670 us).
+// comparisons would be joined by scalar instructions, whose unit is this
+// kernel's busiest (18.3K of them a wave and 670 us that way, 12.5K and 517 so).
 __device__ __forceinline__ float box_gap(const float (&lo)[3], const float (&hi)[3], float lx, float ly, float lz,
                                          float hx, float hy, float hz) {
   const float a = fmaxf(fmaxf(lo[0] - hx, lx - hi[0]), lo[1] - hy);

@@ -97,8 +97,8 @@ __device__ __forceinline__ void write_result(uint32_t qi, int32_t best, float be
 // leaf at a time a test, a hundred instructions and three 16-byte loads, ran
 // with 12% of the lanes on.  The wave takes the step most lanes wait for:
 // expanding a node, popping the stack or testing.  4M queries of 1.3M
-// triangles: 3.94 ms with each lane testing its own leaf, 2.58 ms here, bound by
-// VALU issue (94%).  Slower: 4 to 12 stack entries in LDS (fewer waves), lanes
+// triangles: 3.94 ms with each lane testing its own leaf, 2.49 ms here, bound by
+// VALU issue (99%).  Slower: 4 to 12 stack entries in LDS (fewer waves), lanes
 // that take a new query when they are done (waves of several hundred queries end
 // far apart), scalar loads where all lanes are at one node.
 constexpr int kTriLeafMax = 8;  // triangles of a lane's leaf dealt out at once

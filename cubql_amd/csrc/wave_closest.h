@@ -29,13 +29,13 @@
 namespace cubql {
 
 // Queue slots of a wave: 512 leave fewer waves in flight (10M queries of 10M
-// points: 2.21 ms a call against 2.04 ms), 256 send more queries of clustered
-// and Gaussian clouds to the deep kernel.  A task is {offset, distance with the query's lane
+// points: 2.21 ms a call against 2.04 ms), with 256 more queries of clustered
+// and Gaussian clouds lose a task and run again.  A task is {offset, distance with the query's lane
 // in its low 6 bits (rounded down: the test only gets weaker)} and the
 // prim count (0: an inner node).
 constexpr int kTaskCap = 320;
-// steps of one descent after which a query goes to the deep kernel (the
-// depth that kernel's stack holds)
+// steps of one descent after which a query has to run again, in the end in the
+// deep kernel (the depth that kernel's stack holds)
 constexpr uint32_t kMaxSteps = 1024;
 
 struct WaveTasks {
@@ -50,9 +50,14 @@ struct WaveTasksAux : WaveTasks {
   uint32_t aux[kWave];
 };
 
-// Waves that a small batch is spread over: 1000 queries of 1M points take
-// 25.6 us as 1000 waves of one query, whose subtrees the other lanes take,
-// and took 87.7 us as 16 waves of one query per lane.
+// Waves that a small batch is spread over: in a wave of few queries the other
+// lanes take their subtrees.  Calls on a tree of 1M points, spread so and as
+// waves of 64 queries (us):
+//   queries          64    1000    4096   16000   64000
+//   closest       38/47   40/54   42/56   48/69  90/103
+//   k = 8        61/122  63/167  78/179  99/181 176/216
+// (100000 Gaussian points: 38/51, 39/54, 43/55, 43/56, 89/95 and 63/133,
+// 63/152, 76/158, 87/158, 153/191.)
 constexpr uint32_t kWavesWanted = 4096;
 // Queries of one wave: 64 once they fill the chip, fewer for small batches,
 // whose time is one wave's chain of dependent loads.
