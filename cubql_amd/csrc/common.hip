@@ -1,7 +1,6 @@
 // common.hip -- error state, memory resource and small utility kernels.
 #include <cstdarg>
 #include <mutex>
-#include <vector>
 
 #include "common.h"
 #include "host_words.h"
@@ -72,23 +71,19 @@ int mem_free(const cubql_mem_resource *mem, void *ptr, hipStream_t s) {
   return CUBQL_OK;
 }
 
-// (Not destroyed at exit: a static destructor could run after the runtime's.)
-struct HostBlocks {
+// (An array: nothing here allocates, throws or is destroyed at exit, which could be
+// after the runtime.)
+static struct {
   std::mutex mu;
-  std::vector<uint32_t *> free;
-};
-static HostBlocks &host_blocks() {
-  static HostBlocks *b = new HostBlocks;
-  return *b;
-}
+  uint32_t *block[HostWords::kKept];
+  size_t count;
+} host_blocks;
 
 HostWords::HostWords() {
-  HostBlocks &b = host_blocks();
   {
-    std::lock_guard<std::mutex> lk(b.mu);
-    if (!b.free.empty()) {
-      p_ = b.free.back();
-      b.free.pop_back();
+    std::lock_guard<std::mutex> lk(host_blocks.mu);
+    if (host_blocks.count) {
+      p_ = host_blocks.block[--host_blocks.count];
       return;
     }
   }
@@ -101,11 +96,10 @@ HostWords::HostWords() {
 
 HostWords::~HostWords() {
   if (!p_) return;
-  HostBlocks &b = host_blocks();
   {
-    std::lock_guard<std::mutex> lk(b.mu);
-    if (b.free.size() < kKept) {
-      b.free.push_back(p_);
+    std::lock_guard<std::mutex> lk(host_blocks.mu);
+    if (host_blocks.count < kKept) {
+      host_blocks.block[host_blocks.count++] = p_;
       return;
     }
   }
